@@ -1,0 +1,133 @@
+"""Scoring on the matrix cores (ytm_matrix.hip) against the oracle: every number of literal
+steps and of patch tiles per wave, the edges of the tiles of 32 patches, clauses and samples,
+samples whose negated literals are not complements, and weights of one to five digits.  Class
+sums are whole numbers: compared bit for bit."""
+import numpy as np
+import pytest
+
+from oracle import oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+ytm_amd = pytest.importorskip("ytm_amd")
+from ytm_amd import MultiClassTM  # noqa: E402
+
+
+def pair(clauses, dim, classes, rng, weight=50, **kw):
+    """The GPU model and the oracle with one random state: clauses of no, few and many literals,
+    some with a literal and its negation."""
+    tm = MultiClassTM(clauses, 50, 5.0, dim, classes, seed=7, **kw)
+    ref = orc.OracleTM(clauses, 50, 5.0, dim, classes, seed=7, **kw)
+    C, L = tm.number_of_clauses, tm.number_of_literals
+    p = np.choose(rng.integers(0, 10, C), [0.0] + [2.0 / L] * 6 + [5.0 / L] * 2 + [0.3])
+    inc = rng.random((C, L)) < p[:, None]
+    ta = np.where(inc, 200, 60).astype(np.uint32)
+    w = rng.integers(-weight, weight + 1, (C, classes)).astype(np.float32)
+    tm.load_state_dict({"state": {"ta_state": ta, "clause_weights": w, "min_y": None, "max_y": None,
+                                  "patch_weights": np.zeros((C, tm.number_of_patches), np.int32)}})
+    ref.ta[...] = ta.reshape(ref.ta.shape)
+    ref.w[...] = w.reshape(ref.w.shape)
+    return tm, ref
+
+
+def check(tm, ref, enc):
+    data = tm._device_data(enc)
+    want = ref.score(enc)
+    np.testing.assert_array_equal(tm.score_device(data), want)
+    np.testing.assert_array_equal(tm.score_device(data), want)  # the kept operands
+    return want
+
+
+def image(rng, n, dim):
+    return (rng.random((n, dim[0] * dim[1] * dim[2])) < 0.6).astype(np.uint32)
+
+
+@pytest.mark.parametrize("dim,patch,clauses,n", [
+    ((3, 2, 1), (2, 2), 1, 1),         # 2 patches, 1 step, one clause and sample
+    ((7, 6, 1), (2, 3), 33, 70),       # 24 patches: samples share a wave
+    ((9, 7, 1), (2, 3), 64, 33),       # 40 patches: tiles of one sample in two waves
+    ((6, 9, 9), (3, 2), 31, 5),        # 32 patches: a whole tile
+    ((13, 12, 10), (3, 4), 300, 9),    # 2 literal steps
+    ((20, 20, 1), (10, 12), 290, 6),   # 99 patches
+    ((28, 28, 1), (10, 10), 500, 7),   # 361 patches, 3 steps
+    ((12, 12, 24), (3, 3), 270, 40),   # 4 steps
+    ((32, 32, 24), (3, 3), 2600, 3),   # 900 patches, 5 steps: one sample fills the waves
+    ((40, 33, 24), (3, 3), 100, 2),    # 1178 patches: a sample in two rounds
+    ((10, 10, 33), (3, 3), 130, 21),   # 6 steps
+    ((9, 8, 47), (3, 3), 65, 20),      # 7 steps
+    ((9, 8, 54), (3, 3), 65, 20),      # 8 steps
+    ((9, 8, 62), (3, 3), 65, 20),      # 9 steps
+])
+def test_steps_and_tiles(dim, patch, clauses, n):
+    rng = np.random.default_rng(3)
+    tm, ref = pair(clauses, dim, 3, rng, patch_dim=patch)
+    want = check(tm, ref, tm.encode(image(rng, n, dim)))
+    assert clauses < 30 or np.unique(want).size > 1
+
+
+@pytest.mark.parametrize("dim,patch,negated", [
+    ((12, 12, 2), (4, 4), False),    # no negations: all literals, 1 step
+    ((28, 28, 1), (10, 10), True),   # 272 literals without complements: 5 steps
+    ((14, 14, 24), (3, 3), True),    # 476: 8 steps
+    ((9, 8, 62), (3, 3), True),      # beyond 9 steps: the literal lists
+])
+def test_all_literals(dim, patch, negated):
+    """Samples whose negated literals are not the complements of the positive ones (encoded
+    elsewhere), beside the same model's scores of framework-encoded samples."""
+    rng = np.random.default_rng(4)
+    tm, ref = pair(200, dim, 4, rng, patch_dim=patch, append_negated=negated)
+    enc = tm.encode(image(rng, 12, dim))
+    odd = enc & rng.integers(0, 2**32, enc.shape, dtype=np.uint32) | enc & rng.integers(0, 2**32, enc.shape,
+                                                                                       dtype=np.uint32)
+    check(tm, ref, enc)
+    check(tm, ref, odd)
+    check(tm, ref, enc)
+
+
+@pytest.mark.parametrize("classes,weight", [(2, 1), (10, 127), (10, 128), (17, 32639), (11, 40000), (33, 8355711),
+                                            (7, 9000000), (40, 2**30), (5, 2**31 - 256), (70, 300)])
+def test_weight_digits(classes, weight):
+    """Weights of every number of base-256 digits, at their largest, over one and several column
+    groups; the sums of few firing clauses stay exact in float32 or round once, as the
+    oracle's do."""
+    rng = np.random.default_rng(5)
+    dim, patch = (9, 9, 2), (4, 4)
+    tm, ref = pair(150, dim, classes, rng, weight=weight, patch_dim=patch)
+    w = tm.get_weights()
+    w[::3] = np.where(w[::3] < 0, -weight, weight)
+    state = tm.get_state_dict()
+    state["clause_weights"] = w.reshape(-1)
+    tm.load_state_dict({"state": state})
+    ref.w[...] = w.reshape(ref.w.shape)
+    check(tm, ref, tm.encode(image(rng, 37, dim)))
+
+
+def test_operands_follow_the_model():
+    """Kept operands are made again after a fit, new weights and new states."""
+    rng = np.random.default_rng(6)
+    dim = (10, 10, 1)
+    tm, ref = pair(60, dim, 3, rng, patch_dim=(4, 4))
+    X = image(rng, 50, dim)
+    enc, y = tm.encode(X), rng.integers(0, 3, 50).astype(np.uint32)
+    check(tm, ref, enc)
+    ref.load_state(ref.ta, ref.w, np.zeros((60, tm.number_of_patches), np.int32), 0)
+    tm.fit(enc, y, is_X_encoded=True)
+    ref.fit_encoded(enc, ref.encode_y_multiclass(y))
+    check(tm, ref, enc)
+    state = tm.get_state_dict()
+    state["clause_weights"] = -state["clause_weights"]
+    tm.load_state_dict({"state": state})
+    ref.w[...] = -ref.w
+    check(tm, ref, enc)
+
+
+def test_literal_lists_of_wide_patches(monkeypatch):
+    """Patches of more literals than the product's registers hold keep the literal-list scorer:
+    blocks over every clause of a sample and over chunks of 4096 clauses."""
+    rng = np.random.default_rng(7)
+    dim = (16, 16, 64)
+    tm, ref = pair(4200, dim, 3, rng, patch_dim=(3, 3))
+    enc = tm.encode(image(rng, 5, dim))
+    for least in ("1", "1000000"):
+        monkeypatch.setenv("YTM_SCORE_WHOLE_MIN", least)
+        check(tm, ref, enc)

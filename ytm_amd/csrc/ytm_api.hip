@@ -40,11 +40,13 @@ struct ytm_model {
   size_t sacc_bytes = 0, sout_bytes = 0, slists_bytes = 0;
   void* h_sout = nullptr;  // pinned host staging of the class sums (hipHostMalloc)
   size_t h_sout_bytes = 0;
-  // The TA states change with every fit and ytm_set_ta_state (planes_version counts them);
-  // the one-patch literal lists in d_slists hold those of version slists_version, so that
-  // scoring again an unchanged model does not rebuild them.
-  uint64_t planes_version = 0;
+  // The state changes with every fit, ytm_set_ta_state and ytm_set_weights (state_version
+  // counts them); d_slists holds the one-patch literal lists or the matrix operands
+  // (slists_kind) of version slists_version, so that scoring again an unchanged model does
+  // not rebuild them.
+  uint64_t state_version = 0;
   uint64_t slists_version = ~0ull;
+  int slists_kind = 0;
   // Upper bound of |clause weight|: 1 after initialisation, the largest loaded magnitude
   // after ytm_set_weights, and + 1 per trained sample (a sample moves a weight by at most 1).
   double w_bound = 1.0;
@@ -65,8 +67,8 @@ struct ytm_dataset {
   uint32_t* d_X;   // [N][P][W]
   int32_t* d_Y;    // [N][K]
   int64_t N;
-  uint32_t* d_XT;  // [N][L][ceil(P/32)] literal-major copy (several patches), or null
-  int xt_halves;   // d_XT's literals Lh..L-1 are the complements of 0..Lh-1 (TrainArgs::xt_halves)
+  uint32_t* d_XT;  // [N][L][ceil(P/32)] literal-major copy (several patches, where a kernel reads it), or null
+  int halves;      // every sample's literals Lh..L-1 are the complements of 0..Lh-1 (several patches)
   uint32_t* d_order;  // [kOrderBuckets][W] literal order of the training lists (with d_XT), or null
 };
 
@@ -700,27 +702,30 @@ int ytm_dataset_create(ytm_model* m, const uint32_t* encX, const int32_t* encY, 
   ytm_dataset* ds = new ytm_dataset{m, nullptr, nullptr, N, nullptr, 0, nullptr};
   int rc = upload((void**)&ds->d_X, encX, (size_t)(N * g.P * g.W) * 4, m->stream);
   if (!rc && encY) rc = upload((void**)&ds->d_Y, encY, (size_t)(N * g.K) * 4, m->stream);
-  if (!rc && ytm::literal_major(g) && N > 0) {
-    // Several patches: the training kernel evaluates clauses on a literal-major copy.
+  if (!rc && g.P > 1 && g.append_negated && N > 0) {
+    // Encoded samples hold the negations as complements (BaseTM.encode); samples encoded
+    // elsewhere may not, so training and scoring rely on it only where this check holds.
+    int* d_ok = nullptr;
+    int ok = 1;
+    hipError_t e = hipMalloc(&d_ok, sizeof(int));
+    if (e == hipSuccess) e = hipMemcpyAsync(d_ok, &ok, sizeof(int), hipMemcpyHostToDevice, m->stream);
+    if (e == hipSuccess) e = ytm::launch_halves_check(ds->d_X, N, g, d_ok, m->stream);
+    if (e == hipSuccess) e = hipMemcpyAsync(&ok, d_ok, sizeof(int), hipMemcpyDeviceToHost, m->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(m->stream);
+    if (d_ok) (void)hipFree(d_ok);
+    if (e != hipSuccess) rc = fail(YTM_EHIP, std::string("sample check: ") + hipGetErrorString(e));
+    ds->halves = ok == 1;
+  }
+  if (!rc && ytm::literal_major(g) && N > 0 &&
+      (encY || ytm::matrix_plan(g, ds->halves != 0, m->w_bound).steps == 0)) {
+    // Several patches: the training kernel evaluates clauses on a literal-major copy, and so
+    // do the scorers of models that the matrix cores do not take.
     const size_t bytes = (size_t)(N * g.L * ((g.P + 31) / 32)) * 4;
     hipError_t e = hipMalloc(&ds->d_XT, bytes);
     if (e == hipSuccess) e = ytm::launch_transpose(ds->d_X, N, ds->d_XT, g, m->stream);
     // the order of the training kernels' literal lists, from the densities of the first samples
     if (e == hipSuccess) e = hipMalloc(&ds->d_order, (size_t)ytm::kOrderBuckets * g.W * 4);
     if (e == hipSuccess) e = ytm::launch_literal_order(nullptr, ds->d_XT, N, g, ds->d_order, m->stream);
-    if (e == hipSuccess && g.append_negated) {
-      // Encoded samples hold the negations as complements (BaseTM.encode); samples encoded
-      // elsewhere may not, so the training kernels rely on it only where this check holds.
-      int* d_ok = nullptr;
-      int ok = 1;
-      e = hipMalloc(&d_ok, sizeof(int));
-      if (e == hipSuccess) e = hipMemcpyAsync(d_ok, &ok, sizeof(int), hipMemcpyHostToDevice, m->stream);
-      if (e == hipSuccess) e = ytm::launch_xt_halves_check(ds->d_XT, N, g, d_ok, m->stream);
-      if (e == hipSuccess) e = hipMemcpyAsync(&ok, d_ok, sizeof(int), hipMemcpyDeviceToHost, m->stream);
-      if (e == hipSuccess) e = hipStreamSynchronize(m->stream);
-      if (d_ok) (void)hipFree(d_ok);
-      ds->xt_halves = e == hipSuccess && ok == 1;
-    }
     if (e != hipSuccess) rc = fail(YTM_EHIP, std::string("literal-major copy: ") + hipGetErrorString(e));
   }
   if (!rc) {
@@ -809,7 +814,7 @@ int ytm_fit_dataset(ytm_model* m, const ytm_dataset* ds, int64_t first, int64_t 
 namespace {
 int fit_range(ytm_model* m, const ytm_dataset* ds, int64_t first, int64_t count, const uint32_t* drop,
               const float* inject) {
-  ++m->planes_version;  // before any launch: also when the fit fails part-way
+  ++m->state_version;  // before any launch: also when the fit fails part-way
   m->stats.last_fit_samples = 0;
   m->stats.last_fit_updates = 0;
   m->stats.last_fit_kernel_ms = 0.0;
@@ -938,7 +943,7 @@ int fit_range(ytm_model* m, const ytm_dataset* ds, int64_t first, int64_t count,
     const char* sg_env = std::getenv("YTM_TRAIN_STREAM_GENS");  // test hook: stops per stream
     a.stream_gens = sg_env ? std::max(0, std::atoi(sg_env)) : 0;
     const char* xh_env = std::getenv("YTM_TRAIN_XT_HALVES");  // 0: stage the whole literal-major copy
-    a.xt_halves = ds->xt_halves && !(xh_env && std::atoi(xh_env) == 0);
+    a.xt_halves = ds->halves && !(xh_env && std::atoi(xh_env) == 0);
     const char* lo_env = std::getenv("YTM_LIST_ORDER");  // 0: literal lists in index order
     a.lit_order = (lo_env && std::atoi(lo_env) == 0) ? nullptr : ds->d_order;
     const char* tt_env = std::getenv("YTM_TRAIN_TEST_TIMEOUT");  // test hook of the timeout path
@@ -1009,17 +1014,22 @@ int ytm_fit(ytm_model* m, const uint32_t* encX, const int32_t* encY, int64_t N, 
 namespace {
 
 // Which scoring kernel a dataset takes, and the device buffers it needs besides the output:
-// literal lists (lists_bytes, several patches or one patch with wide clauses) and the int64
-// class-sum accumulators, acc_per_sample bytes per sample (per-chunk slices for the tiled
-// one-patch scorer, chunks > 0).
+// lists_bytes of model operands (matrix operands, or literal lists of several patches or of
+// one patch with wide clauses) and acc_per_sample bytes per sample (a row of firing words, or
+// int64 class-sum accumulators, per-chunk slices for the tiled one-patch scorer, chunks > 0).
 struct ScorePlan {
+  ytm::MatrixPlan mm;  // mm.steps > 0: the matrix cores
   size_t lists_bytes;
   bool wide;
   int64_t chunks;
   size_t acc_per_sample;
+  // what d_slists holds that outlives a call on an unchanged model, 0 for nothing (the lists of
+  // several patches are in the order of the batch they score)
+  int kept() const { return mm.steps ? 2 + mm.ternary : wide; }
 };
 
-ScorePlan score_plan(const Geom& g, bool has_xt) {
+// Without the matrix cores; has_xt: there is a literal-major copy.
+ScorePlan list_plan(const Geom& g, bool has_xt) {
   ScorePlan p{};
   // the list-based and tiled scorers keep a class per lane: more than 64 classes take
   // launch_score's class-sum kernel
@@ -1033,6 +1043,22 @@ ScorePlan score_plan(const Geom& g, bool has_xt) {
   return p;
 }
 
+ScorePlan score_plan(const ytm_model* m, const ytm_dataset* ds) {
+  ScorePlan p{};
+  p.mm = ytm::matrix_plan(m->g, ds->halves != 0, m->w_bound);
+  if (!p.mm.steps) return list_plan(m->g, ds->d_XT != nullptr);
+  p.lists_bytes = p.mm.bytes;
+  p.acc_per_sample = (size_t)p.mm.row_words * 4;
+  return p;
+}
+
+// Samples per pass that keep the rows of firing words within 256 MiB (the accumulators of the
+// other scorers are a few words per class).
+int64_t score_pass(const ScorePlan& p, int64_t N) {
+  if (!p.mm.steps) return N;
+  return std::min<int64_t>(N, std::max<int64_t>(1024, (int64_t)(((size_t)256 << 20) / p.acc_per_sample)));
+}
+
 // Class sums of N samples (X [N][P][W], XT its literal-major copy or null) into out (device
 // float [N][K]), with the caller's buffers acc (plan.acc_per_sample * N bytes) and lists
 // (plan.lists_bytes).  Enqueued on the model's stream; the include counts are current when
@@ -1041,6 +1067,11 @@ hipError_t score_samples(ytm_model* m, const ScorePlan& plan, const uint32_t* X,
                          long long* acc, void* lists, float* out, bool lists_ready = false) {
   const Geom& g = m->g;
   hipError_t e = hipSuccess;
+  if (plan.mm.steps) {
+    if (!lists_ready) e = ytm::launch_matrix_pack(m->d_planes, m->d_w, g, plan.mm, lists, m->stream);
+    if (e != hipSuccess) return e;
+    return ytm::launch_matrix_score(X, N, g, plan.mm, lists, m->cus, m->d_bias, (uint32_t*)acc, out, m->stream);
+  }
   if (!plan.chunks) e = ytm::launch_fill_u64((unsigned long long*)acc, N * g.K, m->stream);
   if (e != hipSuccess) return e;
   if (plan.wide)
@@ -1097,23 +1128,28 @@ int ytm_score_dataset(ytm_model* m, const ytm_dataset* ds, float* class_sums) {
   const Geom& g = m->g;
   const int64_t N = ds->N;
   if (N == 0) return YTM_OK;
-  const ScorePlan plan = score_plan(g, ds->d_XT != nullptr);
-  hipError_t e = ensure_buffer(&m->d_sacc, &m->sacc_bytes, (size_t)N * plan.acc_per_sample);
+  const ScorePlan plan = score_plan(m, ds);
+  const int64_t per_pass = score_pass(plan, N);
+  hipError_t e = ensure_buffer(&m->d_sacc, &m->sacc_bytes, (size_t)per_pass * plan.acc_per_sample);
   if (e == hipSuccess) e = ensure_buffer(&m->d_sout, &m->sout_bytes, (size_t)(N * g.K) * 4);
   const void* lists_before = m->d_slists;
   if (e == hipSuccess && plan.lists_bytes) e = ensure_buffer(&m->d_slists, &m->slists_bytes, plan.lists_bytes);
   if (m->d_slists != lists_before) m->slists_version = ~0ull;
-  // one-patch lists (no literal order) depend on the TA states only: kept from the last call
-  const bool lists_ready = plan.wide && m->slists_version == m->planes_version;
+  // operands that depend on the model alone are kept from the last call
+  bool lists_ready = plan.kept() && m->slists_kind == plan.kept() && m->slists_version == m->state_version;
   float* dout = (float*)m->d_sout;
   int rc = YTM_OK;
   // the include counts, for the scorers that read them (the list-based ones count their lists)
   if (e == hipSuccess && !plan.lists_bytes) e = ytm::launch_ninc(m->d_planes, m->d_ninc, g, m->stream);
   if (e == hipSuccess) e = hipEventRecord(m->ev0, m->stream);
-  if (e == hipSuccess)
-    e = score_samples(m, plan, ds->d_X, ds->d_XT, N, (long long*)m->d_sacc, plan.lists_bytes ? m->d_slists : nullptr,
-                      dout, lists_ready);
-  m->slists_version = e == hipSuccess && plan.wide ? m->planes_version : ~0ull;
+  for (int64_t first = 0; e == hipSuccess && first < N; first += per_pass) {
+    // more than one pass only without a literal-major copy (score_pass)
+    e = score_samples(m, plan, ds->d_X + first * g.P * g.W, ds->d_XT, std::min(per_pass, N - first),
+                      (long long*)m->d_sacc, plan.lists_bytes ? m->d_slists : nullptr, dout + first * g.K, lists_ready);
+    lists_ready = plan.kept() != 0;
+  }
+  m->slists_version = e == hipSuccess && plan.kept() ? m->state_version : ~0ull;
+  m->slists_kind = plan.kept();
   if (e == hipSuccess) e = hipEventRecord(m->ev1, m->stream);
   // the sums come back through a pinned staging buffer of the model (a direct copy into
   // pageable memory goes through the runtime's own staging, in smaller pieces)
@@ -1141,12 +1177,16 @@ int ytm_score_dataset_noalloc(ytm_model* m, const ytm_dataset* ds, float* d_clas
   const Geom& g = m->g;
   const int64_t N = ds->N;
   if (N == 0) return YTM_OK;
-  const ScorePlan plan = score_plan(g, ds->d_XT != nullptr);
-  const size_t lists_room = (plan.lists_bytes + 255) & ~(size_t)255;  // the sums start 256-byte aligned
-  if (lists_room + plan.acc_per_sample > kNoAllocScratchBytes)
+  auto room = [](const ScorePlan& p) { return (p.lists_bytes + 255) & ~(size_t)255; };  // the sums start 256-byte aligned
+  auto fits = [&](const ScorePlan& p) { return room(p) + p.acc_per_sample <= kNoAllocScratchBytes; };
+  const ScorePlan listed = list_plan(g, ytm::literal_major(g));
+  if (!fits(listed))
     return fail(YTM_EINVAL, "model too large for the allocation-free scorer: it needs " +
-                                std::to_string(lists_room + plan.acc_per_sample) + " bytes of scratch for one sample, " +
+                                std::to_string(room(listed) + listed.acc_per_sample) + " bytes of scratch for one sample, " +
                                 "the scratch holds " + std::to_string(kNoAllocScratchBytes));
+  ScorePlan plan = score_plan(m, ds);
+  if (!fits(plan)) plan = list_plan(g, ds->d_XT != nullptr);
+  const size_t lists_room = room(plan);
   if (m->device < 0 || m->device >= kMaxDevices) return fail(YTM_EINVAL, "device index out of range for the scratch table");
   std::lock_guard<std::mutex> lock(g_scratch_mu[m->device]);
   void* base = nullptr;
@@ -1162,7 +1202,7 @@ int ytm_score_dataset_noalloc(ytm_model* m, const ytm_dataset* ds, float* d_clas
   for (int64_t first = 0; e == hipSuccess && first < N; first += per_pass) {
     const int64_t n = N - first < per_pass ? N - first : per_pass;
     e = score_samples(m, plan, ds->d_X + first * g.P * g.W, ds->d_XT ? ds->d_XT + first * g.L * PW : nullptr, n, acc,
-                      lists, d_class_sums + first * g.K);
+                      lists, d_class_sums + first * g.K, first > 0 && plan.kept());
   }
   if (e == hipSuccess) e = hipEventRecord(m->ev1, m->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(m->stream);
@@ -1247,7 +1287,7 @@ int ytm_get_ta_state(ytm_model* m, uint32_t* out) {
 int ytm_set_ta_state(ytm_model* m, const uint32_t* in) {
   if (!m || !in) return fail(YTM_EINVAL, "null argument");
   const Geom& g = m->g;
-  ++m->planes_version;
+  ++m->state_version;
   // Representable and closed under the feedback dynamics: s' = s + off < 2^np.
   const uint64_t limit = ((uint64_t)1 << g.np) - 1 - g.off;
   for (int64_t i = 0; i < g.C * g.L; ++i)
@@ -1279,6 +1319,7 @@ int ytm_set_weights(ytm_model* m, const float* in) {
     if (!(std::fabs(v) < 2147483648.0f) || std::nearbyint(v) != v)
       return fail(YTM_ERANGE, "clause weights must be integer-valued floats below 2^31 in magnitude");
   }
+  ++m->state_version;
   HIP_TRY(hipMemcpyAsync(m->d_w, in, (size_t)(m->g.C * m->g.K) * 4, hipMemcpyHostToDevice, m->stream));
   HIP_TRY(hipStreamSynchronize(m->stream));
   double bound = 0.0;

@@ -14,8 +14,6 @@ namespace ytm {
 hipError_t launch_encode(const uint32_t* X, int64_t N, uint32_t* out, const Geom& g, hipStream_t s);
 // Literal-major copy of encoded samples (several patches): XT [N][L][ceil(P/32)].
 hipError_t launch_transpose(const uint32_t* X, int64_t N, uint32_t* XT, const Geom& g, hipStream_t s);
-// Clears *ok unless every literal Lh + f of XT is the complement of literal f (ok set before).
-hipError_t launch_xt_halves_check(const uint32_t* XT, int64_t N, const Geom& g, int* ok, hipStream_t s);
 hipError_t launch_ta_to_planes(const uint32_t* ta, uint32_t* planes, const Geom& g, hipStream_t s);
 hipError_t launch_planes_to_ta(const uint32_t* planes, uint32_t* ta, const Geom& g, hipStream_t s);
 hipError_t launch_init_state(uint32_t* planes, float* w, const Geom& g, uint64_t seed, hipStream_t s);
@@ -52,6 +50,27 @@ hipError_t launch_score_wide(const uint32_t* planes, const float* w, const uint3
                              void* scratch, bool lists_ready, long long* acc, hipStream_t s);
 hipError_t launch_score_finish(const long long* acc, const float* bias, int64_t N, const Geom& g,
                                float* out, hipStream_t s);
+// Scoring on the matrix cores (ytm_matrix.hip).  steps 0: the model does not take it.  The
+// scratch (bytes) holds the clause operands, at need_at their thresholds and at weights_at the
+// weight operands; each sample needs a row of row_words firing words besides.
+struct MatrixPlan {
+  int steps;     // literal steps of 64
+  bool ternary;  // the product runs over the positive literals alone
+  int digits, groups;  // base-256 digits of a weight, column groups of the votes
+  int64_t row_words;
+  size_t need_at, weights_at, bytes;
+};
+// halves: the samples' negated literals are the complements of the positive ones; w_bound: an
+// upper bound of |weight|.
+MatrixPlan matrix_plan(const Geom& g, bool halves, double w_bound);
+hipError_t launch_matrix_pack(const uint32_t* planes, const float* w, const Geom& g, const MatrixPlan& p,
+                              void* scratch, hipStream_t s);
+// Class sums of N samples (encoded words X) into out (float [N][K]); masks: N * row_words words.
+hipError_t launch_matrix_score(const uint32_t* X, int64_t N, const Geom& g, const MatrixPlan& p, const void* scratch,
+                               int cus, const float* bias, uint32_t* masks, float* out, hipStream_t s);
+// Clears *ok unless every negated literal of the N samples' encoded rows is the complement of
+// its positive one (ok set before; models with appended negations).
+hipError_t launch_halves_check(const uint32_t* X, int64_t N, const Geom& g, int* ok, hipStream_t s);
 // Clause outputs; mode 0: any patch (N, C); 1: per patch (N, C, P); 2: per patch, bit-packed
 // (N, C, ceil(P/32)).
 hipError_t launch_transform(const uint32_t* planes, const int32_t* ninc, const uint32_t* X, int64_t N,
