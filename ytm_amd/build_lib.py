@@ -14,7 +14,7 @@ HERE = Path(__file__).resolve().parent
 ROOT = HERE.parent
 CSRC = HERE / "csrc"
 SOURCES = [CSRC / "ytm_kernels.hip", CSRC / "ytm_api.hip", CSRC / "ytm_jit.hip", CSRC / "ytm_binarize.hip",
-           CSRC / "ytm_matrix.hip"]
+           CSRC / "ytm_matrix.hip", CSRC / "ytm_memory.hip"]
 OUT = HERE / "libytm.so"
 # Device headers that the run-time specialised compile (hipRTC) needs, embedded as text.
 JIT_HEADERS = ["ytm_types.h", "ytm_device.h", "ytm_train.h"]

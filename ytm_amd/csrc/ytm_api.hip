@@ -156,23 +156,20 @@ int resolve_geometry(const ytm_params& p, Geom* out) {
 // A grow-only device buffer: *p holds at least bytes after a successful call.
 hipError_t ensure_buffer(void** p, size_t* have, size_t bytes) {
   if (*have >= bytes && *p) return hipSuccess;
-  if (*p) {
-    const hipError_t e = hipFree(*p);
-    if (e != hipSuccess) return e;
-  }
+  ytm::pool_free(*p);
   *p = nullptr;
   *have = 0;
-  const hipError_t e = hipMalloc(p, bytes > 0 ? bytes : 4);
+  const hipError_t e = ytm::pool_alloc(p, bytes);
   if (e == hipSuccess) *have = bytes;
   return e;
 }
 
 int ensure_slots(ytm_model* m, size_t bytes) {
   if (m->slots_bytes >= bytes) return YTM_OK;
-  if (m->d_slots) HIP_TRY(hipFree(m->d_slots));
+  ytm::pool_free(m->d_slots);
   m->d_slots = nullptr;
   m->slots_bytes = 0;
-  HIP_TRY(hipMalloc(&m->d_slots, bytes));
+  HIP_TRY(ytm::pool_alloc((void**)&m->d_slots, bytes));
   m->slots_bytes = bytes;
   return YTM_OK;
 }
@@ -223,7 +220,7 @@ size_t dtype_size(int dtype) {
 }
 
 int upload(void** dst, const void* src, size_t bytes, hipStream_t s) {
-  HIP_TRY(hipMalloc(dst, bytes > 0 ? bytes : 4));
+  HIP_TRY(ytm::pool_alloc(dst, bytes));
   if (bytes) HIP_TRY(hipMemcpyAsync(*dst, src, bytes, hipMemcpyHostToDevice, s));
   return YTM_OK;
 }
@@ -382,16 +379,17 @@ int fit_steps(ytm_model* m, const ytm_dataset* ds, int64_t first, int64_t count,
   rc = upload((void**)&d_drop, drop, (size_t)g.C * 4, m->stream);
   if (rc) return rc;
   if (inj) {
-    hipError_t e = hipMalloc(&d_inj, (size_t)(chunk * block) * 4);
+    hipError_t e = ytm::pool_alloc((void**)&d_inj, (size_t)(chunk * block) * 4);
     if (e != hipSuccess) {
-      (void)hipFree(d_drop);
+      (void)hipStreamSynchronize(m->stream);  // before the buffer is used again
+      ytm::pool_free(d_drop);
       return fail(YTM_EHIP, std::string("hipMalloc(inject) failed: ") + hipGetErrorString(e));
     }
   }
   auto finish = [&](int code) {
     (void)hipStreamSynchronize(m->stream);
-    (void)hipFree(d_drop);
-    if (d_inj) (void)hipFree(d_inj);
+    ytm::pool_free(d_drop);
+    ytm::pool_free(d_inj);
     return code;
   };
 #define BANK_TRY(expr)                                                                          \
@@ -465,6 +463,7 @@ const char* ytm_last_error(void) { return g_error.c_str(); }
 
 int ytm_shutdown(void) {
   const int failed = ytm::jit_unload_all();
+  ytm::memory_trim();
   if (failed) return fail(YTM_EHIP, std::to_string(failed) + " training-kernel module(s) failed to unload");
   return YTM_OK;
 }
@@ -497,14 +496,14 @@ int ytm_create(const ytm_params* params, ytm_model** out) {
   CREATE_TRY(hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking));
   CREATE_TRY(hipEventCreate(&m->ev0));
   CREATE_TRY(hipEventCreate(&m->ev1));
-  CREATE_TRY(hipMalloc(&m->d_planes, (size_t)(g.C * g.np * g.W) * 4));
-  CREATE_TRY(hipMalloc(&m->d_w, (size_t)(g.C * g.K) * 4));
-  CREATE_TRY(hipMalloc(&m->d_pw, (size_t)(g.C * g.P) * 4));
-  CREATE_TRY(hipMalloc(&m->d_bias, (size_t)g.K * 4));
-  CREATE_TRY(hipMalloc(&m->d_ninc, (size_t)g.C * 4));
-  CREATE_TRY(hipMalloc(&m->d_inv_rank, (size_t)(g.P + 1) * 4));
-  CREATE_TRY(hipMalloc(&m->d_counters, 128));
-  CREATE_TRY(hipMalloc(&m->d_err, 16));
+  CREATE_TRY(ytm::pool_alloc((void**)&m->d_planes, (size_t)(g.C * g.np * g.W) * 4));
+  CREATE_TRY(ytm::pool_alloc((void**)&m->d_w, (size_t)(g.C * g.K) * 4));
+  CREATE_TRY(ytm::pool_alloc((void**)&m->d_pw, (size_t)(g.C * g.P) * 4));
+  CREATE_TRY(ytm::pool_alloc((void**)&m->d_bias, (size_t)g.K * 4));
+  CREATE_TRY(ytm::pool_alloc((void**)&m->d_ninc, (size_t)g.C * 4));
+  CREATE_TRY(ytm::pool_alloc((void**)&m->d_inv_rank, (size_t)(g.P + 1) * 4));
+  CREATE_TRY(ytm::pool_alloc((void**)&m->d_counters, 128));
+  CREATE_TRY(ytm::pool_alloc((void**)&m->d_err, 16));
   std::vector<float> inv((size_t)g.P + 1);
   inv[0] = 0.0f;
   for (int64_t r = 1; r <= g.P; ++r) inv[r] = 1.0f / (float)r;  // IEEE fp32 division
@@ -524,7 +523,7 @@ void ytm_destroy(ytm_model* m) {
   void* bufs[] = {m->d_planes, m->d_w,    m->d_pw,   m->d_bias, m->d_ninc,  m->d_inv_rank,
                   m->d_counters, m->d_err, m->d_slots, m->d_sacc, m->d_sout, m->d_slists};
   for (void* b : bufs)
-    if (b) (void)hipFree(b);
+    ytm::pool_free(b);
   if (m->h_sout) (void)hipHostFree(m->h_sout);
   if (m->ev0) (void)hipEventDestroy(m->ev0);
   if (m->ev1) (void)hipEventDestroy(m->ev1);
@@ -617,10 +616,10 @@ int ytm_encode(ytm_model* m, const uint32_t* X, int64_t N, uint32_t* out) {
   const int64_t per = std::max<int64_t>(1, ((int64_t)1 << 30) / (g.P * g.W * 4));
   uint32_t *dX = nullptr, *dO = nullptr;
   const int64_t chunk = std::min(per, N);
-  HIP_TRY(hipMalloc(&dX, (size_t)(chunk * g.F) * 4));
-  hipError_t e = hipMalloc(&dO, (size_t)(chunk * g.P * g.W) * 4);
+  HIP_TRY(ytm::pool_alloc((void**)&dX, (size_t)(chunk * g.F) * 4));
+  hipError_t e = ytm::pool_alloc((void**)&dO, (size_t)(chunk * g.P * g.W) * 4);
   if (e != hipSuccess) {
-    (void)hipFree(dX);
+    ytm::pool_free(dX);
     return fail(YTM_EHIP, std::string("hipMalloc failed: ") + hipGetErrorString(e));
   }
   double ms_total = 0.0;
@@ -632,7 +631,7 @@ int ytm_encode(ytm_model* m, const uint32_t* X, int64_t N, uint32_t* out) {
     if (e == hipSuccess) e = ytm::launch_encode(dX, n, dO, g, m->stream);
     if (e == hipSuccess) e = hipEventRecord(m->ev1, m->stream);
     if (e == hipSuccess)
-      e = hipMemcpyAsync(out + s * g.P * g.W, dO, (size_t)(n * g.P * g.W) * 4, hipMemcpyDeviceToHost, m->stream);
+      e = ytm::copy_to_host(out + s * g.P * g.W, dO, (size_t)(n * g.P * g.W) * 4, m->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(m->stream);
     float ms = 0.0f;
     if (e == hipSuccess) e = hipEventElapsedTime(&ms, m->ev0, m->ev1);
@@ -640,8 +639,9 @@ int ytm_encode(ytm_model* m, const uint32_t* X, int64_t N, uint32_t* out) {
     if (e != hipSuccess) rc = fail(YTM_EHIP, std::string("encode failed: ") + hipGetErrorString(e));
   }
   m->stats.last_encode_kernel_ms = ms_total;
-  (void)hipFree(dX);
-  (void)hipFree(dO);
+  if (rc) (void)hipStreamSynchronize(m->stream);  // before the buffers are used again
+  ytm::pool_free(dX);
+  ytm::pool_free(dO);
   return rc;
 }
 
@@ -668,8 +668,8 @@ int ytm_encode_binarized(ytm_model* m, const void* X, int x_dtype, int64_t N, co
   uint32_t* dO = nullptr;
   int rc = upload(&dT, thresholds, (size_t)nthr * 8, m->stream);
   hipError_t e = hipSuccess;
-  if (!rc) e = hipMalloc(&dX, (size_t)(chunk * Fr) * es);
-  if (!rc && e == hipSuccess) e = hipMalloc((void**)&dO, (size_t)(chunk * g.P * g.W) * 4);
+  if (!rc) e = ytm::pool_alloc((void**)&dX, (size_t)(chunk * Fr) * es);
+  if (!rc && e == hipSuccess) e = ytm::pool_alloc((void**)&dO, (size_t)(chunk * g.P * g.W) * 4);
   double ms_total = 0.0;
   for (int64_t s = 0; !rc && e == hipSuccess && s < N; s += chunk) {
     const int64_t n = std::min(chunk, N - s);
@@ -681,7 +681,7 @@ int ytm_encode_binarized(ytm_model* m, const void* X, int x_dtype, int64_t N, co
                                     g, m->stream);
     if (e == hipSuccess) e = hipEventRecord(m->ev1, m->stream);
     if (e == hipSuccess)
-      e = hipMemcpyAsync(out + s * g.P * g.W, dO, (size_t)(n * g.P * g.W) * 4, hipMemcpyDeviceToHost, m->stream);
+      e = ytm::copy_to_host(out + s * g.P * g.W, dO, (size_t)(n * g.P * g.W) * 4, m->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(m->stream);
     float ms = 0.0f;
     if (e == hipSuccess) e = hipEventElapsedTime(&ms, m->ev0, m->ev1);
@@ -689,9 +689,10 @@ int ytm_encode_binarized(ytm_model* m, const void* X, int x_dtype, int64_t N, co
   }
   if (!rc && e != hipSuccess) rc = fail(YTM_EHIP, std::string("encode failed: ") + hipGetErrorString(e));
   m->stats.last_encode_kernel_ms = ms_total;
-  if (dT) (void)hipFree(dT);
-  if (dX) (void)hipFree(dX);
-  if (dO) (void)hipFree(dO);
+  if (rc) (void)hipStreamSynchronize(m->stream);  // before the buffers are used again
+  ytm::pool_free(dT);
+  ytm::pool_free(dX);
+  ytm::pool_free(dO);
   return rc;
 }
 
@@ -707,12 +708,12 @@ int ytm_dataset_create(ytm_model* m, const uint32_t* encX, const int32_t* encY, 
     // elsewhere may not, so training and scoring rely on it only where this check holds.
     int* d_ok = nullptr;
     int ok = 1;
-    hipError_t e = hipMalloc(&d_ok, sizeof(int));
+    hipError_t e = ytm::pool_alloc((void**)&d_ok, sizeof(int));
     if (e == hipSuccess) e = hipMemcpyAsync(d_ok, &ok, sizeof(int), hipMemcpyHostToDevice, m->stream);
     if (e == hipSuccess) e = ytm::launch_halves_check(ds->d_X, N, g, d_ok, m->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(&ok, d_ok, sizeof(int), hipMemcpyDeviceToHost, m->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(m->stream);
-    if (d_ok) (void)hipFree(d_ok);
+    ytm::pool_free(d_ok);
     if (e != hipSuccess) rc = fail(YTM_EHIP, std::string("sample check: ") + hipGetErrorString(e));
     ds->halves = ok == 1;
   }
@@ -721,10 +722,10 @@ int ytm_dataset_create(ytm_model* m, const uint32_t* encX, const int32_t* encY, 
     // Several patches: the training kernel evaluates clauses on a literal-major copy, and so
     // do the scorers of models that the matrix cores do not take.
     const size_t bytes = (size_t)(N * g.L * ((g.P + 31) / 32)) * 4;
-    hipError_t e = hipMalloc(&ds->d_XT, bytes);
+    hipError_t e = ytm::pool_alloc((void**)&ds->d_XT, bytes);
     if (e == hipSuccess) e = ytm::launch_transpose(ds->d_X, N, ds->d_XT, g, m->stream);
     // the order of the training kernels' literal lists, from the densities of the first samples
-    if (e == hipSuccess) e = hipMalloc(&ds->d_order, (size_t)ytm::kOrderBuckets * g.W * 4);
+    if (e == hipSuccess) e = ytm::pool_alloc((void**)&ds->d_order, (size_t)ytm::kOrderBuckets * g.W * 4);
     if (e == hipSuccess) e = ytm::launch_literal_order(nullptr, ds->d_XT, N, g, ds->d_order, m->stream);
     if (e != hipSuccess) rc = fail(YTM_EHIP, std::string("literal-major copy: ") + hipGetErrorString(e));
   }
@@ -733,6 +734,7 @@ int ytm_dataset_create(ytm_model* m, const uint32_t* encX, const int32_t* encY, 
     if (e != hipSuccess) rc = fail(YTM_EHIP, hipGetErrorString(e));
   }
   if (rc) {
+    (void)hipStreamSynchronize(m->stream);  // before the buffers are used again
     ytm_dataset_destroy(ds);
     return rc;
   }
@@ -742,10 +744,10 @@ int ytm_dataset_create(ytm_model* m, const uint32_t* encX, const int32_t* encY, 
 
 void ytm_dataset_destroy(ytm_dataset* ds) {
   if (!ds) return;
-  if (ds->d_X) (void)hipFree(ds->d_X);
-  if (ds->d_Y) (void)hipFree(ds->d_Y);
-  if (ds->d_XT) (void)hipFree(ds->d_XT);
-  if (ds->d_order) (void)hipFree(ds->d_order);
+  ytm::pool_free(ds->d_X);
+  ytm::pool_free(ds->d_Y);
+  ytm::pool_free(ds->d_XT);
+  ytm::pool_free(ds->d_order);
   delete ds;
 }
 
@@ -889,16 +891,17 @@ int fit_range(ytm_model* m, const ytm_dataset* ds, int64_t first, int64_t count,
   rc = upload((void**)&d_drop, drop, (size_t)g.C * 4, m->stream);
   if (rc) return rc;
   if (inj) {
-    hipError_t e = hipMalloc(&d_inj, (size_t)(per_launch * block) * 4);
+    hipError_t e = ytm::pool_alloc((void**)&d_inj, (size_t)(per_launch * block) * 4);
     if (e != hipSuccess) {
-      (void)hipFree(d_drop);
+      (void)hipStreamSynchronize(m->stream);  // before the buffer is used again
+      ytm::pool_free(d_drop);
       return fail(YTM_EHIP, std::string("hipMalloc(inject) failed: ") + hipGetErrorString(e));
     }
   }
   auto finish = [&](int code) {
     (void)hipStreamSynchronize(m->stream);
-    if (d_drop) (void)hipFree(d_drop);
-    if (d_inj) (void)hipFree(d_inj);
+    ytm::pool_free(d_drop);
+    ytm::pool_free(d_inj);
     return code;
   };
 #define FIT_TRY(expr)                                                                           \
@@ -1242,10 +1245,10 @@ int ytm_transform(ytm_model* m, const uint32_t* encX, int64_t N, int mode, uint3
   chunk = chunk < 1 ? 1 : (chunk > N ? N : chunk);
   uint32_t *dX = nullptr, *dXT = nullptr, *dO = nullptr;
   void* dL = nullptr;
-  hipError_t e = hipMalloc(&dX, (size_t)(chunk * g.P * g.W) * 4);
-  if (e == hipSuccess) e = hipMalloc(&dO, (size_t)(chunk * per_out) * 4);
-  if (e == hipSuccess && lm) e = hipMalloc(&dXT, (size_t)(chunk * g.L * PW) * 4);
-  if (e == hipSuccess && lists_bytes) e = hipMalloc(&dL, lists_bytes);
+  hipError_t e = ytm::pool_alloc((void**)&dX, (size_t)(chunk * g.P * g.W) * 4);
+  if (e == hipSuccess) e = ytm::pool_alloc((void**)&dO, (size_t)(chunk * per_out) * 4);
+  if (e == hipSuccess && lm) e = ytm::pool_alloc((void**)&dXT, (size_t)(chunk * g.L * PW) * 4);
+  if (e == hipSuccess && lists_bytes) e = ytm::pool_alloc((void**)&dL, lists_bytes);
   if (e == hipSuccess) e = ytm::launch_ninc(m->d_planes, m->d_ninc, g, m->stream);
   for (int64_t first = 0; e == hipSuccess && first < N; first += chunk) {
     const int64_t n = N - first < chunk ? N - first : chunk;
@@ -1260,14 +1263,15 @@ int ytm_transform(ytm_model* m, const uint32_t* encX, int64_t N, int mode, uint3
       e = ytm::launch_transform(m->d_planes, m->d_ninc, dX, n, g, mode, dO, m->stream);
     }
     if (e == hipSuccess)
-      e = hipMemcpyAsync(out + first * per_out, dO, (size_t)(n * per_out) * 4, hipMemcpyDeviceToHost, m->stream);
+      e = ytm::copy_to_host(out + first * per_out, dO, (size_t)(n * per_out) * 4, m->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(m->stream);
   }
   const int rc = e == hipSuccess ? YTM_OK : fail(YTM_EHIP, std::string("transform failed: ") + hipGetErrorString(e));
-  if (dX) (void)hipFree(dX);
-  if (dO) (void)hipFree(dO);
-  if (dXT) (void)hipFree(dXT);
-  if (dL) (void)hipFree(dL);
+  if (rc) (void)hipStreamSynchronize(m->stream);  // before the buffers are used again
+  ytm::pool_free(dX);
+  ytm::pool_free(dO);
+  ytm::pool_free(dXT);
+  ytm::pool_free(dL);
   return rc;
 }
 
@@ -1275,11 +1279,12 @@ int ytm_get_ta_state(ytm_model* m, uint32_t* out) {
   if (!m || !out) return fail(YTM_EINVAL, "null argument");
   const Geom& g = m->g;
   uint32_t* d = nullptr;
-  HIP_TRY(hipMalloc(&d, (size_t)(g.C * g.L) * 4));
+  HIP_TRY(ytm::pool_alloc((void**)&d, (size_t)(g.C * g.L) * 4));
   hipError_t e = ytm::launch_planes_to_ta(m->d_planes, d, g, m->stream);
-  if (e == hipSuccess) e = hipMemcpyAsync(out, d, (size_t)(g.C * g.L) * 4, hipMemcpyDeviceToHost, m->stream);
+  if (e == hipSuccess) e = ytm::copy_to_host(out, d, (size_t)(g.C * g.L) * 4, m->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(m->stream);
-  (void)hipFree(d);
+  if (e != hipSuccess) (void)hipStreamSynchronize(m->stream);  // before the buffer is used again
+  ytm::pool_free(d);
   if (e != hipSuccess) return fail(YTM_EHIP, std::string("get_ta_state failed: ") + hipGetErrorString(e));
   return YTM_OK;
 }
@@ -1296,10 +1301,15 @@ int ytm_set_ta_state(ytm_model* m, const uint32_t* in) {
                                   std::to_string(limit));
   uint32_t* d = nullptr;
   int rc = upload((void**)&d, in, (size_t)(g.C * g.L) * 4, m->stream);
-  if (rc) return rc;
+  if (rc) {
+    (void)hipStreamSynchronize(m->stream);
+    ytm::pool_free(d);
+    return rc;
+  }
   hipError_t e = ytm::launch_ta_to_planes(d, m->d_planes, g, m->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(m->stream);
-  (void)hipFree(d);
+  if (e != hipSuccess) (void)hipStreamSynchronize(m->stream);  // before the buffer is used again
+  ytm::pool_free(d);
   if (e != hipSuccess) return fail(YTM_EHIP, std::string("set_ta_state failed: ") + hipGetErrorString(e));
   note_reload(m, 1);
   return YTM_OK;
@@ -1307,8 +1317,7 @@ int ytm_set_ta_state(ytm_model* m, const uint32_t* in) {
 
 int ytm_get_weights(ytm_model* m, float* out) {
   if (!m || !out) return fail(YTM_EINVAL, "null argument");
-  HIP_TRY(hipMemcpyAsync(out, m->d_w, (size_t)(m->g.C * m->g.K) * 4, hipMemcpyDeviceToHost, m->stream));
-  HIP_TRY(hipStreamSynchronize(m->stream));
+  HIP_TRY(ytm::copy_to_host(out, m->d_w, (size_t)(m->g.C * m->g.K) * 4, m->stream));
   return YTM_OK;
 }
 
@@ -1331,8 +1340,7 @@ int ytm_set_weights(ytm_model* m, const float* in) {
 
 int ytm_get_patch_weights(ytm_model* m, int32_t* out) {
   if (!m || !out) return fail(YTM_EINVAL, "null argument");
-  HIP_TRY(hipMemcpyAsync(out, m->d_pw, (size_t)(m->g.C * m->g.P) * 4, hipMemcpyDeviceToHost, m->stream));
-  HIP_TRY(hipStreamSynchronize(m->stream));
+  HIP_TRY(ytm::copy_to_host(out, m->d_pw, (size_t)(m->g.C * m->g.P) * 4, m->stream));
   return YTM_OK;
 }
 
@@ -1378,14 +1386,15 @@ int ytm_binarize(const void* X, int x_dtype, int64_t n, const void* thresholds, 
   int rc = upload(&dX, X, (size_t)n * es, nullptr);
   if (!rc) rc = upload(&dT, thresholds, (size_t)nthr * 8, nullptr);
   hipError_t e = hipSuccess;
-  if (!rc) e = hipMalloc(&dO, (size_t)(n * width) * 4);
+  if (!rc) e = ytm::pool_alloc((void**)&dO, (size_t)(n * width) * 4);
   if (!rc && e == hipSuccess)
     e = ytm::launch_binarize(dX, x_dtype, n, dT, int_thresholds != 0, nthr, kind == 1, edge_bins != 0, dO, nullptr);
-  if (!rc && e == hipSuccess) e = hipMemcpy(out, dO, (size_t)(n * width) * 4, hipMemcpyDeviceToHost);
+  if (!rc && e == hipSuccess) e = ytm::copy_to_host(out, dO, (size_t)(n * width) * 4, nullptr);
   if (!rc && e != hipSuccess) rc = fail(YTM_EHIP, std::string("binarize failed: ") + hipGetErrorString(e));
-  if (dX) (void)hipFree(dX);
-  if (dT) (void)hipFree(dT);
-  if (dO) (void)hipFree(dO);
+  if (rc) (void)hipStreamSynchronize(nullptr);  // before the buffers are used again
+  ytm::pool_free(dX);
+  ytm::pool_free(dT);
+  ytm::pool_free(dO);
   return rc;
 }
 
@@ -1397,13 +1406,14 @@ int ytm_collapse_bins(const uint32_t* B, int64_t rows, int64_t width, int kind, 
   int64_t* dO = nullptr;
   int rc = upload(&dB, B, (size_t)(rows * width) * 4, nullptr);
   hipError_t e = hipSuccess;
-  if (!rc) e = hipMalloc(&dO, (size_t)rows * 8);
+  if (!rc) e = ytm::pool_alloc((void**)&dO, (size_t)rows * 8);
   if (!rc && e == hipSuccess)
     e = ytm::launch_collapse_bins((const uint32_t*)dB, rows, width, kind == 1, edge_bins != 0, dO, nullptr);
-  if (!rc && e == hipSuccess) e = hipMemcpy(out, dO, (size_t)rows * 8, hipMemcpyDeviceToHost);
+  if (!rc && e == hipSuccess) e = ytm::copy_to_host(out, dO, (size_t)rows * 8, nullptr);
   if (!rc && e != hipSuccess) rc = fail(YTM_EHIP, std::string("collapse_bins failed: ") + hipGetErrorString(e));
-  if (dB) (void)hipFree(dB);
-  if (dO) (void)hipFree(dO);
+  if (rc) (void)hipStreamSynchronize(nullptr);  // before the buffers are used again
+  ytm::pool_free(dB);
+  ytm::pool_free(dO);
   return rc;
 }
 

@@ -11,6 +11,15 @@
 
 namespace ytm {
 
+// Device memory of the current device, kept between calls (ytm_memory.hip).  Blocks come with
+// whatever they held before; a block is freed once nothing on the GPU uses it any more.
+hipError_t pool_alloc(void** p, size_t bytes);
+void pool_free(void* p);
+// Copies device memory to a host array after the work of stream s; done on return.
+hipError_t copy_to_host(void* dst, const void* src, size_t bytes, hipStream_t s);
+// Gives everything kept back to the devices and the host.
+void memory_trim();
+
 hipError_t launch_encode(const uint32_t* X, int64_t N, uint32_t* out, const Geom& g, hipStream_t s);
 // Literal-major copy of encoded samples (several patches): XT [N][L][ceil(P/32)].
 hipError_t launch_transpose(const uint32_t* X, int64_t N, uint32_t* XT, const Geom& g, hipStream_t s);
