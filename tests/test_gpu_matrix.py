@@ -121,6 +121,42 @@ def test_operands_follow_the_model():
     check(tm, ref, enc)
 
 
+@pytest.mark.parametrize("bits,clauses,n", [
+    (600, 70, 1),      # one sample
+    (33, 40, 31),      # 2 steps, a tile less one
+    (32, 33, 33),      # 1 step made 2, a tile and one
+    (200, 2000, 65),   # few samples: a block per tile
+    (784, 300, 7000),  # many samples: 256 by 256 tiles, a partial one in each direction
+    (100, 8200, 257),  # 257 clause tiles
+    (2111, 257, 8193),
+    (513, 40, 40001),  # one clause tile beyond the first of a block
+])
+def test_one_patch(bits, clauses, n):
+    rng = np.random.default_rng(8)
+    tm, ref = pair(clauses, (bits, 1, 1), 5, rng)
+    enc = tm.encode(image(rng, n, (bits, 1, 1)))
+    want = check(tm, ref, enc)
+    assert np.unique(want).size > 1
+    odd = enc & rng.integers(0, 2**32, enc.shape, dtype=np.uint32)  # negations are not complements
+    check(tm, ref, odd)
+    check(tm, ref, enc)
+
+
+@pytest.mark.parametrize("bits,clauses,n,negated", [(90, 64, 300, False), (1000, 33, 70000, False),
+                                                    (10000, 40, 7000, True), (10000, 7000, 300, True)])
+def test_one_patch_without_allocation(bits, clauses, n, negated):
+    """The allocation-free scorer: operands and samples in the scratch, in one pass and several,
+    and the literal lists where the operands exceed it (7000 clauses of 20000 literals)."""
+    from test_zz_no_alloc import score_both
+
+    rng = np.random.default_rng(9)
+    tm, ref = pair(clauses, (bits, 1, 1), 4, rng, append_negated=negated)
+    enc = tm.encode(image(rng, n, (bits, 1, 1)))
+    got, noalloc = score_both(tm, tm._device_data(enc), 4)
+    np.testing.assert_array_equal(got, noalloc)
+    np.testing.assert_array_equal(got[:200], ref.score(enc[:200]))
+
+
 def test_literal_lists_of_wide_patches(monkeypatch):
     """Patches of more literals than the product's registers hold keep the literal-list scorer:
     blocks over every clause of a sample and over chunks of 4096 clauses."""

@@ -61,21 +61,31 @@ hipError_t launch_score_finish(const long long* acc, const float* bias, int64_t 
                                float* out, hipStream_t s);
 // Scoring on the matrix cores (ytm_matrix.hip).  steps 0: the model does not take it.  The
 // scratch (bytes) holds the clause operands, at need_at their thresholds and at weights_at the
-// weight operands; each sample needs a row of row_words firing words besides.
+// weight operands; N samples scored together need matrix_rows_bytes besides: a row of
+// row_words firing words each and, with one patch, their operands (sample_bytes each).
 struct MatrixPlan {
   int steps;     // literal steps of 64
   bool ternary;  // the product runs over the positive literals alone
+  int half_steps;  // > 0 (one patch): the samples are looked at as they are scored, and the product
+                   // takes the operands over the positive literals (at half_at) where it may
   int digits, groups;  // base-256 digits of a weight, column groups of the votes
   int64_t row_words;
-  size_t need_at, weights_at, bytes;
+  size_t sample_bytes;
+  size_t half_at, need_at, flag_at, weights_at, bytes;
 };
-// halves: the samples' negated literals are the complements of the positive ones; w_bound: an
-// upper bound of |weight|.
-MatrixPlan matrix_plan(const Geom& g, bool halves, double w_bound);
+// halves: the N samples' negated literals are the complements of the positive ones (1), are not
+// (0), or may be (-1, one patch); w_bound: an upper bound of |weight|.
+MatrixPlan matrix_plan(const Geom& g, int halves, double w_bound, int64_t N);
 hipError_t launch_matrix_pack(const uint32_t* planes, const float* w, const Geom& g, const MatrixPlan& p,
                               void* scratch, hipStream_t s);
-// Class sums of N samples (encoded words X) into out (float [N][K]); masks: N * row_words words.
-hipError_t launch_matrix_score(const uint32_t* X, int64_t N, const Geom& g, const MatrixPlan& p, const void* scratch,
+// One patch: N samples are so few that a block per product tile takes them.
+bool few_rows(const Geom& g, int64_t N);
+// One patch: the product of N samples over all literals takes 70 us or more, twice that over the
+// positive ones.
+bool long_rows(const Geom& g, int64_t N);
+size_t matrix_rows_bytes(const MatrixPlan& p, int64_t N);
+// Class sums of N samples (encoded words X) into out (float [N][K]); masks: matrix_rows_bytes.
+hipError_t launch_matrix_score(const uint32_t* X, int64_t N, const Geom& g, const MatrixPlan& p, void* scratch,
                                int cus, const float* bias, uint32_t* masks, float* out, hipStream_t s);
 // Clears *ok unless every negated literal of the N samples' encoded rows is the complement of
 // its positive one (ok set before; models with appended negations).

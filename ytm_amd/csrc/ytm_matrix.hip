@@ -11,8 +11,8 @@
 // does, 65536 literal tests an instruction of 32 cycles.
 //
 // Scoring (calc_class_sums_infer_batch, kernel.cu:319-343) then has three steps: the include
-// masks become FP4 fragments (pack_clauses_kernel, kept while the model is unchanged), a
-// product gives each sample's firing clauses as a bit row (fire_patches_kernel), and a second
+// masks become FP4 fragments (pack_model_kernel, kept while the model is unchanged), a
+// product gives each sample's firing clauses as a bit row (fire_patches_kernel, fire_rows_kernel), and a second
 // product, of these bits and the weights' base-256 digits on the int8 matrix cores, gives the
 // class sums (votes_kernel).
 #include <hip/hip_runtime.h>
@@ -68,46 +68,106 @@ __device__ __forceinline__ uint32_t bits_at(const uint32_t* m, int64_t W, int64_
   return left >= 32 ? v : v & ((1u << left) - 1u);
 }
 
-// Clause operands: frag[tile of 32 clauses][step][lane], lane l holding 32 values (literals
-// 64 step + 32 (l / 32) ...) of clause 32 tile + l % 32; zero past the last clause or literal.
-__global__ __launch_bounds__(256) void pack_clauses_kernel(const uint32_t* __restrict__ planes, Geom g, int steps,
-                                                           int ternary, v4i* __restrict__ frag) {
+// Whether word j of the encoded row x's positive literals is the complement of the negated ones.
+__device__ __forceinline__ bool complements(const uint32_t* x, const Geom& g, int64_t j) {
+  const uint32_t valid = g.Lh - 32 * j >= 32 ? 0xFFFFFFFFu : (1u << (g.Lh - 32 * j)) - 1u;
+  return (bits_at(x, g.W, 0, g.Lh, j) ^ bits_at(x, g.W, g.Lh, g.Lh, j)) == valid;
+}
+
+// The model's operands, three independent parts of one launch (after every change of the model
+// and before its first score: 784 bits, 2000 clauses 15.6 us in a launch each, 9.2 us in one):
+//  - clause operands frag[tile of 32 clauses][step][lane], lane l holding 32 values (literals
+//    64 step + 32 (l / 32) ...) of clause 32 tile + l % 32; zero past the last clause or literal;
+//  - thresholds need[32 tiles]: the value a clause's product reaches where it fires, plus the
+//    1 that the products start from; a wave per clause;
+//  - weight operands wfrag[word of 32 clauses][column group][lane], lane l holding 16 int8
+//    values (clauses 32 word + 16 (l / 32) ...) of column l % 32: digit col % D of class
+//    group * (32 / D) + col / D, the weights in signed base-256 digits, least significant first.
+// With half_steps, operands and thresholds over the positive literals alone come besides.
+__global__ __launch_bounds__(256) void pack_model_kernel(const uint32_t* __restrict__ planes,
+                                                         const float* __restrict__ w, Geom g, MatrixPlan p,
+                                                         unsigned char* __restrict__ base, int64_t need_blocks,
+                                                         int64_t weight_blocks) {
+  v4i* frag = (v4i*)base;
+  v4i* half = (v4i*)(base + p.half_at);
+  float* need = (float*)(base + p.need_at);
+  v4i* wfrag = (v4i*)(base + p.weights_at);
   const int64_t ct = (g.C + kTile - 1) / kTile;
-  const int64_t n = ternary ? g.Lh : g.L;
-  for (int64_t idx = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; idx < ct * steps * kWave;
-       idx += (int64_t)gridDim.x * blockDim.x) {
+  const int64_t n = p.ternary ? g.Lh : g.L;
+  if (blockIdx.x < need_blocks) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) *(int*)(base + p.flag_at) = 0;
+    const int lane = lane_id();
+    const int64_t nwaves = need_blocks * blockDim.x / kWave;
+    for (int64_t c = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) / kWave; c < ct * kTile; c += nwaves) {
+      int pos = 0, first = 0, all = 0;
+      if (c < g.C) {
+        const uint32_t* m = planes + (c * g.np + g.np - 1) * g.W;
+        for (int64_t j = lane; j < g.W; j += kWave) {
+          pos += __popc(bits_at(m, g.W, 0, n, j));
+          first += __popc(bits_at(m, g.W, 0, g.Lh, j));
+          all |= m[j] != 0u;
+        }
+      }
+      pos = wave_sum_i32(pos);
+      first = wave_sum_i32(first);
+      const bool empty = !__any(all);
+      if (lane == 0) {
+        need[c] = empty ? kNever : (float)(pos + 1);
+        if (p.half_steps) need[ct * kTile + c] = empty ? kNever : (float)(first + 1);
+      }
+    }
+    return;
+  }
+  int64_t first = blockIdx.x - need_blocks;
+  if (first < weight_blocks) {
+    const int per = kTile / p.digits;
+    for (int64_t idx = first * (int64_t)blockDim.x + threadIdx.x; idx < p.row_words * p.groups * kWave;
+         idx += weight_blocks * (int64_t)blockDim.x) {
+      const int l = (int)(idx % kWave), grp = (int)(idx / kWave % p.groups);
+      const int64_t c0 = idx / kWave / p.groups * kTile + 16 * (l >> 5);
+      const int col = l & 31, k = grp * per + col / p.digits, digit = col % p.digits;
+      v4i r;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        uint32_t word = 0u;
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+          const int64_t c = c0 + 4 * q + b;
+          long long v = c < g.C && col / p.digits < per && k < g.K ? (long long)w[c * g.K + k] : 0;
+          int d = 0;
+          for (int i = 0; i <= digit; ++i) {
+            d = (int)(signed char)(v & 255);
+            v = (v - d) >> 8;
+          }
+          word |= (uint32_t)(d & 255) << (8 * b);
+        }
+        r[q] = (int)word;
+      }
+      wfrag[idx] = r;
+    }
+    return;
+  }
+  first -= weight_blocks;
+  const int64_t blocks = gridDim.x - need_blocks - weight_blocks;
+  const int each = p.steps + p.half_steps;
+  for (int64_t idx = first * (int64_t)blockDim.x + threadIdx.x; idx < ct * each * kWave;
+       idx += blocks * (int64_t)blockDim.x) {
     const int l = (int)(idx % kWave);
-    const int64_t s = idx / kWave % steps, c = idx / kWave / steps * kTile + (l & 31);
-    const int64_t j = 2 * s + (l >> 5);
+    const int64_t tile = idx / kWave / each, c = tile * kTile + (l & 31);
+    const int st = (int)(idx / kWave % each), s = st < p.steps ? st : st - p.steps;
+    const bool ternary = p.ternary || st >= p.steps;
+    const int64_t j = 2 * (int64_t)s + (l >> 5);
     uint32_t pos = 0u, neg = 0u;
     if (c < g.C) {
       const uint32_t* m = planes + (c * g.np + g.np - 1) * g.W;
-      pos = bits_at(m, g.W, 0, n, j);
+      pos = bits_at(m, g.W, 0, ternary ? g.Lh : g.L, j);
       if (ternary) neg = bits_at(m, g.W, g.Lh, g.Lh, j);
     }
-    frag[idx] = fp4_of(pos ^ neg, neg & ~pos);
-  }
-}
-
-// The value a clause's product reaches where it fires, plus the 1 that the products start
-// from; a wave per clause.  [32 tiles] floats.
-__global__ __launch_bounds__(256) void clause_need_kernel(const uint32_t* __restrict__ planes, Geom g, int ternary,
-                                                          float* __restrict__ need) {
-  const int lane = lane_id();
-  const int64_t n = ternary ? g.Lh : g.L, rows = (g.C + kTile - 1) / kTile * kTile;
-  const int64_t nwaves = (int64_t)gridDim.x * blockDim.x / kWave;
-  for (int64_t c = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) / kWave; c < rows; c += nwaves) {
-    int pos = 0, all = 0;
-    if (c < g.C) {
-      const uint32_t* m = planes + (c * g.np + g.np - 1) * g.W;
-      for (int64_t j = lane; j < g.W; j += kWave) {
-        pos += __popc(bits_at(m, g.W, 0, n, j));
-        all |= m[j] != 0u;
-      }
-    }
-    pos = wave_sum_i32(pos);
-    const bool empty = !__any(all);
-    if (lane == 0) need[c] = empty ? kNever : (float)(pos + 1);
+    const v4i v = fp4_of(pos ^ neg, neg & ~pos);
+    if (st < p.steps)
+      frag[(tile * p.steps + s) * kWave + l] = v;
+    else
+      half[(tile * p.half_steps + s) * kWave + l] = v;
   }
 }
 
@@ -271,36 +331,196 @@ __global__ __launch_bounds__(64 * WAVES) void fire_patches_kernel(const uint32_t
   }
 }
 
-// Weight operands of votes_kernel: frag[word of 32 clauses][column group][lane], lane l holding
-// 16 int8 values (clauses 32 word + 16 (l / 32) ...) of column l % 32: digit col % D of class
-// group * (32 / D) + col / D, the weights in signed base-256 digits, least significant first.
-__global__ __launch_bounds__(256) void pack_weights_kernel(const float* __restrict__ w, Geom g, int64_t words, int D,
-                                                           int groups, v4i* __restrict__ frag) {
-  const int per = kTile / D;
-  for (int64_t idx = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; idx < words * groups * kWave;
+// One patch: the rows of a product tile are samples.
+
+// Sample operands of fire_rows_kernel: frag[tile of 32 samples][step][lane], zero past the last
+// sample's words (the rows past the last sample repeat it).  With half_steps, sets *odd when a
+// sample's negated literals are not the complements of its positive ones.
+__global__ __launch_bounds__(256) void pack_samples_kernel(const uint32_t* __restrict__ X, int64_t N, Geom g,
+                                                           int steps, int half_steps, int* odd,
+                                                           v4i* __restrict__ frag) {
+  const int64_t total = (N + kTile - 1) / kTile * steps * kWave;
+  const int64_t hw = half_steps ? (g.Lh + 31) / 32 : 0;
+  bool bad = false;
+  for (int64_t idx = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; idx < total;
        idx += (int64_t)gridDim.x * blockDim.x) {
-    const int l = (int)(idx % kWave), grp = (int)(idx / kWave % groups);
-    const int64_t c0 = idx / kWave / groups * kTile + 16 * (l >> 5);
-    const int col = l & 31, k = grp * per + col / D, digit = col % D;
-    v4i r;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      uint32_t word = 0u;
-#pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        const int64_t c = c0 + 4 * q + b;
-        long long v = c < g.C && col / D < per && k < g.K ? (long long)w[c * g.K + k] : 0;
-        int d = 0;
-        for (int i = 0; i <= digit; ++i) {
-          d = (int)(signed char)(v & 255);
-          v = (v - d) >> 8;
-        }
-        word |= (uint32_t)(d & 255) << (8 * b);
-      }
-      r[q] = (int)word;
-    }
-    frag[idx] = r;
+    const int l = (int)(idx % kWave);
+    const int64_t w = idx / kWave % steps * 2 + (l >> 5), e = idx / kWave / steps * kTile + (l & 31);
+    const uint32_t* x = X + (e < N ? e : N - 1) * g.W;
+    frag[idx] = fp4_of(w < g.W ? x[w] : 0u, 0u);
+    if (w < hw) bad = bad || !complements(x, g, w);
   }
+  if (bad) *odd = 1;
+}
+
+// The firing words of a product tile, from its sums d (a lane: one clause, 16 samples) and the
+// lane's threshold: lane i < 32 returns sample i's word, bit j = clause j.
+__device__ __forceinline__ uint32_t row_words_of(const v16f& d, float want) {
+  const int lane = lane_id();
+  const int mine = ((lane >> 3) & 3) << 2 | (lane & 3);  // the register that holds sample `lane`
+  uint32_t word = 0u;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    const unsigned long long hit = __ballot(d[r] == want);
+    const uint32_t w = (lane >> 2) & 1 ? (uint32_t)(hit >> 32) : (uint32_t)hit;
+    word = mine == r ? w : word;
+  }
+  return word;
+}
+
+// Firing clauses of one-patch samples, bit c % 32 of masks[e][c / 32]: a product of 256 samples
+// by 256 clauses per block, each of its 8 waves 128 by 64 (eight tiles whose sums stay in
+// registers).  Both operands stream through four LDS buffers of two steps, copied there
+// directly from global memory three buffers ahead, which covers the latency of a line that
+// another XCD's L2 or the memory holds; six operand reads serve eight product instructions.
+// Consecutive blocks go to different XCDs, so the block index is split such that an XCD works
+// on neighbouring tiles and finds their operands in its own L2.
+// Bound by the matrix cores, behind them by the operands' way through LDS.  20000 literals,
+// 10000 clauses, 10000 samples: 3.77 ms with include masks and literal lists, 0.46 ms now, of
+// them 0.43 here; the products alone would take 0.27 ms.
+constexpr int kRowSteps = 2, kRowBuffers = 4, kBlockTiles = 8;
+// Samples not yet looked at (half_steps): *odd says whether the product over the positive
+// literals alone, in its own operands, will do; the samples' operands begin alike.
+__global__ __launch_bounds__(512) void fire_rows_kernel(const v4i* __restrict__ sfrag, int64_t N, int64_t C,
+                                                        const unsigned char* __restrict__ base, MatrixPlan p,
+                                                        uint32_t* __restrict__ masks) {
+  constexpr int MT = 4, NT = 2;
+  constexpr int kBufFrags = 2 * kBlockTiles * kRowSteps;  // samples, then clauses
+  extern __shared__ __attribute__((aligned(16))) unsigned char s_mem[];
+  const int lane = lane_id();
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
+  const int64_t mtiles = (N + kTile - 1) / kTile, ctiles = (C + kTile - 1) / kTile;
+  const int64_t mb = (mtiles + kBlockTiles - 1) / kBlockTiles, cb = (ctiles + kBlockTiles - 1) / kBlockTiles;
+  const int64_t nblk = mb * cb, share = (nblk + 7) / 8;
+  const bool half = p.half_steps && *(const int*)(base + p.flag_at) == 0;
+  const v4i* cfrag = (const v4i*)(base + (half ? p.half_at : 0));
+  const float* need = (const float*)(base + p.need_at) + (half ? ctiles * kTile : 0);
+  const int steps = half ? p.half_steps : p.steps, nstage = steps / kRowSteps;
+  const int64_t row_words = p.row_words;
+  for (int64_t blk = blockIdx.x; blk < 8 * share; blk += gridDim.x) {
+    const int64_t idx = blk % 8 * share + blk / 8;  // this XCD's range
+    if (idx >= nblk) continue;
+    // columns of four sample blocks: their tiles share clause operands
+    const int64_t grp = idx / (4 * cb), first = grp * 4, rows = mb - first < 4 ? mb - first : 4;
+    const int64_t in = idx - grp * 4 * cb;
+    const int64_t m0 = (first + in % rows) * kBlockTiles, c0 = in / rows * kBlockTiles;
+    // The wave's copies of stage st: one tile of samples and one of clauses, both steps
+    const int64_t mt = m0 + wave < mtiles ? m0 + wave : mtiles - 1, ct = c0 + wave < ctiles ? c0 + wave : ctiles - 1;
+    const v4i* sa = sfrag + mt * p.steps * kWave + lane;
+    const v4i* sb = cfrag + ct * steps * kWave + lane;
+    auto fill = [&](int st) {
+      const int at = (st < nstage ? st : nstage - 1) * kRowSteps;  // past the end: copied again, not read
+      unsigned char* dst = s_mem + (st & (kRowBuffers - 1)) * kBufFrags * kFragBytes;
+#pragma unroll
+      for (int k = 0; k < kRowSteps; ++k) {
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(sa + (at + k) * kWave),
+                                         (__attribute__((address_space(3))) void*)(dst + (k * kBlockTiles + wave) * kFragBytes),
+                                         16, 0, 0);
+        __builtin_amdgcn_global_load_lds(
+            (const __attribute__((address_space(1))) void*)(sb + (at + k) * kWave),
+            (__attribute__((address_space(3))) void*)(dst + ((kRowSteps + k) * kBlockTiles + wave) * kFragBytes), 16, 0, 0);
+      }
+    };
+    __syncthreads();  // the buffers are no longer read
+    for (int st = 0; st < kRowBuffers - 1; ++st) fill(st);
+    v16f d[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) d[i][j][r] = 1.0f;
+    const int wm = (wave & 1) * MT, wc = (wave >> 1) * NT;
+    for (int st = 0; st < nstage; ++st) {
+      // this wave's copies of stage st: the 2 * 2 * kRowSteps after them may be in flight
+      asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+      static_assert(kRowSteps == 2 && kRowBuffers == 4, "copies in flight");
+      __syncthreads();  // everyone's; the buffer of stage st - 1 is no longer read
+      fill(st + kRowBuffers - 1);
+      const v4i* buf = (const v4i*)(s_mem + (st & (kRowBuffers - 1)) * kBufFrags * kFragBytes) + lane;
+      v4i av[kRowSteps][MT], bv[kRowSteps][NT];
+#pragma unroll
+      for (int k = 0; k < kRowSteps; ++k) {
+#pragma unroll
+        for (int j = 0; j < NT; ++j) bv[k][j] = buf[((kRowSteps + k) * kBlockTiles + wc + j) * kWave];
+#pragma unroll
+        for (int i = 0; i < MT; ++i) av[k][i] = buf[(k * kBlockTiles + wm + i) * kWave];
+      }
+#pragma unroll
+      for (int k = 0; k < kRowSteps; ++k)
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+          for (int j = 0; j < NT; ++j)
+            d[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(wide(av[k][i]), wide(bv[k][j]), d[i][j], 4, 4, 0, 0, 0, 0);
+      // the first step's operands, then the second's beside the first's products
+      __builtin_amdgcn_sched_group_barrier(0x100, MT + NT, 0);
+#pragma unroll
+      for (int q = 0; q < MT + NT; ++q) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      }
+      __builtin_amdgcn_sched_group_barrier(0x008, 2 * MT * NT - MT - NT, 0);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the copies past the end
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+      const int64_t c = c0 + wc + j;
+      if (c >= ctiles) continue;
+      const float want = need[c * kTile + (lane & 31)];
+#pragma unroll
+      for (int i = 0; i < MT; ++i) {
+        const uint32_t word = row_words_of(d[i][j], want);
+        const int64_t e = (m0 + wm + i) * kTile + lane;
+        if (lane < kTile && e < N) masks[e * row_words + c] = word;
+      }
+    }
+  }
+}
+
+// The same for few samples: a block per product tile, its four waves sharing the steps, the
+// operands read straight from global memory (the samples' from their encoded words) and the
+// partial sums put together in LDS.
+__global__ __launch_bounds__(256) void fire_few_kernel(const uint32_t* __restrict__ X, int64_t N, Geom g,
+                                                       const v4i* __restrict__ cfrag, const float* __restrict__ need,
+                                                       int steps, int64_t row_words, uint32_t* __restrict__ masks) {
+  __shared__ float s_d[3][16][kWave];
+  const int lane = lane_id(), wave = threadIdx.x / kWave;
+  const int64_t mtiles = (N + kTile - 1) / kTile, ctiles = (g.C + kTile - 1) / kTile;
+  const int64_t mt = blockIdx.x % mtiles, ct = blockIdx.x / mtiles;
+  if (ct >= ctiles) return;
+  const int64_t e = mt * kTile + (lane & 31) < N ? mt * kTile + (lane & 31) : N - 1;
+  const uint32_t* x = X + e * g.W;
+  const v4i* cf = cfrag + ct * steps * kWave + lane;
+  v16f d;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) d[r] = wave == 0 ? 1.0f : 0.0f;
+  const float want = need[ct * kTile + (lane & 31)];
+  constexpr int kAhead = 4;  // operands in flight
+  for (int s0 = wave; s0 < steps; s0 += 4 * kAhead) {
+    uint32_t xw[kAhead];
+    v4i bv[kAhead];
+#pragma unroll
+    for (int q = 0; q < kAhead; ++q) {
+      const int st = s0 + 4 * q < steps ? s0 + 4 * q : steps - 1;  // clamped: every load unconditional
+      const int64_t w = 2 * st + (lane >> 5);
+      xw[q] = x[w < g.W ? w : g.W - 1];  // past the words the clause operand is 0
+      bv[q] = cf[st * kWave];
+    }
+#pragma unroll
+    for (int q = 0; q < kAhead; ++q)
+      if (s0 + 4 * q < steps)
+        d = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(wide(fp4_of(xw[q], 0u)), wide(bv[q]), d, 4, 4, 0, 0, 0, 0);
+  }
+  if (wave > 0)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) s_d[wave - 1][r][lane] = d[r];
+  __syncthreads();
+  if (wave > 0) return;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) d[r] += s_d[0][r][lane] + s_d[1][r][lane] + s_d[2][r][lane];
+  const uint32_t word = row_words_of(d, want);
+  if (lane < kTile && mt * kTile + lane < N) masks[(mt * kTile + lane) * row_words + ct] = word;
 }
 
 // Class sums of 32 samples from their firing bits: the product of the bits (0 / 1) and the
@@ -313,8 +533,9 @@ constexpr int kVoteWaves = 8;
 __global__ __launch_bounds__(64 * kVoteWaves) void votes_kernel(const uint32_t* __restrict__ masks, int64_t row_words,
                                                                 int64_t N, const v4i* __restrict__ frag, Geom g, int D,
                                                                 int groups, const float* __restrict__ bias,
-                                                                float* __restrict__ out) {
+                                                                float* __restrict__ out, int* __restrict__ odd) {
   __shared__ int s_sum[kVoteWaves][kTile][kTile];  // [wave][sample][column]
+  if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *odd = 0;  // for the next samples
   const int lane = lane_id(), col = lane & 31, half = lane >> 5;
   const int wave = threadIdx.x / kWave;
   const int64_t e0 = (int64_t)blockIdx.x * kTile;
@@ -363,10 +584,7 @@ __global__ __launch_bounds__(256) void halves_kernel(const uint32_t* __restrict_
   bool bad = false;
   for (int64_t idx = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; idx < rows * hw;
        idx += (int64_t)gridDim.x * blockDim.x) {
-    const uint32_t* x = X + idx / hw * g.W;
-    const int64_t j = idx % hw;
-    const uint32_t valid = g.Lh - 32 * j >= 32 ? 0xFFFFFFFFu : (1u << (g.Lh - 32 * j)) - 1u;
-    bad = bad || (bits_at(x, g.W, 0, g.Lh, j) ^ bits_at(x, g.W, g.Lh, g.Lh, j)) != valid;
+    bad = bad || !complements(X + idx / hw * g.W, g, idx % hw);
   }
   if (bad) *ok = 0;
 }
@@ -424,21 +642,46 @@ hipError_t fire_steps(const uint32_t* X, int64_t N, const Geom& g, const v4i* fr
   return launch_fire<KS, HI, W, true>(X, N, g, frag, need, cus, row_words, masks, s);
 }
 
+// Bytes of the firing words of N samples, before the samples' operands.
+size_t rows_room(const MatrixPlan& p, int64_t N) { return ((size_t)N * p.row_words * 4 + 255) & ~(size_t)255; }
+
 }  // namespace
+
+size_t matrix_rows_bytes(const MatrixPlan& p, int64_t N) {
+  return rows_room(p, N) + (size_t)((N + kTile - 1) / kTile * kTile) * p.sample_bytes;
+}
 
 hipError_t launch_halves_check(const uint32_t* X, int64_t N, const Geom& g, int* ok, hipStream_t s) {
   halves_kernel<<<blocks_for(N * g.P * ((g.Lh + 31) / 32), 256), 256, 0, s>>>(X, N * g.P, g, ok);
   return hipGetLastError();
 }
 
-MatrixPlan matrix_plan(const Geom& g, bool halves, double w_bound) {
+bool long_rows(const Geom& g, int64_t N) {
+  return (N + kTile - 1) / kTile * clause_tiles(g) * ((g.L + kStep - 1) / kStep) > (4 << 20);
+}
+
+bool few_rows(const Geom& g, int64_t N) { return (N + kTile - 1) / kTile * clause_tiles(g) <= 2048; }
+
+MatrixPlan matrix_plan(const Geom& g, int halves, double w_bound, int64_t N) {
   MatrixPlan p{};
-  p.ternary = halves && g.append_negated;
-  const int64_t n = p.ternary ? g.Lh : g.L;
-  const int64_t steps = (n + kStep - 1) / kStep;
-  if (g.P < 2 || steps > kMaxSteps || clause_tiles(g) > (1 << 19)) return p;
-  p.steps = (int)steps;
   const int64_t tiles = clause_tiles(g);
+  if (tiles > (1 << 19)) return p;
+  p.ternary = halves == 1 && g.append_negated;
+  auto steps_of = [](int64_t n) { return (n + kStep - 1) / kStep; };
+  const int64_t steps = steps_of(p.ternary ? g.Lh : g.L);
+  if (g.P > 1) {
+    if (steps > kMaxSteps) return p;
+    p.steps = (int)steps;
+  } else {
+    // Up to 32 clauses of up to 512 literals, the register tiles of samples take less than the
+    // operands' passes (100000 samples, 10 clauses of 32 literals: 13 against 31 us; 32 clauses:
+    // 21 against 31, of 512: 40 against 37; 64 clauses: 32 and 59 against 33 and 39).
+    if (steps > (1 << 16) || (g.W <= 16 && g.C <= 32)) return p;
+    auto even = [](int64_t n) { return (int)((n + kRowSteps - 1) / kRowSteps * kRowSteps); };
+    p.steps = even(steps);
+    p.sample_bytes = (size_t)p.steps * kFragBytes / kTile;
+    if (halves < 0 && g.append_negated && !few_rows(g, N)) p.half_steps = even(steps_of(g.Lh));
+  }
   p.row_words = (tiles + 3) / 4 * 4;
   // digits that hold every weight of magnitude up to w_bound
   double top = 127.0;
@@ -446,8 +689,10 @@ MatrixPlan matrix_plan(const Geom& g, bool halves, double w_bound) {
   const int per = kTile / p.digits;
   p.groups = (int)((g.K + per - 1) / per);
   auto room = [](size_t n) { return (n + 255) & ~(size_t)255; };
-  p.need_at = room((size_t)(tiles * steps) * kFragBytes);
-  p.weights_at = p.need_at + room((size_t)tiles * kTile * 4);
+  p.half_at = room((size_t)tiles * p.steps * kFragBytes);
+  p.need_at = p.half_at + room((size_t)tiles * p.half_steps * kFragBytes);
+  p.flag_at = p.need_at + room((size_t)tiles * kTile * 4 * (p.half_steps ? 2 : 1));
+  p.weights_at = p.flag_at + 256;
   p.bytes = p.weights_at + (size_t)(p.row_words * p.groups) * kFragBytes;
   return p;
 }
@@ -456,22 +701,34 @@ hipError_t launch_matrix_pack(const uint32_t* planes, const float* w, const Geom
                               void* scratch, hipStream_t s) {
   unsigned char* base = (unsigned char*)scratch;
   const int64_t tiles = clause_tiles(g);
-  pack_clauses_kernel<<<blocks_for(tiles * p.steps * kWave, 256), 256, 0, s>>>(planes, g, p.steps, p.ternary,
-                                                                              (v4i*)base);
-  clause_need_kernel<<<blocks_for(tiles * kTile * kWave, 256), 256, 0, s>>>(planes, g, p.ternary,
-                                                                           (float*)(base + p.need_at));
-  pack_weights_kernel<<<blocks_for(p.row_words * p.groups * kWave, 256), 256, 0, s>>>(
-      w, g, p.row_words, p.digits, p.groups, (v4i*)(base + p.weights_at));
+  const int need_blocks = blocks_for(tiles * kTile * kWave, 256);
+  const int weight_blocks = blocks_for(p.row_words * p.groups * kWave, 256);
+  pack_model_kernel<<<need_blocks + weight_blocks + blocks_for(tiles * (p.steps + p.half_steps) * kWave, 256), 256, 0,
+                      s>>>(planes, w, g, p, base, need_blocks, weight_blocks);
   return hipGetLastError();
 }
 
-hipError_t launch_matrix_score(const uint32_t* X, int64_t N, const Geom& g, const MatrixPlan& p, const void* scratch,
+hipError_t launch_matrix_score(const uint32_t* X, int64_t N, const Geom& g, const MatrixPlan& p, void* scratch,
                                int cus, const float* bias, uint32_t* masks, float* out, hipStream_t s) {
-  const unsigned char* base = (const unsigned char*)scratch;
+  if (N == 0) return hipSuccess;
+  unsigned char* base = (unsigned char*)scratch;
+  int* flag = (int*)(base + p.flag_at);
   const v4i* frag = (const v4i*)base;
   const float* need = (const float*)(base + p.need_at);
   hipError_t e = hipSuccess;
-  switch (p.steps) {
+  const int64_t mtiles = (N + kTile - 1) / kTile, ctiles = clause_tiles(g);
+  if (g.P == 1 && few_rows(g, N)) {
+    fire_few_kernel<<<(unsigned)(mtiles * ctiles), 256, 0, s>>>(X, N, g, frag, need, p.steps, p.row_words, masks);
+    e = hipGetLastError();
+  } else if (g.P == 1) {
+    v4i* sfrag = (v4i*)((unsigned char*)masks + rows_room(p, N));
+    pack_samples_kernel<<<blocks_for(mtiles * p.steps * kWave, 256), 256, 0, s>>>(X, N, g, p.steps, p.half_steps, flag, sfrag);
+    const int64_t blocks = ((mtiles + kBlockTiles - 1) / kBlockTiles) * ((ctiles + kBlockTiles - 1) / kBlockTiles);
+    const size_t lds = (size_t)kRowBuffers * 2 * kBlockTiles * kRowSteps * kFragBytes;
+    fire_rows_kernel<<<(unsigned)std::min<int64_t>((blocks + 7) / 8 * 8, 1 << 22), 512, lds, s>>>(
+        sfrag, N, g.C, base, p, masks);
+    e = hipGetLastError();
+  } else switch (p.steps) {
 #define YTM_FIRE(KS, HI, LO)                                                             \
   case KS:                                                                               \
     e = fire_steps<KS, HI, LO>(X, N, g, frag, need, cus, p.row_words, masks, s);         \
@@ -491,7 +748,7 @@ hipError_t launch_matrix_score(const uint32_t* X, int64_t N, const Geom& g, cons
   }
   if (e != hipSuccess) return e;
   votes_kernel<<<dim3((unsigned)((N + kTile - 1) / kTile), (unsigned)p.groups), 64 * kVoteWaves, 0, s>>>(
-      masks, p.row_words, N, (const v4i*)(base + p.weights_at), g, p.digits, p.groups, bias, out);
+      masks, p.row_words, N, (const v4i*)(base + p.weights_at), g, p.digits, p.groups, bias, out, flag);
   return hipGetLastError();
 }
 

@@ -1,11 +1,11 @@
 // ytm_memory.hip -- device memory kept between calls and large copies to host arrays.
 //
 // Calls that take host arrays (encode, fit, predict, transform) need device buffers of their
-// inputs and outputs for the length of the call.  The runtime hands out blocks of up to about
-// 2 MB from its own pool in under a microsecond, but a larger hipMalloc and hipFree take 40 to
-// 290 us each pair, which for a call of a few hundred microseconds is most of it; such blocks
-// are kept here when a call is done with them, up to kKeep bytes a device, and given back by
-// memory_trim (ytm_shutdown) or when an allocation fails.
+// inputs and outputs for the length of the call.  A hipMalloc and hipFree above 2 MB take 40 to
+// 290 us a pair, which for a call of a few hundred microseconds is most of it, and so does a
+// small one that finds the runtime's own chunk of small blocks gone; blocks are therefore kept
+// here when a call is done with them, up to kKeep bytes a device, and given back by memory_trim
+// (ytm_shutdown) or when an allocation fails.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -24,8 +24,8 @@ namespace ytm {
 
 namespace {
 
-constexpr size_t kSmall = (size_t)1 << 20;  // below: the runtime's own pool
-constexpr size_t kUnit = (size_t)2 << 20;   // kept blocks are whole units
+constexpr size_t kSmall = (size_t)1 << 20;  // below: powers of two
+constexpr size_t kUnit = (size_t)2 << 20;   // from there on: whole units
 constexpr size_t kKeep = (size_t)1 << 30;   // idle bytes kept per device
 
 struct Block {
@@ -59,8 +59,11 @@ void trim_locked(int device) {
 
 hipError_t pool_alloc(void** p, size_t bytes) {
   *p = nullptr;
-  if (bytes < kSmall) return hipMalloc(p, bytes > 0 ? bytes : 4);
-  const size_t want = (bytes + kUnit - 1) / kUnit * kUnit;
+  size_t want = 256;
+  if (bytes < kSmall)
+    while (want < bytes) want *= 2;
+  else
+    want = (bytes + kUnit - 1) / kUnit * kUnit;
   int device = 0;
   hipError_t e = hipGetDevice(&device);
   if (e != hipSuccess) return e;
@@ -161,7 +164,8 @@ hipError_t ready_staging(int device) {
 hipError_t copy_to_host(void* dst, const void* src, size_t bytes, hipStream_t s) {
   std::unique_lock<std::mutex> lock(g_staging_mu, std::defer_lock);
   int device = 0;
-  const int threads = (int)std::min<unsigned>(kThreads, std::max(1u, std::thread::hardware_concurrency() / 2));
+  static const int threads =  // asked once: the answer takes longer than a small copy
+      (int)std::min<unsigned>(kThreads, std::max(1u, std::thread::hardware_concurrency() / 2));
   // another thread's copy has the buffers, there are few CPUs, or they cannot be had: the
   // runtime's own copy
   if (bytes < kStaged || threads < 2 || hipGetDevice(&device) != hipSuccess || !lock.try_lock() ||
