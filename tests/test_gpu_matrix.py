@@ -167,3 +167,49 @@ def test_literal_lists_of_wide_patches(monkeypatch):
     for least in ("1", "1000000"):
         monkeypatch.setenv("YTM_SCORE_WHOLE_MIN", least)
         check(tm, ref, enc)
+
+
+@pytest.mark.parametrize("dim,clauses,wgs,opts", [
+    ((33, 3, 1), 33, "2", {}),                            # 31 patches, 1 step, 16 or 17 clauses a workgroup
+    ((34, 3, 4), 64, "2", {}),                            # 32 patches, 2 steps, 32 clauses
+    ((35, 3, 11), 66, "2", dict(append_negated=False)),   # 33 patches, binary literals, 33 clauses
+    ((34, 34, 20), 97, "1", {}),                          # 1024 patches, 4 steps, one workgroup of 97
+    ((47, 47, 1), 130, "1", {}),                          # 2025 patches: 64 words of them
+    ((5, 4, 53), 96, "1", {}),                            # 6 patches, 8 steps
+])
+@pytest.mark.parametrize("env", [{}, {"YTM_TRAIN_THREADS": "256"}, {"YTM_JIT": "0"}])
+def test_training_on_several_patches(monkeypatch, dim, clauses, wgs, opts, env):
+    """The training kernel of clause state in global memory with its evaluation as a product:
+    edges of the tiles of patches and clauses, of the literal steps and of the workgroup's waves,
+    dropped clauses, and samples whose negated literals are not complements (the list walks),
+    against the oracle, bit for bit."""
+    monkeypatch.setenv("YTM_TRAIN_GLOBAL", "1")
+    monkeypatch.setenv("YTM_TRAIN_WGS", wgs)
+    for k, v in env.items():
+        monkeypatch.setenv(k, v)
+    print(f"[training] {dim} {clauses} {wgs} {opts} {env}", flush=True)
+    rng = np.random.default_rng(dim[2])
+    kw = dict(patch_dim=(3, 3), **opts)
+    tm, ref = pair(clauses, dim, 3, rng, **kw)
+    n = 6
+    X = (rng.random((n, int(np.prod(dim)))) < 0.4).astype(np.uint32)
+    y = rng.integers(0, 3, n)
+    enc = tm.encode(X)
+    odd = enc.copy()
+    odd[:, 0, 0] ^= np.uint32(4)
+    encY = ref.encode_y_multiclass(y)
+    drops = np.random.default_rng(7)  # the model's numpy generator
+    for data, p, inject in ((enc, 0.0, False), (enc, 0.3, False), (odd, 0.0, False), (enc, 0.0, True)):
+        kw, kr = {}, {}
+        if inject:
+            kw["random_stream"] = kr["inject"] = rng.random(tm.random_stream_size(n)).astype(np.float32)
+        if p:
+            kw["clause_drop_p"] = p
+            kr["drop"] = (drops.random(ref.C) <= p).astype(np.uint32)
+        tm.fit(data, y, is_X_encoded=True, **kw)
+        upd = ref.fit_encoded(data, encY, **kr)
+        st = tm.stats()
+        assert st["train_kind"] == 2 and st["last_fit_updates"] == upd
+        np.testing.assert_array_equal(tm.get_ta_state().reshape(ref.ta.shape), ref.ta)
+        np.testing.assert_array_equal(tm.get_weights().reshape(ref.w.shape), ref.w)
+        np.testing.assert_array_equal(tm.get_patch_weights().reshape(ref.pw.shape), ref.pw)

@@ -124,6 +124,49 @@ __device__ __forceinline__ void planes_dec(uint32_t* pl, int np, uint32_t m) {
   }
 }
 
+// ---------------------------------------------------------------- matrix-core operands
+// A clause's test of a patch as a sum (see ytm_matrix.hip): operands of
+// v_mfma_f32_32x32x64_f8f6f4 in FP4 (E2M1), a lane holding 32 literals of a row (patch or
+// sample) or a column (clause).  Nibble n of register q takes literal 4 n + q of the lane's
+// literal word, on both sides alike, which makes an operand from a word in a shift and an AND a
+// register: 0.5 (0x1) for a literal that is 1, and 2 or -2 (0x4, 0xC) for one that is included
+// or whose negation is, so that every product is 1, -1 or 0.
+typedef int v4i __attribute__((ext_vector_type(4)));
+typedef int v8i __attribute__((ext_vector_type(8)));
+typedef float v16f __attribute__((ext_vector_type(16)));
+
+__device__ __forceinline__ v4i fp4_row(uint32_t x) {
+  v4i r;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) r[q] = (int)((x >> q) & 0x11111111u);
+  return r;
+}
+
+__device__ __forceinline__ v4i fp4_column(uint32_t on, uint32_t neg) {
+  v4i r;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) r[q] = (int)(((on >> q) & 0x11111111u) << 2 | ((neg >> q) & 0x11111111u) << 3);
+  return r;
+}
+
+// d + the product of a row and a column operand.
+__device__ __forceinline__ v16f fp4_product(v4i a, v4i b, v16f d) {
+  return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(__builtin_shufflevector(a, a, 0, 1, 2, 3, -1, -1, -1, -1),
+                                                         __builtin_shufflevector(b, b, 0, 1, 2, 3, -1, -1, -1, -1), d,
+                                                         4, 4, 0, 0, 0, 0);
+}
+
+// Word j of the bits [from, from + n) of row m (W words), bit b = bit from + 32 j + b.
+__device__ __forceinline__ uint32_t bits_at(const uint32_t* m, int64_t W, int64_t from, int64_t n, int64_t j) {
+  const int64_t left = n - 32 * j;
+  if (left <= 0) return 0u;
+  const int64_t at = from + 32 * j, w = at >> 5;
+  const int sh = (int)(at & 31);
+  const uint32_t lo = m[w], hi = sh && w + 1 < W ? m[w + 1] : 0u;
+  const uint32_t v = sh ? (lo >> sh) | (hi << (32 - sh)) : lo;
+  return left >= 32 ? v : v & ((1u << left) - 1u);
+}
+
 // ---------------------------------------------------------------- wave64 helpers
 // Inclusive scans over the 64 lanes with DPP (data-parallel primitives: VALU operands read
 // from another lane), which avoid the LDS crossbar that lane shuffles go through: shifts by

@@ -1289,6 +1289,15 @@ int train_rng_slots(int cpw, const Geom& g) {
   return (int)std::max<size_t>(1, std::min<size_t>((size_t)cpw * g.K, budget / per_slot));
 }
 
+// With g.mma (train_global_body): include counts [cpw, rounded to even], clause operands
+// [ceil(cpw/32)][steps][64] of 16 bytes (aligned), sample rows [2][PW][steps][64], thresholds
+// [cpw], firing words [cpw][PW], firing clauses [2][cpw], changed clauses [cpw], include masks [cpw][W].
+static size_t mm_lds_bytes(const Geom& g, int cpw) {
+  const size_t C = (size_t)cpw, ct = (C + 31) / 32, PW = (size_t)((g.P + 31) / 32);
+  return (C + 1) / 2 * 8 + 16 + ct * (size_t)mm_steps(g) * 1024 + 2 * PW * (size_t)mm_steps(g) * 256 +
+         4 * (C + C * PW + 2 * C + C + C * (size_t)g.W);
+}
+
 size_t train_lds_bytes(TrainKind kind, int cpw, int rng_slots, const Geom& g) {
   // literal lists (several patches): include counts [cpw, rounded to even] and lists [cpw][cap] u16
   const size_t cap = g.P > 1 ? (size_t)g.list_cap : 0;
@@ -1299,6 +1308,7 @@ size_t train_lds_bytes(TrainKind kind, int cpw, int rng_slots, const Geom& g) {
                                      // patches the reservoir thresholds [P+1] and rank bits [2][cpw]
     return (size_t)3 * cpw * 8 + (size_t)6 * cpw * sizeof(int) + lists +
            (literal_major_lds(g) ? (size_t)(g.L * ((g.P + 31) / 32)) * 4 : 0) +
+           (g.mma ? mm_lds_bytes(g, cpw) : 0) +
            (g.mask_lds ? (size_t)(cpw + 2) * g.W * 4 : 0) + (size_t)cpw * g.K * 4 + (size_t)cpw * 4 +
            (g.P > 1 ? (size_t)(g.P + 1) * 4 + (size_t)2 * cpw * 4 : 0);
   // Resident kernel (layout of train_resident_body): task masks [cpw][3] u64; planes

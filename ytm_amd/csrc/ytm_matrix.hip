@@ -27,10 +27,7 @@ namespace ytm {
 
 namespace {
 
-typedef int v4i __attribute__((ext_vector_type(4)));
-typedef int v8i __attribute__((ext_vector_type(8)));
 typedef int v16i __attribute__((ext_vector_type(16)));
-typedef float v16f __attribute__((ext_vector_type(16)));
 
 constexpr int kTile = 32;        // rows (patches) and columns (clauses) of one product tile
 constexpr int kStep = 64;        // literals of one product instruction
@@ -38,35 +35,6 @@ constexpr int kFragBytes = 1024; // one operand of one instruction: 64 lanes x 3
 constexpr int kMaxSteps = 9;     // literal steps whose patch operands fit registers
 // What no product reaches: the threshold of an empty clause, which does not vote.
 constexpr float kNever = 1.0e9f;
-
-// Bits of v (8 of them) as the low bits of 8 nibbles.
-__device__ __forceinline__ uint32_t nibbles(uint32_t v) {
-  v = (v | (v << 12)) & 0x000F000Fu;
-  v = (v | (v << 6)) & 0x03030303u;
-  return (v | (v << 3)) & 0x11111111u;
-}
-
-// 32 FP4 values, 1.0 (0x2) where the bit of `on` is set, negative (0x8) where `neg` is set too.
-__device__ __forceinline__ v4i fp4_of(uint32_t on, uint32_t neg) {
-  v4i r;
-#pragma unroll
-  for (int q = 0; q < 4; ++q)
-    r[q] = (int)((nibbles((on >> (8 * q)) & 0xFFu) << 1) | (nibbles((neg >> (8 * q)) & 0xFFu) << 3));
-  return r;
-}
-
-__device__ __forceinline__ v8i wide(v4i x) { return __builtin_shufflevector(x, x, 0, 1, 2, 3, -1, -1, -1, -1); }
-
-// Word j of the bits [from, from + n) of row m (W words), bit b = bit from + 32 j + b.
-__device__ __forceinline__ uint32_t bits_at(const uint32_t* m, int64_t W, int64_t from, int64_t n, int64_t j) {
-  const int64_t left = n - 32 * j;
-  if (left <= 0) return 0u;
-  const int64_t at = from + 32 * j, w = at >> 5;
-  const int sh = (int)(at & 31);
-  const uint32_t lo = m[w], hi = sh && w + 1 < W ? m[w + 1] : 0u;
-  const uint32_t v = sh ? (lo >> sh) | (hi << (32 - sh)) : lo;
-  return left >= 32 ? v : v & ((1u << left) - 1u);
-}
 
 // Whether word j of the encoded row x's positive literals is the complement of the negated ones.
 __device__ __forceinline__ bool complements(const uint32_t* x, const Geom& g, int64_t j) {
@@ -163,7 +131,7 @@ __global__ __launch_bounds__(256) void pack_model_kernel(const uint32_t* __restr
       pos = bits_at(m, g.W, 0, ternary ? g.Lh : g.L, j);
       if (ternary) neg = bits_at(m, g.W, g.Lh, g.Lh, j);
     }
-    const v4i v = fp4_of(pos ^ neg, neg & ~pos);
+    const v4i v = fp4_column(pos ^ neg, neg & ~pos);
     if (st < p.steps)
       frag[(tile * p.steps + s) * kWave + l] = v;
     else
@@ -255,7 +223,7 @@ __global__ __launch_bounds__(64 * WAVES) void fire_patches_kernel(const uint32_t
 #pragma unroll
         for (int k = 0; k < KS; ++k) {
           const int w = 2 * k + half;
-          a[t][k] = fp4_of(x[w < g.W ? w : g.W - 1], 0u);  // past the literals the clause operand is 0
+          a[t][k] = fp4_row(x[w < g.W ? w : g.W - 1]);  // past the literals the clause operand is 0
         }
       }
       for (int at = 0, b = 0; at < nct; at += CT, b ^= 1) {
@@ -301,7 +269,7 @@ __global__ __launch_bounds__(64 * WAVES) void fire_patches_kernel(const uint32_t
               v16f x = ones;
 #pragma unroll
               for (int k = 0; k < KS; ++k)
-                x = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(wide(a[t][k]), wide(bv[k]), x, 4, 4, 0, 0, 0, 0);
+                x = fp4_product(a[t][k], bv[k], x);
               d[cur] = x;
               if (t > 0) {
                 look(d[cur ^ 1], t - 1, j, want);
@@ -347,7 +315,7 @@ __global__ __launch_bounds__(256) void pack_samples_kernel(const uint32_t* __res
     const int l = (int)(idx % kWave);
     const int64_t w = idx / kWave % steps * 2 + (l >> 5), e = idx / kWave / steps * kTile + (l & 31);
     const uint32_t* x = X + (e < N ? e : N - 1) * g.W;
-    frag[idx] = fp4_of(w < g.W ? x[w] : 0u, 0u);
+    frag[idx] = fp4_row(w < g.W ? x[w] : 0u);
     if (w < hw) bad = bad || !complements(x, g, w);
   }
   if (bad) *odd = 1;
@@ -452,7 +420,7 @@ __global__ __launch_bounds__(512) void fire_rows_kernel(const v4i* __restrict__ 
         for (int i = 0; i < MT; ++i)
 #pragma unroll
           for (int j = 0; j < NT; ++j)
-            d[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(wide(av[k][i]), wide(bv[k][j]), d[i][j], 4, 4, 0, 0, 0, 0);
+            d[i][j] = fp4_product(av[k][i], bv[k][j], d[i][j]);
       // the first step's operands, then the second's beside the first's products
       __builtin_amdgcn_sched_group_barrier(0x100, MT + NT, 0);
 #pragma unroll
@@ -510,7 +478,7 @@ __global__ __launch_bounds__(256) void fire_few_kernel(const uint32_t* __restric
 #pragma unroll
     for (int q = 0; q < kAhead; ++q)
       if (s0 + 4 * q < steps)
-        d = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(wide(fp4_of(xw[q], 0u)), wide(bv[q]), d, 4, 4, 0, 0, 0, 0);
+        d = fp4_product(fp4_row(xw[q]), bv[q], d);
   }
   if (wave > 0)
 #pragma unroll

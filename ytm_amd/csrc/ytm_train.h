@@ -1345,6 +1345,239 @@ __device__ __forceinline__ void global_phase_a(const TrainArgs& a, const Geom& g
   }
 }
 
+// ---------------------------------------------------------------- matrix cores
+// Phase A of a model with several patches as a product (g.mma): the workgroup's clauses are
+// columns (operands s_bf[tile of 32 clauses][step][lane], thresholds s_need), the sample's
+// patches rows.  The list walks it replaces read a literal's bitset per included literal and
+// clause, behind a copy of the literal-major sample into LDS that every wave waited for; the
+// product reads each patch's words straight from the encoded sample, one iteration ahead.
+// 32x32x24 in 3x3 patches, 20000 clauses (78 a workgroup, 29 patch tiles, 5 steps), sixth epoch:
+// 12.7 us per sample with the lists, 10.3 with the product.  Its matrix instructions alone are
+// 1.6 us of a sample; tiles, thresholds and selections take 5 to 6, beside the exchange.
+
+// The operands (the literals' words half by half: lanes 0..31 hold words 0 .. steps - 1, the others
+// the next ones, so that a row is read as consecutive words), the threshold (the included
+// positive literals) and the include count of own clause idx from its include mask m (LDS), by
+// one wave.
+__device__ __forceinline__ void mm_store_clause(const Geom& g, const uint32_t* m, int idx, v4i* s_bf, float* s_need,
+                                                int* s_nlit) {
+  const int lane = lane_id();
+  const int KS = (int)mm_steps(g);
+  uint32_t pos = 0u, neg = 0u;
+  if (lane < 2 * KS) {
+    pos = bits_at(m, g.W, 0, g.append_negated ? g.Lh : g.L, lane);
+    if (g.append_negated) neg = bits_at(m, g.W, g.Lh, g.Lh, lane);
+    const int half = lane >= KS, k = lane - half * KS;
+    s_bf[((idx >> 5) * KS + k) * kWave + half * 32 + (idx & 31)] = fp4_column(pos ^ neg, neg & ~pos);
+  }
+  const int n = wave_sum_i32(__popc(pos) + __popc(neg)), np = wave_sum_i32(__popc(pos));
+  if (lane == 0) {
+    s_need[idx] = (float)np;
+    s_nlit[idx] = n;
+  }
+}
+
+// Copies the rows of sample xe ([P][W]) into LDS as the lanes use them, s_xw[patch tile][step][lane]:
+// lane l's word of step k is word steps * (l / 32) + k of patch 32 tile + l % 32 (rows past the last
+// patch repeat it; past the literals the clause operand is 0).  Copied there directly from
+// global memory, by waves first, first + count, ... of count; each waits for its own copies
+// (vmcnt) before the barrier that makes them everyone's.
+__device__ __forceinline__ void mm_stage(const Geom& g, const uint32_t* xe, uint32_t* s_xw, int first, int count) {
+  const int lane = lane_id(), KS = (int)mm_steps(g), PW = (int)((g.P + 31) / 32);
+  const int from = lane < 32 ? 0 : KS;
+  for (int it = first; it < PW * KS; it += count) {
+    const int tile = it / KS, w = from + it - tile * KS, p = tile * 32 + (lane & 31);
+    const uint32_t* src = xe + (int64_t)(p < (int)g.P ? p : (int)g.P - 1) * g.W + (w < (int)g.W ? w : (int)g.W - 1);
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                     (__attribute__((address_space(3))) void*)(s_xw + it * kWave), 4, 0, 0);
+  }
+}
+
+// Bits of the 32 rows of a tile whose sum reaches `want`, which no sum exceeds: the same word in
+// lane c and lane c + 32, column c.  A sum's distance is negative where it falls short, so its
+// sign is shifted in, two operations a row and no branch.
+__device__ __forceinline__ uint32_t mm_word(const v16f& d, float want) {
+  uint32_t w = 0u;
+#pragma unroll
+  for (int r = 15; r >= 0; --r) {
+    w = __builtin_amdgcn_alignbit(w, (uint32_t)__float_as_int(d[r] - want), 31);  // (w << 1) | sign
+    if ((r & 3) == 0 && r > 0) w <<= 4;  // rows 8 (r / 4) + r % 4, and 4 more in the upper lanes
+  }
+  w = (~w & 0x0F0F0F0Fu) << (4 * (lane_id() >> 5));
+  const auto sw = __builtin_amdgcn_permlane32_swap(w, w, false, false);
+  return sw[0] | sw[1];
+}
+
+// The words of patch tile `tile` of the sample in s_xw, of clauses cols[0 .. ncol) (null: the first
+// ncol own ones) into s_bm[clause][PW], and a 1 into s_any[clause] for those that fire in it.
+// By one wave, NQ clause tiles at once beside each other: a row operand is made once for them,
+// and the next step's operands are read beside a step's products.  No LDS atomics: the
+// compiler lets one wait for the copies of the next sample (mm_stage).  The operands a step
+// ahead, without a branch per clause tile, against one read, wait and product after another:
+// 3 against 8.3 us per sample and wave.
+template <int NQ>
+__device__ __forceinline__ void mm_tile(const Geom& g, const uint32_t* s_xw, int tile, int ncol, const int* cols,
+                                        const v4i* s_bf, const float* s_need, uint32_t* s_bm, int* s_any) {
+  const int lane = lane_id(), row = lane & 31;
+  const int KS = (int)mm_steps(g), PW = (int)((g.P + 31) / 32);
+  const uint32_t last = (g.P & 31) ? (1u << (g.P & 31)) - 1u : 0xFFFFFFFFu;  // patches of the last tile
+  const uint32_t valid = tile == PW - 1 ? last : 0xFFFFFFFFu;
+  const uint32_t* xl = s_xw + tile * KS * kWave + lane;
+  uint32_t x[kMmSteps];
+#pragma unroll
+  for (int k = 0; k < kMmSteps; ++k) x[k] = k < KS ? xl[k * kWave] : 0u;
+  for (int c0 = 0; c0 < ncol; c0 += 32 * NQ) {
+    int idx[NQ];
+    const v4i* b[NQ];
+    float want[NQ];
+    v16f d[NQ];
+    v4i bv[2][NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+      const int col = c0 + 32 * q + row < ncol ? c0 + 32 * q + row : ncol - 1;  // columns past the last repeat it
+      idx[q] = cols ? cols[col] : col;
+      b[q] = s_bf + (idx[q] >> 5) * KS * kWave + (lane & 32) + (idx[q] & 31);
+      // started at 1, 2 and 4: one shared start would be held in registers, each of these is part
+      // of its instruction
+#pragma unroll
+      for (int r = 0; r < 16; ++r) d[q][r] = (float)(1 << q);
+    }
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) bv[0][q] = b[q][0];
+#pragma unroll
+    for (int k = 0; k < kMmSteps; ++k)
+      if (k < KS) {
+        const v4i av = fp4_row(x[k]);
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) {
+          if (k + 1 < KS) bv[(k + 1) & 1][q] = b[q][(k + 1) * kWave];
+        }
+        if (k + 1 == KS) {
+#pragma unroll
+          for (int q = 0; q < NQ; ++q) want[q] = s_need[idx[q]] + (float)(1 << q);
+        }
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) d[q] = fp4_product(av, bv[k & 1][q], d[q]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+      const uint32_t w = mm_word(d[q], want[q]) & valid;
+      if (lane < 32 && c0 + 32 * q + row < ncol) {
+        s_bm[idx[q] * PW + tile] = w;
+        if (w) s_any[idx[q]] = 1;
+      }
+    }
+  }
+}
+
+// mm_tile with as many clause tiles at once as ncol fills.
+__device__ __forceinline__ void mm_tile_of(const Geom& g, const uint32_t* s_xw, int tile, int ncol, const int* cols,
+                                           const v4i* s_bf, const float* s_need, uint32_t* s_bm, int* s_any) {
+  if (ncol > 32)
+    mm_tile<3>(g, s_xw, tile, ncol, cols, s_bf, s_need, s_bm, s_any);
+  else
+    mm_tile<1>(g, s_xw, tile, ncol, cols, s_bf, s_need, s_bm, s_any);
+}
+
+// Sum and maximum of v over the 16 lanes of a row, in each of them.
+__device__ __forceinline__ int row_sum(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x128, 0xf, 0xf, false);  // row_ror:8, 4, 2, 1
+  v += __builtin_amdgcn_update_dpp(0, v, 0x124, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x122, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x121, 0xf, 0xf, false);
+  return v;
+}
+__device__ __forceinline__ int row_max(int v) {
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x128, 0xf, 0xf, false));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x124, 0xf, 0xf, false));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x122, 0xf, 0xf, false));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x121, 0xf, 0xf, false));
+  return v;
+}
+
+// The selected patches (select_from_bitmap) of up to four clauses at once on sample t, one per 16
+// lanes (a wave's firing clauses one after another: 2.7 us per sample, so 1.4): clause c of each
+// row from its firing words bm (null: no clause in this row), with its rank_bits pre (or -1).  -1 in the row's lanes when no patch is selected.
+template <bool INJECT>
+__device__ __forceinline__ int mm_select(const TrainArgs& a, const Geom& g, const float* inj, int64_t c, uint64_t t,
+                                         const uint32_t* bm, const float* inv_rank, int pre) {
+  const int q = lane_id() & 15, PW = (int)((g.P + 31) / 32), per = (PW + 15) / 16;  // <= 4 words per lane
+  uint32_t v[4];
+  int pc = 0;
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    v[u] = u < per && bm && q * per + u < PW ? bm[q * per + u] : 0u;
+    pc += __popc(v[u]);
+  }
+  int incl = pc;
+  incl += __builtin_amdgcn_update_dpp(0, incl, kDppRowShr1, 0xf, 0xf, false);
+  incl += __builtin_amdgcn_update_dpp(0, incl, kDppRowShr2, 0xf, 0xf, false);
+  incl += __builtin_amdgcn_update_dpp(0, incl, kDppRowShr4, 0xf, 0xf, false);
+  incl += __builtin_amdgcn_update_dpp(0, incl, kDppRowShr8, 0xf, 0xf, false);
+  const int R = row_sum(pc);
+  // the rank, as reservoir_rank finds it: from the top, 64 ranks of each clause at a time
+  int best = 0, g0 = R > 0 ? (R - 1) >> 2 : -1;
+  if (!INJECT && pre >= 0 && R <= 4) {
+    const unsigned hits = (unsigned)pre & ((1u << R) - 1u);
+    best = hits ? 32 - __builtin_clz(hits) : 0;
+    g0 = -1;
+  }
+  while (__any(g0 >= 0)) {
+    int lb = 0;
+    const int gl = g0 - q;
+    if (gl >= 0) {
+      if (INJECT) {
+        for (int j = 0; j < 4; ++j) {
+          const int r = 4 * gl + 1 + j;
+          if (r <= R && inj[c * g.P + (r - 1)] < inv_rank[r]) lb = r;
+        }
+      } else {
+        const U4 z = counted_site(a, t, (uint32_t)c, TAG_SEL, (uint32_t)gl);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int r = 4 * gl + 1 + j;
+          if (r <= R && uniform_from_word(word_of(z, j)) < inv_rank[r]) lb = r;
+        }
+      }
+    }
+    lb = row_max(lb);
+    if (g0 >= 0) {
+      best = lb;
+      g0 = lb > 0 ? -1 : g0 - 16;
+    }
+  }
+  int n = best - (incl - pc), pos = -1;  // the lane's n-th firing patch, if it has it
+  if (best > 0 && n >= 1 && n <= pc) {
+    uint32_t w = v[0];
+    int at = 0;
+#pragma unroll
+    for (int u = 1; u < 4; ++u) {
+      const int p = __popc(w);
+      if (n > p) {
+        n -= p;
+        w = v[u];
+        at = u;
+      }
+    }
+    for (int j = 1; j < n; ++j) w &= w - 1u;
+    pos = 32 * (q * per + at) + __builtin_ctz(w);
+  }
+  return row_max(pos + 1) - 1;
+}
+
+// The votes of the clauses of mm_select (c and its weights of each row) to the partial sums.
+__device__ __forceinline__ void mm_vote(const Geom& g, long long* s_part, bool fires, int64_t c, const float* wrow) {
+  const int q = lane_id() & 15;
+  if (!fires) return;
+  if (g.coalesced) {
+    for (int k = q; k < g.K; k += 16) atomicAdd((unsigned long long*)&s_part[k], (unsigned long long)(long long)wrow[k]);
+  } else if (q == 0) {
+    const int64_t k = c / g.per_bank;
+    atomicAdd((unsigned long long*)&s_part[k], (unsigned long long)(long long)wrow[k]);
+  }
+}
+
 // Clause state in global memory (L2/MALL resident across samples); any P.  A software
 // pipeline over samples, like the resident kernel's; per sample i:
 //   1. wave 0 adds the patch weights of sample i's selections (select_active,
@@ -1371,6 +1604,8 @@ __device__ __forceinline__ void train_global_body(const TrainArgs& a, const Geom
   __shared__ int s_abort;
   __shared__ int s_ntask;
   __shared__ int s_anyfb;  // some class of the current sample may update
+  __shared__ int s_nchg;   // mm: own clauses whose include mask the current sample changes
+  __shared__ int s_mm_done;  // mm: waves whose tiles of the sample's product are in s_bm, over all samples
   const int lane = lane_id();
   const int wave = threadIdx.x / kWave;
   const int nwv = (int)(blockDim.x / kWave);
@@ -1384,15 +1619,29 @@ __device__ __forceinline__ void train_global_body(const TrainArgs& a, const Geom
   int* s_task_idx = s_ninc + 2 * cpw;                          // [cpw]
   int* s_task_sb = s_task_idx + cpw;                           // [cpw] (zero: no precomputed draws)
   const int cap = VANILLA ? 0 : g.list_cap;                    // literal list capacity
-  int* s_nlit = s_task_sb + cpw;                               // [cpw] include counts (cap > 0)
-  uint16_t* s_lits = (uint16_t*)(s_nlit + (cap > 0 ? 2 * ((cpw + 1) / 2) : 0));  // [cpw][cap] literal lists
+  const bool mm = !VANILLA && g.mma != 0;                      // clauses on the matrix cores
+  int* s_nlit = s_task_sb + cpw;                               // [cpw] include counts (cap > 0 or mm)
+  uint16_t* s_lits = (uint16_t*)(s_nlit + (cap > 0 || mm ? 2 * ((cpw + 1) / 2) : 0));  // [cpw][cap] literal lists
   uint32_t* s_xt = (uint32_t*)(s_lits + (int64_t)cpw * cap);  // [L][PW] when literal_major_lds(g)
   const int64_t cw = (int64_t)g.np * g.W;
   const int64_t xt_words = literal_major(g) ? g.L * ((g.P + 31) / 32) : 0;
   // mask_lds (one patch): the own clauses' include masks [cpw][W], kept current by the
   // literal updates, and the words of samples i and i+1 [2][W]
-  uint32_t* s_mask = s_xt + (literal_major_lds(g) ? xt_words : 0);
-  uint32_t* s_xs = s_mask + (g.mask_lds ? (int64_t)cpw * g.W : 0);
+  // mm: the clause operands [ceil(cpw / 32)][steps][64] (16-byte aligned), the rows of samples
+  // i and i+1 [2][PW][steps][64], the clauses' thresholds [cpw], the firing words of the sample
+  // being evaluated [cpw][PW], the clauses that fire on samples i and i+1 [2][cpw], the own clauses whose include mask sample i changes
+  // [cpw], then the include masks
+  const int mm_ct = (cpw + 31) / 32, mm_pw = (int)((g.P + 31) / 32);
+  const int mm_at = 12 * cpw + 2 * ((cpw + 1) / 2);  // words before s_xt (without lists)
+  v4i* s_bf = (v4i*)(s_xt + ((4 - mm_at % 4) & 3));
+  const int mm_xw = mm_pw * (int)mm_steps(g) * kWave;  // words of a sample's rows
+  uint32_t* s_xw = (uint32_t*)(s_bf + (mm ? mm_ct * (int)mm_steps(g) * kWave : 0));
+  float* s_need = (float*)(s_xw + (mm ? 2 * mm_xw : 0));
+  uint32_t* s_bm = (uint32_t*)(s_need + (mm ? cpw : 0));
+  int* s_any = (int*)(s_bm + (mm ? cpw * mm_pw : 0));
+  int* s_chg_idx = s_any + (mm ? 2 * cpw : 0);
+  uint32_t* s_mask = mm ? (uint32_t*)(s_chg_idx + cpw) : s_xt + (literal_major_lds(g) ? xt_words : 0);
+  uint32_t* s_xs = s_mask + (g.mask_lds || mm ? (int64_t)cpw * g.W : 0);
   float* s_wg = (float*)(s_xs + (g.mask_lds ? 2 * g.W : 0));  // the own clauses' weights [cpw][K]
   int* s_drop = (int*)(s_wg + (int64_t)cpw * g.K);              // [cpw] dropped (1) or not
   // several patches: the reservoir thresholds 1.0f / r, r = 0..P (a.inv_rank)
@@ -1416,15 +1665,22 @@ __device__ __forceinline__ void train_global_body(const TrainArgs& a, const Geom
   if (threadIdx.x == 0) {
     s_abort = 0;
     s_next_a = 0;
+    s_nchg = 0;
+    s_mm_done = 0;
   }
   for (int64_t j = threadIdx.x; j < n_own * g.K; j += blockDim.x) s_wg[j] = a.weights[c_begin * g.K + j];
   for (int j = threadIdx.x; j < n_own; j += blockDim.x) s_drop[j] = a.drop[c_begin + j] == 1u;
   if (g.P > 1)
     for (int64_t j = threadIdx.x; j <= g.P; j += blockDim.x) s_invr[j] = a.inv_rank[j];
-  if (g.mask_lds)  // include masks of the own clauses (visible after the first barrier below)
+  if (g.mask_lds || mm)  // include masks of the own clauses (visible after the first barrier below)
     for (int idx = wave; idx < n_own; idx += nwv)
       for (int64_t w = lane; w < g.W; w += kWave)
         s_mask[(int64_t)idx * g.W + w] = a.planes[(c_begin + idx) * cw + (int64_t)(g.np - 1) * g.W + w];
+  if (mm) {  // the operands, each clause by the wave that has just written its mask
+    for (int j = threadIdx.x; j < 2 * cpw; j += blockDim.x) s_any[j] = 0;
+    for (int idx = wave; idx < n_own; idx += nwv)
+      mm_store_clause(g, s_mask + (int64_t)idx * g.W, idx, s_bf, s_need, s_nlit);
+  }
   if (cap > 0)  // literal lists of the own clauses (visible after the first barrier below)
     for (int idx = wave; idx < n_own; idx += nwv) {
       const int n = build_literal_list<false>(g, a.planes + (c_begin + idx) * cw + (int64_t)(g.np - 1) * g.W,
@@ -1479,9 +1735,66 @@ __device__ __forceinline__ void train_global_body(const TrainArgs& a, const Geom
   auto xe_of = [&](int j) -> const uint32_t* {
     return g.mask_lds ? s_xs + (int64_t)(j & 1) * g.W : a.X + (int64_t)j * g.P * g.W;
   };
+  // mm: wave 0 waits for the totals, the others evaluate, the last one once it has copied the
+  // sample after
+  const int mm_nw = nwv - 1, mm_t0 = wave - 1;
+  // Phase A of sample j: the product's tiles, claimed one by one (a SIMD that holds wave 0 has one
+  // wave less for them; in turn: 11.1 us per sample, claimed 10.3), then, once all are in, the selections of the
+  // clauses that fire, in turn over the waves.
+  auto mm_phase_a = [&](int j, int* sel_n, long long* part) {
+    if (wave == 0) return;
+    if (wave == nwv - 1 && j + 1 < a.N)  // into the buffer of the sample before
+      mm_stage(g, a.X + (int64_t)(j + 1) * g.P * g.W, s_xw + ((j + 1) & 1) * mm_xw, 0, 1);
+    const uint64_t tj = a.step0 + (uint64_t)j;
+    const float* injj = INJECT ? a.inject + (int64_t)j * a.inject_block : nullptr;
+    const uint32_t* x = s_xw + (j & 1) * mm_xw;
+    int* any = s_any + (j & 1) * cpw;
+    for (;;) {
+      int t0 = 0;
+      if (lane == 0) t0 = atomicAdd(&s_next_a, 1);
+      t0 = lane_value(t0, 0);
+      if (t0 >= mm_pw) break;
+      mm_tile_of(g, x, t0, n_own, nullptr, s_bf, s_need, s_bm, any);
+    }
+    // every evaluating wave comes here once a sample, so the count ends each wave's wait
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    if (lane == 0) __hip_atomic_fetch_add(&s_mm_done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    while (__hip_atomic_load(&s_mm_done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) < (j + 1) * mm_nw)
+      __builtin_amdgcn_s_sleep(0);
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    // The firing clauses in turn over the waves, each wave's four at a time.
+    const int row = lane >> 4;
+    int turn = 0, c0 = 0, have = 0, idx = -1;
+    unsigned long long m = 0ull;
+    for (;;) {
+      while (have < 4) {
+        while (m == 0ull && c0 < n_own) {
+          const bool f = c0 + lane < n_own && any[c0 + lane < n_own ? c0 + lane : 0] != 0;
+          const unsigned long long fm = __ballot(f);
+          const int ord = turn + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(fm >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)fm, 0u));
+          m = __ballot(f && ord % mm_nw == mm_t0);
+          turn += __popcll(fm);
+          c0 += kWave;
+        }
+        if (m == 0ull) break;
+        if (row == have) idx = c0 - kWave + __ffsll((long long)m) - 1;
+        m &= m - 1ull;
+        ++have;
+      }
+      if (have == 0) break;
+      const int ix = row < have ? idx : 0;
+      const int sel = mm_select<INJECT>(a, g, injj, c_begin + ix, tj,
+                                        row < have && s_drop[ix] == 0 ? s_bm + ix * mm_pw : nullptr, s_invr,
+                                        use_rb ? s_rb[(j & 1) * cpw + ix] : -1);
+      if (sel >= 0 && (lane & 15) == 0) sel_n[ix] = sel;
+      mm_vote(g, part, sel >= 0, c_begin + ix, s_wg + (int64_t)ix * g.K);
+      have = 0;
+    }
+  };
   const int kn = g.coalesced ? (int)g.K : 1;
   const int cpp = kWave / kn;
   if (prefetched && a.N > 0) prefetch(0);
+  if (mm && a.N > 0) mm_stage(g, a.X, s_xw, wave, nwv);
   // i = -1 is the prologue: every wave stages sample 0 and takes part in its phase A
   for (int i = -1; i < a.N; ++i) {
     const uint64_t t = a.step0 + (uint64_t)i;
@@ -1499,7 +1812,16 @@ __device__ __forceinline__ void train_global_body(const TrainArgs& a, const Geom
         s_next_a = 0;
         s_next_d = 0;
         s_ntask = 0;
+        s_nchg = 0;
       }
+    }
+    if (mm && more) {  // no clause selected yet on sample i+1; the buffers were sample i-1's
+      for (int idx = threadIdx.x; idx < n_own; idx += blockDim.x) {
+        sel_n[idx] = -1;
+        ninc_n[idx] = s_nlit[idx];
+        s_any[bn * cpw + idx] = 0;
+      }
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's copies of sample i+1's rows
     }
     if (more) {
       if (prefetched) {
@@ -1515,10 +1837,6 @@ __device__ __forceinline__ void train_global_body(const TrainArgs& a, const Geom
     // ---- 2: the totals of sample i (wave 0, which publishes them first: the other waves
     // need not wait for that); speculative phase A of sample i+1 (the others)
     if (i >= 0 && wave == 0) {
-      for (int idx = lane; idx < n_own; idx += kWave) {
-        const int sl = sel_i[idx];
-        if (sl >= 0) atomicAdd(&a.patch_w[(c_begin + idx) * g.P + sl], 1);
-      }
       exchange_publish(a, g, i, s_part[b]);
       // the rank bits of sample i+2 while the sums are in flight (buffer i & 1: sample i's
       // phase A and re-evaluations are over)
@@ -1535,8 +1853,17 @@ __device__ __forceinline__ void train_global_body(const TrainArgs& a, const Geom
       if (lane == 0) s_anyfb = anyfb;
       YTM_PROF_MARK(1);
     }
+    // The patch weights of sample i, by the last wave: wave 0's would be in front of its class sums
+    // (a reply waits for the earlier atomics of its wave).
+    if (i >= 0 && wave == nwv - 1)
+      for (int idx = lane; idx < n_own; idx += kWave) {
+        const int sl = sel_i[idx];
+        if (sl >= 0) atomicAdd(&a.patch_w[(c_begin + idx) * g.P + sl], 1);
+      }
     // phase A of sample i+1: the other waves from the start, wave 0 once it has the totals
-    if (more)
+    if (mm) {
+      if (more) mm_phase_a(i + 1, sel_n, s_part[bn]);
+    } else if (more)
       global_phase_a<VANILLA, INJECT>(a, g, i + 1, c_begin, n_own, &s_next_a, s_lits, s_nlit, cap, xt_of(i + 1),
                                       xe_of(i + 1), s_mask, sel_n, ninc_n, s_wg, s_part[bn], s_invr, s_drop,
                                       use_rb ? s_rb + ((i + 1) & 1) * cpw : nullptr);
@@ -1629,8 +1956,26 @@ __device__ __forceinline__ void train_global_body(const TrainArgs& a, const Geom
         // narrow clauses: up to 64 / W queued updates per wave at once
         const int per = tasks_per_wave(g, ntask, nwv);
         for (int tk0 = wave * per; tk0 < ntask; tk0 += nwv * per)
-          apply_tasks<INJECT>(a, g, inj, c_begin, t, tk0, per, ntask, s_task_idx, s_task_m, s_task_sb, sel_i,
-                              a.planes + c_begin * cw, xe, nullptr, 0, g.mask_lds ? s_mask : nullptr);
+          if (mm) {
+            // the wave's clauses whose include mask changes get new operands and are evaluated
+            // again below; the others keep their evaluation of sample i+1 and only vote again
+            unsigned long long chg = 0ull;
+            apply_tasks<INJECT>(a, g, inj, c_begin, t, tk0, per, ntask, s_task_idx, s_task_m, s_task_sb, sel_i,
+                                a.planes + c_begin * cw, xe, nullptr, 0, s_mask, &chg);
+            const unsigned long long wmask = (1ull << g.W) - 1ull;
+            for (int tk = tk0; tk < tk0 + per && tk < ntask; ++tk) {
+              const int idx = s_task_idx[tk];
+              if ((chg >> ((tk - tk0) * g.W)) & wmask) {
+                mm_store_clause(g, s_mask + (int64_t)idx * g.W, idx, s_bf, s_need, s_nlit);
+                if (lane == 0) s_chg_idx[atomicAdd(&s_nchg, 1)] = idx;
+              } else if (more && sel_n[idx] >= 0) {
+                add_partial(a, g, s_part[bn], c_begin + idx, s_wg + (int64_t)idx * g.K);
+              }
+            }
+          } else {
+            apply_tasks<INJECT>(a, g, inj, c_begin, t, tk0, per, ntask, s_task_idx, s_task_m, s_task_sb, sel_i,
+                                a.planes + c_begin * cw, xe, nullptr, 0, g.mask_lds ? s_mask : nullptr);
+          }
       } else {
         // wide clauses: (update, 64-word chunk) items over all waves; the chunks of one
         // clause touch disjoint literals
@@ -1649,7 +1994,28 @@ __device__ __forceinline__ void train_global_body(const TrainArgs& a, const Geom
     YTM_PROF_MARK(4);
 
     // ---- 4: the updated clauses' literal lists, and their phase A of sample i+1 again
-    {
+    if (mm) {
+      const int nchg = s_nchg;
+      if (more && nchg > 0) {
+        for (int t0 = wave; t0 < mm_pw; t0 += nwv)
+          mm_tile_of(g, s_xw + ((i + 1) & 1) * mm_xw, t0, nchg, s_chg_idx, s_bf, s_need, s_bm, s_any + bn * cpw);
+        __syncthreads();  // every tile's words
+        const float* injn = INJECT ? a.inject + (int64_t)(i + 1) * a.inject_block : nullptr;
+        for (int q0 = wave; q0 < nchg; q0 += 4 * nwv) {  // four clauses at a time
+          const int q = q0 + nwv * (lane >> 4);
+          const bool has = q < nchg;
+          const int idx = s_chg_idx[has ? q : q0];
+          const int sel = mm_select<INJECT>(a, g, injn, c_begin + idx, t + 1,
+                                            has && s_drop[idx] == 0 ? s_bm + idx * mm_pw : nullptr, s_invr,
+                                            use_rb ? s_rb[((i + 1) & 1) * cpw + idx] : -1);
+          if (has && (lane & 15) == 0) {
+            sel_n[idx] = sel;
+            ninc_n[idx] = s_nlit[idx];
+          }
+          mm_vote(g, s_part[bn], sel >= 0, c_begin + idx, s_wg + (int64_t)idx * g.K);
+        }
+      }
+    } else {
       const int ntask = s_ntask;
       const uint64_t tn = t + 1;
       const float* injn = INJECT && more ? a.inject + (int64_t)(i + 1) * a.inject_block : nullptr;
@@ -1679,6 +2045,7 @@ __device__ __forceinline__ void train_global_body(const TrainArgs& a, const Geom
     __syncthreads();
     YTM_PROF_MARK(5);
   }
+  if (mm) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // an aborted run leaves copies in flight
   __syncthreads();
   for (int64_t j = threadIdx.x; j < n_own * g.K; j += blockDim.x) a.weights[c_begin * g.K + j] = s_wg[j];
   if (lane == 0 && my_updates) atomicAdd(&a.counters[0], my_updates);

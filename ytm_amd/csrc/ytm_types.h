@@ -56,6 +56,7 @@ constexpr int kMaxPlanesHost = 32;  // must equal kMaxPlanes of ytm_device.h
   X(int, groups)           /* training launch: class-sum groups, ceil(grid / group_size) */          \
   X(int, list_cap)         /* training launch: literal-list capacity per clause (0: none) */       \
   X(int, mask_lds)         /* training launch, global one-patch kernel: include masks and sample in LDS */ \
+  X(int, mma)              /* training launch, global several-patch kernel: clauses on the matrix cores */ \
   X(int, vote_table)       /* training launch, streaming kernel: class votes from nibble tables in LDS */
 
 struct Geom {
@@ -68,9 +69,17 @@ struct Geom {
 // sample (one bitset over the patches per literal), when a bitset fits one 32-bit word per
 // wave lane.
 __host__ __device__ constexpr bool literal_major(const Geom& g) { return g.P > 1 && (g.P + 31) / 32 <= 64; }
+// Clause evaluation on the matrix cores (mm_tile): literal steps of 64 of a product over the
+// positive literals, and whether a model's training kernel may take them (the samples' negated
+// literals are then complements of the positive ones).
+constexpr int kMmSteps = 8;
+__host__ __device__ constexpr int64_t mm_steps(const Geom& g) { return ((g.append_negated ? g.Lh : g.L) + 63) / 64; }
+__host__ __device__ constexpr bool mm_fits(const Geom& g) {
+  return literal_major(g) && g.W <= 32 && mm_steps(g) <= kMmSteps;
+}
 // The training kernel keeps the current literal-major sample in LDS when it fits 120 KiB.
 __host__ __device__ constexpr bool literal_major_lds(const Geom& g) {
-  return literal_major(g) && g.L * ((g.P + 31) / 32) * 4 <= 120 * 1024;
+  return !g.mma && literal_major(g) && g.L * ((g.P + 31) / 32) * 4 <= 120 * 1024;
 }
 
 // Streaming training kernel (train_stream_body): in-flight samples per workgroup (a power
