@@ -213,3 +213,30 @@ def test_training_on_several_patches(monkeypatch, dim, clauses, wgs, opts, env):
         np.testing.assert_array_equal(tm.get_ta_state().reshape(ref.ta.shape), ref.ta)
         np.testing.assert_array_equal(tm.get_weights().reshape(ref.w.shape), ref.w)
         np.testing.assert_array_equal(tm.get_patch_weights().reshape(ref.pw.shape), ref.pw)
+
+
+@pytest.mark.parametrize("clauses,wgs", [(130, "1"), (160, "2")])
+def test_first_sample_of_a_launch_counts_includes(monkeypatch, clauses, wgs):
+    """Injected fits of one sample each, so that every sample is the first of its launch: its
+    include counts, on both sides of max_included_literals over more clauses than a workgroup
+    has waves, decide between Type Ia and Ib feedback."""
+    monkeypatch.setenv("YTM_TRAIN_GLOBAL", "1")
+    monkeypatch.setenv("YTM_TRAIN_WGS", wgs)
+    print(f"[first sample] {clauses} {wgs}", flush=True)
+    rng = np.random.default_rng(12)
+    dim = (12, 12, 2)
+    tm, ref = pair(clauses, dim, 3, rng, patch_dim=(3, 3), max_included_literals=3)
+    counts = (ref.ta > 128).sum(-1)
+    assert (counts > 3).sum() > 20 and ((counts > 0) & (counts <= 3)).sum() > 20
+    X = image(rng, 8, dim)
+    y = rng.integers(0, 3, 8)
+    enc, encY = tm.encode(X), ref.encode_y_multiclass(y)
+    for e in range(8):
+        draws = rng.random(tm.random_stream_size(1)).astype(np.float32)
+        tm.fit(enc[e:e + 1], y[e:e + 1], is_X_encoded=True, random_stream=draws)
+        upd = ref.fit_encoded(enc[e:e + 1], encY[e:e + 1], inject=draws)
+        st = tm.stats()
+        assert st["train_kind"] == 2 and st["last_fit_updates"] == upd
+        np.testing.assert_array_equal(tm.get_ta_state().reshape(ref.ta.shape), ref.ta)
+        np.testing.assert_array_equal(tm.get_weights().reshape(ref.w.shape), ref.w)
+        np.testing.assert_array_equal(tm.get_patch_weights().reshape(ref.pw.shape), ref.pw)

@@ -1687,8 +1687,9 @@ __device__ __forceinline__ void train_global_body(const TrainArgs& a, const Geom
                                        s_lits + (int64_t)idx * cap, cap, a.lit_order);
       if (lane == 0) s_nlit[idx] = n;
     }
-  if (use_rb) {  // the rank bits of samples 0 and 1 (from the thresholds, once they are in LDS)
-    __syncthreads();
+  // mm: the first sample's include counts are read below by other waves than wrote them
+  if (mm || use_rb) __syncthreads();
+  if (use_rb) {  // the rank bits of samples 0 and 1 (from the thresholds, now in LDS)
     for (int j = 0; j < 2 && j < a.N; ++j) fill_rb(j, threadIdx.x, blockDim.x);
   }
   // The LDS copy of sample j (threads [first, first + count)): literal-major words, or with
