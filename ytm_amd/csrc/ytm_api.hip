@@ -79,8 +79,16 @@ namespace {
 thread_local std::string g_error;
 
 int fail(int code, const std::string& msg) {
+  if (code == YTM_EHIP) (void)hipGetLastError();  // or this thread's next launch would report it again
   g_error = msg;
   return code;
+}
+
+// Waits for stream s; a failure is not left for this thread's next launch to report.
+hipError_t settle(hipStream_t s) {
+  const hipError_t e = hipStreamSynchronize(s);
+  if (e != hipSuccess) (void)hipGetLastError();
+  return e;
 }
 
 #define HIP_TRY(expr)                                                                            \
@@ -88,6 +96,18 @@ int fail(int code, const std::string& msg) {
     hipError_t e_ = (expr);                                                                      \
     if (e_ != hipSuccess)                                                                        \
       return fail(YTM_EHIP, std::string(#expr) + " failed: " + hipGetErrorString(e_));           \
+  } while (0)
+
+// The same where work may be under way on stream s: an error waits for it first, since the
+// caller's arrays are borrowed for the call alone and blocks go back to the pool, which hands
+// them on without waiting.
+#define WAIT_TRY(s, expr)                                                                        \
+  do {                                                                                           \
+    hipError_t e_ = (expr);                                                                      \
+    if (e_ != hipSuccess) {                                                                      \
+      (void)settle(s);                                                                           \
+      return fail(YTM_EHIP, std::string(#expr) + " failed: " + hipGetErrorString(e_));           \
+    }                                                                                            \
   } while (0)
 
 int ceil_log2(int64_t x) {
@@ -221,10 +241,15 @@ size_t dtype_size(int dtype) {
   }
 }
 
+// A new block *dst with a copy of src, made on stream s; null on failure.
 int upload(void** dst, const void* src, size_t bytes, hipStream_t s) {
   HIP_TRY(ytm::pool_alloc(dst, bytes));
-  if (bytes) HIP_TRY(hipMemcpyAsync(*dst, src, bytes, hipMemcpyHostToDevice, s));
-  return YTM_OK;
+  const hipError_t e = bytes ? hipMemcpyAsync(*dst, src, bytes, hipMemcpyHostToDevice, s) : hipSuccess;
+  if (e == hipSuccess) return YTM_OK;
+  (void)settle(s);
+  ytm::pool_free(*dst);
+  *dst = nullptr;
+  return fail(YTM_EHIP, std::string("copy to the device failed: ") + hipGetErrorString(e));
 }
 
 // Picks the persistent grid (one workgroup per CU at most, at least ~12 clauses each, and
@@ -402,13 +427,14 @@ int fit_steps(ytm_model* m, const ytm_dataset* ds, int64_t first, int64_t count,
   if (inj) {
     hipError_t e = ytm::pool_alloc((void**)&d_inj, (size_t)(chunk * block) * 4);
     if (e != hipSuccess) {
-      (void)hipStreamSynchronize(m->stream);  // before the buffer is used again
+      (void)settle(m->stream);  // before the buffer is used again
       ytm::pool_free(d_drop);
       return fail(YTM_EHIP, std::string("hipMalloc(inject) failed: ") + hipGetErrorString(e));
     }
   }
   auto finish = [&](int code) {
-    (void)hipStreamSynchronize(m->stream);
+    const hipError_t idle = settle(m->stream);
+    if (!code && idle != hipSuccess) code = fail(YTM_EHIP, std::string("fit failed: ") + hipGetErrorString(idle));
     ytm::pool_free(d_drop);
     ytm::pool_free(d_inj);
     return code;
@@ -540,7 +566,7 @@ int ytm_create(const ytm_params* params, ytm_model** out) {
 
 void ytm_destroy(ytm_model* m) {
   if (!m) return;
-  if (m->stream) (void)hipStreamSynchronize(m->stream);
+  if (m->stream) (void)settle(m->stream);
   void* bufs[] = {m->d_planes, m->d_w,    m->d_pw,   m->d_bias, m->d_ninc,  m->d_inv_rank,
                   m->d_counters, m->d_err, m->d_slots, m->d_sacc, m->d_sout, m->d_slists};
   for (void* b : bufs)
@@ -661,7 +687,7 @@ int ytm_encode(ytm_model* m, const uint32_t* X, int64_t N, uint32_t* out) {
     if (e != hipSuccess) rc = fail(YTM_EHIP, std::string("encode failed: ") + hipGetErrorString(e));
   }
   m->stats.last_encode_kernel_ms = ms_total;
-  if (rc) (void)hipStreamSynchronize(m->stream);  // before the buffers are used again
+  if (rc) (void)settle(m->stream);  // before the buffers are used again
   ytm::pool_free(dX);
   ytm::pool_free(dO);
   return rc;
@@ -711,7 +737,7 @@ int ytm_encode_binarized(ytm_model* m, const void* X, int x_dtype, int64_t N, co
   }
   if (!rc && e != hipSuccess) rc = fail(YTM_EHIP, std::string("encode failed: ") + hipGetErrorString(e));
   m->stats.last_encode_kernel_ms = ms_total;
-  if (rc) (void)hipStreamSynchronize(m->stream);  // before the buffers are used again
+  if (rc) (void)settle(m->stream);  // before the buffers are used again
   ytm::pool_free(dT);
   ytm::pool_free(dX);
   ytm::pool_free(dO);
@@ -764,7 +790,7 @@ int ytm_dataset_create(ytm_model* m, const uint32_t* encX, const int32_t* encY, 
     if (e != hipSuccess) rc = fail(YTM_EHIP, hipGetErrorString(e));
   }
   if (rc) {
-    (void)hipStreamSynchronize(m->stream);  // before the buffers are used again
+    (void)settle(m->stream);  // before the buffers are used again
     ytm_dataset_destroy(ds);
     return rc;
   }
@@ -923,13 +949,14 @@ int fit_range(ytm_model* m, const ytm_dataset* ds, int64_t first, int64_t count,
   if (inj) {
     hipError_t e = ytm::pool_alloc((void**)&d_inj, (size_t)(per_launch * block) * 4);
     if (e != hipSuccess) {
-      (void)hipStreamSynchronize(m->stream);  // before the buffer is used again
+      (void)settle(m->stream);  // before the buffer is used again
       ytm::pool_free(d_drop);
       return fail(YTM_EHIP, std::string("hipMalloc(inject) failed: ") + hipGetErrorString(e));
     }
   }
   auto finish = [&](int code) {
-    (void)hipStreamSynchronize(m->stream);
+    const hipError_t idle = settle(m->stream);
+    if (!code && idle != hipSuccess) code = fail(YTM_EHIP, std::string("fit failed: ") + hipGetErrorString(idle));
     ytm::pool_free(d_drop);
     ytm::pool_free(d_inj);
     return code;
@@ -1180,7 +1207,6 @@ int ytm_score_dataset(ytm_model* m, const ytm_dataset* ds, float* class_sums) {
   // operands that depend on the model alone are kept from the last call
   bool lists_ready = plan.kept() && m->slists_kind == plan.kept() && m->slists_version == m->state_version;
   float* dout = (float*)m->d_sout;
-  int rc = YTM_OK;
   // the include counts, for the scorers that read them (the list-based ones count their lists)
   if (e == hipSuccess && !plan.lists_bytes) e = ytm::launch_ninc(m->d_planes, m->d_ninc, g, m->stream);
   if (e == hipSuccess) e = hipEventRecord(m->ev0, m->stream);
@@ -1208,9 +1234,13 @@ int ytm_score_dataset(ytm_model* m, const ytm_dataset* ds, float* class_sums) {
   if (e == hipSuccess) std::memcpy(class_sums, m->h_sout, out_bytes);
   float ms = 0.0f;
   if (e == hipSuccess) e = hipEventElapsedTime(&ms, m->ev0, m->ev1);
-  if (e != hipSuccess) rc = fail(YTM_EHIP, std::string("score failed: ") + hipGetErrorString(e));
+  if (e != hipSuccess) {
+    m->slists_version = ~0ull;
+    (void)settle(m->stream);  // before the samples and the buffers are used again
+    return fail(YTM_EHIP, std::string("score failed: ") + hipGetErrorString(e));
+  }
   m->stats.last_score_kernel_ms = ms;
-  return rc;
+  return YTM_OK;
 }
 
 int ytm_score_dataset_noalloc(ytm_model* m, const ytm_dataset* ds, float* d_class_sums) {
@@ -1252,7 +1282,10 @@ int ytm_score_dataset_noalloc(ytm_model* m, const ytm_dataset* ds, float* d_clas
   if (e == hipSuccess) e = hipStreamSynchronize(m->stream);
   float ms = 0.0f;
   if (e == hipSuccess) e = hipEventElapsedTime(&ms, m->ev0, m->ev1);
-  if (e != hipSuccess) return fail(YTM_EHIP, std::string("score failed: ") + hipGetErrorString(e));
+  if (e != hipSuccess) {
+    (void)settle(m->stream);  // before another call has the scratch
+    return fail(YTM_EHIP, std::string("score failed: ") + hipGetErrorString(e));
+  }
   m->stats.last_score_kernel_ms = ms;
   return YTM_OK;
 }
@@ -1308,7 +1341,7 @@ int ytm_transform(ytm_model* m, const uint32_t* encX, int64_t N, int mode, uint3
     if (e == hipSuccess) e = hipStreamSynchronize(m->stream);
   }
   const int rc = e == hipSuccess ? YTM_OK : fail(YTM_EHIP, std::string("transform failed: ") + hipGetErrorString(e));
-  if (rc) (void)hipStreamSynchronize(m->stream);  // before the buffers are used again
+  if (rc) (void)settle(m->stream);  // before the buffers are used again
   ytm::pool_free(dX);
   ytm::pool_free(dO);
   ytm::pool_free(dXT);
@@ -1324,7 +1357,7 @@ int ytm_get_ta_state(ytm_model* m, uint32_t* out) {
   hipError_t e = ytm::launch_planes_to_ta(m->d_planes, d, g, m->stream);
   if (e == hipSuccess) e = ytm::copy_to_host(out, d, (size_t)(g.C * g.L) * 4, m->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(m->stream);
-  if (e != hipSuccess) (void)hipStreamSynchronize(m->stream);  // before the buffer is used again
+  if (e != hipSuccess) (void)settle(m->stream);  // before the buffer is used again
   ytm::pool_free(d);
   if (e != hipSuccess) return fail(YTM_EHIP, std::string("get_ta_state failed: ") + hipGetErrorString(e));
   return YTM_OK;
@@ -1342,14 +1375,10 @@ int ytm_set_ta_state(ytm_model* m, const uint32_t* in) {
                                   std::to_string(limit));
   uint32_t* d = nullptr;
   int rc = upload((void**)&d, in, (size_t)(g.C * g.L) * 4, m->stream);
-  if (rc) {
-    (void)hipStreamSynchronize(m->stream);
-    ytm::pool_free(d);
-    return rc;
-  }
+  if (rc) return rc;
   hipError_t e = ytm::launch_ta_to_planes(d, m->d_planes, g, m->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(m->stream);
-  if (e != hipSuccess) (void)hipStreamSynchronize(m->stream);  // before the buffer is used again
+  if (e != hipSuccess) (void)settle(m->stream);  // before the buffer is used again
   ytm::pool_free(d);
   if (e != hipSuccess) return fail(YTM_EHIP, std::string("set_ta_state failed: ") + hipGetErrorString(e));
   note_reload(m, 1);
@@ -1358,7 +1387,7 @@ int ytm_set_ta_state(ytm_model* m, const uint32_t* in) {
 
 int ytm_get_weights(ytm_model* m, float* out) {
   if (!m || !out) return fail(YTM_EINVAL, "null argument");
-  HIP_TRY(ytm::copy_to_host(out, m->d_w, (size_t)(m->g.C * m->g.K) * 4, m->stream));
+  WAIT_TRY(m->stream, ytm::copy_to_host(out, m->d_w, (size_t)(m->g.C * m->g.K) * 4, m->stream));
   return YTM_OK;
 }
 
@@ -1370,8 +1399,8 @@ int ytm_set_weights(ytm_model* m, const float* in) {
       return fail(YTM_ERANGE, "clause weights must be integer-valued floats below 2^31 in magnitude");
   }
   ++m->state_version;
-  HIP_TRY(hipMemcpyAsync(m->d_w, in, (size_t)(m->g.C * m->g.K) * 4, hipMemcpyHostToDevice, m->stream));
-  HIP_TRY(hipStreamSynchronize(m->stream));
+  WAIT_TRY(m->stream, hipMemcpyAsync(m->d_w, in, (size_t)(m->g.C * m->g.K) * 4, hipMemcpyHostToDevice, m->stream));
+  WAIT_TRY(m->stream, hipStreamSynchronize(m->stream));
   double bound = 0.0;
   for (int64_t i = 0; i < m->g.C * m->g.K; ++i) bound = std::max(bound, (double)std::fabs(in[i]));
   m->w_bound = bound;
@@ -1381,22 +1410,22 @@ int ytm_set_weights(ytm_model* m, const float* in) {
 
 int ytm_get_patch_weights(ytm_model* m, int32_t* out) {
   if (!m || !out) return fail(YTM_EINVAL, "null argument");
-  HIP_TRY(ytm::copy_to_host(out, m->d_pw, (size_t)(m->g.C * m->g.P) * 4, m->stream));
+  WAIT_TRY(m->stream, ytm::copy_to_host(out, m->d_pw, (size_t)(m->g.C * m->g.P) * 4, m->stream));
   return YTM_OK;
 }
 
 int ytm_set_patch_weights(ytm_model* m, const int32_t* in) {
   if (!m || !in) return fail(YTM_EINVAL, "null argument");
-  HIP_TRY(hipMemcpyAsync(m->d_pw, in, (size_t)(m->g.C * m->g.P) * 4, hipMemcpyHostToDevice, m->stream));
-  HIP_TRY(hipStreamSynchronize(m->stream));
+  WAIT_TRY(m->stream, hipMemcpyAsync(m->d_pw, in, (size_t)(m->g.C * m->g.P) * 4, hipMemcpyHostToDevice, m->stream));
+  WAIT_TRY(m->stream, hipStreamSynchronize(m->stream));
   note_reload(m, 4);
   return YTM_OK;
 }
 
 int ytm_get_bias(ytm_model* m, float* out) {
   if (!m || !out) return fail(YTM_EINVAL, "null argument");
-  HIP_TRY(hipMemcpyAsync(out, m->d_bias, (size_t)m->g.K * 4, hipMemcpyDeviceToHost, m->stream));
-  HIP_TRY(hipStreamSynchronize(m->stream));
+  WAIT_TRY(m->stream, hipMemcpyAsync(out, m->d_bias, (size_t)m->g.K * 4, hipMemcpyDeviceToHost, m->stream));
+  WAIT_TRY(m->stream, hipStreamSynchronize(m->stream));
   return YTM_OK;
 }
 
@@ -1432,7 +1461,7 @@ int ytm_binarize(const void* X, int x_dtype, int64_t n, const void* thresholds, 
     e = ytm::launch_binarize(dX, x_dtype, n, dT, int_thresholds != 0, nthr, kind == 1, edge_bins != 0, dO, nullptr);
   if (!rc && e == hipSuccess) e = ytm::copy_to_host(out, dO, (size_t)(n * width) * 4, nullptr);
   if (!rc && e != hipSuccess) rc = fail(YTM_EHIP, std::string("binarize failed: ") + hipGetErrorString(e));
-  if (rc) (void)hipStreamSynchronize(nullptr);  // before the buffers are used again
+  if (rc) (void)settle(nullptr);  // before the buffers are used again
   ytm::pool_free(dX);
   ytm::pool_free(dT);
   ytm::pool_free(dO);
@@ -1452,7 +1481,7 @@ int ytm_collapse_bins(const uint32_t* B, int64_t rows, int64_t width, int kind, 
     e = ytm::launch_collapse_bins((const uint32_t*)dB, rows, width, kind == 1, edge_bins != 0, dO, nullptr);
   if (!rc && e == hipSuccess) e = ytm::copy_to_host(out, dO, (size_t)rows * 8, nullptr);
   if (!rc && e != hipSuccess) rc = fail(YTM_EHIP, std::string("collapse_bins failed: ") + hipGetErrorString(e));
-  if (rc) (void)hipStreamSynchronize(nullptr);  // before the buffers are used again
+  if (rc) (void)settle(nullptr);  // before the buffers are used again
   ytm::pool_free(dB);
   ytm::pool_free(dO);
   return rc;

@@ -170,6 +170,7 @@ hipError_t copy_to_host(void* dst, const void* src, size_t bytes, hipStream_t s)
   // runtime's own copy
   if (bytes < kStaged || threads < 2 || hipGetDevice(&device) != hipSuccess || !lock.try_lock() ||
       ready_staging(device) != hipSuccess) {
+    (void)hipGetLastError();
     const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s);
     return e != hipSuccess ? e : hipStreamSynchronize(s);
   }
@@ -203,6 +204,10 @@ hipError_t copy_to_host(void* dst, const void* src, size_t bytes, hipStream_t s)
       const hipError_t err = hipStreamSynchronize(st);
       if (err != hipSuccess) failed = (int)err;
       before = i;
+    }
+    if (failed != (int)hipSuccess) {  // the buffers are used again
+      (void)hipStreamSynchronize(st);
+      (void)hipGetLastError();
     }
   };
   std::vector<std::thread> others;
