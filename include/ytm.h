@@ -123,7 +123,8 @@ const char *ytm_last_error(void);
  * exits; call it after destroying every model and dataset.  A later fit loads what it needs
  * again.  Replaces the context teardown that `import pycuda.autoinit` registers for process
  * exit (src/cutm/base.py:5), which releases the modules SourceModule loaded
- * (src/cutm/base.py:155-159).  YTM_EHIP when a module fails to unload. */
+ * (src/cutm/base.py:155-159).  Also frees every device block kept between calls (ytm_create) and
+ * the pinned buffers of large copies.  YTM_EHIP when a module fails to unload. */
 int ytm_shutdown(void);
 
 /* Model lifetime.  Replaces BaseTM._gpu_init / _reset_clauses / _reset_weights
@@ -132,7 +133,12 @@ int ytm_shutdown(void);
  * Geometry bounds: at most 4096 classes (the reference's kernels take any CLASSES; more
  * than 64 train one sample per launch), any number of patches, any int32
  * number_of_ta_states (up to 32 bit-planes), classes * literal words * 6 below 2^32 (the
- * 32-bit literal-draw site index of the counter stream).  YTM_EINVAL otherwise. */
+ * 32-bit literal-draw site index of the counter stream).  YTM_EINVAL otherwise.
+ *
+ * Device memory that a call is done with (buffers of its host arrays, a destroyed data set's or
+ * model's) is kept for later calls while a model lives on that device, at most 1 GiB of it
+ * idle, the longest unused freed first; ytm_destroy of the device's last model frees it all.
+ * Another allocator of the process cannot have it before. */
 int ytm_create(const ytm_params *params, ytm_model **out);
 void ytm_destroy(ytm_model *m);
 /* L, W (=number_of_literal_chunks), P (=number_of_patches), number of TA bit-planes. */

@@ -7,6 +7,7 @@
 #include <pthread.h>
 #include <stdlib.h>
 #include <string.h>
+#include <unistd.h>
 
 #define DEVICES 2
 #define BLOCKS 65536
@@ -45,6 +46,8 @@ size_t fake_live(int dev) { /* bytes allocated on a device (-1: pinned) */
     pthread_mutex_unlock(&mu);
     return n;
 }
+static int delay_ms;
+void fake_delay_malloc(int ms) { delay_ms = ms; } /* each hipMalloc takes that long */
 long fake_calls(int which) {
     const long c[] = {calls_malloc, calls_free, calls_host_malloc, calls_host_free};
     return c[which];
@@ -86,6 +89,7 @@ static hipError_t drop(void *p, int host) {
 hipError_t hipMalloc(void **p, size_t bytes) {
     MAY_FAIL;
     __sync_fetch_and_add(&calls_malloc, 1);
+    if (delay_ms) usleep(1000 * delay_ms);
     return get(p, bytes, device);
 }
 hipError_t hipFree(void *p) {

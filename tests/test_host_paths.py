@@ -1,7 +1,11 @@
-"""libytm's host code on a HIP runtime of host memory (fake_hip.c): every HIP call that an entry
-point makes fails in turn.  The entry point then reports an error, leaves no work behind on its
-stream (its blocks go back to the pool, which hands them on without waiting), and loses no
-memory.  In a child process, since the runtime stands in for the real one."""
+"""libytm's host code on a HIP runtime of host memory (fake_hip.c), in a child process, since the
+runtime stands in for the real one.
+
+Error exits: every HIP call that an entry point makes fails in turn.  The entry point then
+reports an error, leaves no work behind on its stream (its blocks go back to the pool, which
+hands them on without waiting), and loses no memory.
+
+Memory: which device blocks are kept between calls, and when they are given back."""
 import ctypes
 import os
 import subprocess
@@ -41,6 +45,11 @@ ENTRIES = ["create", "encode", "encode_binarized", "dataset", "dataset_targets",
 @pytest.mark.parametrize("entry", ENTRIES)
 def test_every_call_failing(fake_hip, entry):
     child(fake_hip, entry)
+
+
+@pytest.mark.parametrize("what", ["oldest_leave_first", "given_back_with_the_last_model", "allocations_unlocked"])
+def test_blocks(fake_hip, what):
+    child(fake_hip, what)
 
 
 # ------------------------------------------------------------------------------ the child
@@ -187,6 +196,69 @@ def entry(name, lib, L):
     }[name]()
 
 
+def binarize(lib, n):
+    """A call with blocks of n and 4 n bytes."""
+    X, t, out = np.zeros(n, np.uint8), np.zeros(1, np.float64), np.empty(n, np.uint32)
+    assert lib.ytm_binarize(X.ctypes.data, 0, n, t.ctypes.data, 0, 1, 0, 0, out.ctypes.data) == 0
+
+
+def small_model(lib, L):
+    p = L.YtmParams(clauses=40, classes=3, dim0=20, dim1=1, dim2=1, patch_dim0=20, patch_dim1=1, number_of_ta_states=256,
+                    max_included_literals=40, append_negated=1, encode_loc=1, coalesced=1, negative_polarity=1,
+                    thresh=10, s_inv=0.2, q_prob=1.0, seed=1)
+    m = ctypes.c_void_p()
+    assert lib.ytm_create(ctypes.byref(p), ctypes.byref(m)) == 0
+    return m
+
+
+MALLOC, FREE, HOST_MALLOC, HOST_FREE = range(4)
+MB = 1 << 20
+
+
+def oldest_leave_first(fake, lib, L):
+    """Blocks of sizes that no call asks for any more make room for those that calls use."""
+    m = small_model(lib, L)
+    binarize(lib, 203 * MB)  # blocks of 204 and 812 MB, just below what is kept
+    binarize(lib, 3 * MB)
+    before = fake.fake_calls(MALLOC)
+    for _ in range(5):
+        binarize(lib, 3 * MB)
+    assert fake.fake_calls(MALLOC) == before, "the blocks of the latest calls were not kept"
+    assert fake.fake_live(0) < 1100 * MB, fake.fake_live(0)
+    lib.ytm_destroy(m)
+
+
+def given_back_with_the_last_model(fake, lib, L):
+    binarize(lib, 3 * MB)
+    assert fake.fake_live(0) == 0, "blocks kept without a model"
+    a, b = small_model(lib, L), small_model(lib, L)
+    binarize(lib, 3 * MB)
+    lib.ytm_destroy(a)
+    assert fake.fake_live(0) > 15 * MB, "blocks given back although a model lives"
+    lib.ytm_destroy(b)
+    assert fake.fake_live(0) == 0, fake.fake_live(0)
+
+
+def allocations_unlocked(fake, lib, L):
+    """A long hipMalloc of one thread keeps no other thread from blocks that are idle."""
+    import threading
+    import time
+
+    m = small_model(lib, L)
+    binarize(lib, 1000)
+    fake.fake_delay_malloc(1000)
+    t = threading.Thread(target=binarize, args=(lib, 5 * MB))
+    t.start()
+    time.sleep(0.3)
+    start = time.perf_counter()
+    binarize(lib, 1000)
+    took = time.perf_counter() - start
+    t.join()
+    fake.fake_delay_malloc(0)
+    lib.ytm_destroy(m)
+    assert took < 0.4, took
+
+
 def every_call_failing(name, fake, lib, L):
     prepare, call, free = entry(name, lib, L)
     wrong = []
@@ -223,4 +295,7 @@ if __name__ == "__main__":
     fake.fake_calls.restype = ctypes.c_long
     from ytm_amd import _lib
 
-    every_call_failing(sys.argv[2], fake, _lib.lib, _lib)
+    if sys.argv[2] in ENTRIES:
+        every_call_failing(sys.argv[2], fake, _lib.lib, _lib)
+    else:
+        globals()[sys.argv[2]](fake, _lib.lib, _lib)

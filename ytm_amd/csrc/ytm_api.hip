@@ -19,6 +19,7 @@ struct ytm_model {
   ytm_params params;
   Geom g;
   int device = 0;
+  bool held = false;  // memory_hold of its device
   int cus = 0;
   hipStream_t stream = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -530,6 +531,7 @@ int ytm_create(const ytm_params* params, ytm_model** out) {
     return code;
   };
   if (hipGetDevice(&m->device) != hipSuccess) return cleanup(fail(YTM_EHIP, "no HIP device"));
+  m->held = ytm::memory_hold(m->device);
   hipDeviceProp_t prop;
   if (hipGetDeviceProperties(&prop, m->device) != hipSuccess) return cleanup(fail(YTM_EHIP, "device query failed"));
   m->cus = prop.multiProcessorCount;
@@ -575,6 +577,7 @@ void ytm_destroy(ytm_model* m) {
   if (m->ev0) (void)hipEventDestroy(m->ev0);
   if (m->ev1) (void)hipEventDestroy(m->ev1);
   if (m->stream) (void)hipStreamDestroy(m->stream);
+  if (m->held) ytm::memory_release(m->device);
   delete m;
 }
 

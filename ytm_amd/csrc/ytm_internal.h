@@ -15,6 +15,10 @@ namespace ytm {
 // whatever they held before; a block is freed once nothing on the GPU uses it any more.
 hipError_t pool_alloc(void** p, size_t bytes);
 void pool_free(void* p);
+// A model that lives on a device (false: nothing is kept for it) and its end: the device's blocks
+// are kept while one does.
+bool memory_hold(int device);
+void memory_release(int device);
 // Copies device memory to a host array after the work of stream s; done on return.
 hipError_t copy_to_host(void* dst, const void* src, size_t bytes, hipStream_t s);
 // Gives everything kept back to the devices and the host.

@@ -4,8 +4,9 @@
 // inputs and outputs for the length of the call.  A hipMalloc and hipFree above 2 MB take 40 to
 // 290 us a pair, which for a call of a few hundred microseconds is most of it, and so does a
 // small one that finds the runtime's own chunk of small blocks gone; blocks are therefore kept
-// here when a call is done with them, up to kKeep bytes a device, and given back by memory_trim
-// (ytm_shutdown) or when an allocation fails.
+// here when a call is done with them, while a model lives on their device: up to kKeep bytes a
+// device, the longest unused given back first.  All are given back with the device's last
+// model, by memory_trim (ytm_shutdown), and when an allocation fails.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -27,32 +28,47 @@ namespace {
 constexpr size_t kSmall = (size_t)1 << 20;  // below: powers of two
 constexpr size_t kUnit = (size_t)2 << 20;   // from there on: whole units
 constexpr size_t kKeep = (size_t)1 << 30;   // idle bytes kept per device
+constexpr int kDevices = 64;                // devices whose blocks are kept
 
 struct Block {
   int device;
   size_t bytes;
 };
+struct Idle {
+  void* p;
+  uint64_t since;  // count of blocks given back before it
+};
+struct Pool {
+  std::multimap<size_t, Idle> idle;  // by size
+  size_t idle_bytes = 0;
+  int models = 0;  // living on the device
+};
 
+// Held for the books alone: the runtime's own calls, which may take long, are made outside.
 std::mutex g_mu;
-std::unordered_map<void*, Block> g_blocks;             // every block handed out or idle
-std::map<int, std::multimap<size_t, void*>> g_idle;    // device -> size -> block
-std::map<int, size_t> g_idle_bytes;
+std::unordered_map<void*, Block> g_blocks;  // every block handed out or idle
+std::map<int, Pool> g_pools;                // by device
+uint64_t g_given_back = 0;
 
-// Frees the idle blocks of `device` (-1: of all); the caller holds g_mu.
-void trim_locked(int device) {
-  int prev = 0;
-  (void)hipGetDevice(&prev);
-  for (auto& d : g_idle) {
-    if (device >= 0 && d.first != device) continue;
-    (void)hipSetDevice(d.first);
-    for (auto& b : d.second) {
-      (void)hipFree(b.second);
-      g_blocks.erase(b.second);
-    }
-    d.second.clear();
-    g_idle_bytes[d.first] = 0;
-  }
-  (void)hipSetDevice(prev);
+// Takes the longest idle block of a device out of the books while more than `keep` bytes are
+// idle there; null when they are not.
+void* take_oldest(int device, size_t keep) {
+  std::lock_guard<std::mutex> lock(g_mu);
+  const auto pool = g_pools.find(device);
+  if (pool == g_pools.end() || pool->second.idle_bytes <= keep) return nullptr;
+  auto& idle = pool->second.idle;
+  auto oldest = idle.begin();
+  for (auto it = idle.begin(); it != idle.end(); ++it)
+    if (it->second.since < oldest->second.since) oldest = it;
+  void* p = oldest->second.p;
+  pool->second.idle_bytes -= oldest->first;
+  idle.erase(oldest);
+  g_blocks.erase(p);
+  return p;
+}
+
+void trim_device(int device, size_t keep) {
+  while (void* p = take_oldest(device, keep)) (void)hipFree(p);
 }
 
 }  // namespace
@@ -67,22 +83,28 @@ hipError_t pool_alloc(void** p, size_t bytes) {
   int device = 0;
   hipError_t e = hipGetDevice(&device);
   if (e != hipSuccess) return e;
-  std::lock_guard<std::mutex> lock(g_mu);
-  auto& idle = g_idle[device];
-  const auto it = idle.lower_bound(want);
-  if (it != idle.end() && it->first <= want + want / 2) {  // at most half as much again is left unused
-    *p = it->second;
-    g_idle_bytes[device] -= it->first;
-    idle.erase(it);
-    return hipSuccess;
+  {
+    std::lock_guard<std::mutex> lock(g_mu);
+    const auto pool = g_pools.find(device);
+    if (pool != g_pools.end()) {
+      auto& idle = pool->second.idle;
+      const auto it = idle.lower_bound(want);
+      if (it != idle.end() && it->first <= want + want / 2) {  // at most half as much again is left unused
+        *p = it->second.p;
+        pool->second.idle_bytes -= it->first;
+        idle.erase(it);
+        return hipSuccess;
+      }
+    }
   }
   e = hipMalloc(p, want);
   if (e != hipSuccess) {
     (void)hipGetLastError();
-    trim_locked(device);
+    trim_device(device, 0);
     e = hipMalloc(p, want);
   }
   if (e != hipSuccess) return e;
+  std::lock_guard<std::mutex> lock(g_mu);
   try {
     g_blocks[*p] = Block{device, want};
   } catch (...) {  // not kept later then
@@ -92,23 +114,48 @@ hipError_t pool_alloc(void** p, size_t bytes) {
 
 void pool_free(void* p) {
   if (!p) return;
+  int device = -1;
+  bool kept = false;
   {
     std::lock_guard<std::mutex> lock(g_mu);
     const auto it = g_blocks.find(p);
     if (it != g_blocks.end()) {
       const Block b = it->second;
-      try {
-        if (g_idle_bytes[b.device] + b.bytes <= kKeep) {
-          g_idle[b.device].emplace(b.bytes, p);
-          g_idle_bytes[b.device] += b.bytes;
-          return;
+      device = b.device;
+      const auto pool = g_pools.find(device);
+      if (pool != g_pools.end() && pool->second.models > 0 && b.bytes <= kKeep) try {
+          pool->second.idle.emplace(b.bytes, Idle{p, g_given_back++});
+          pool->second.idle_bytes += b.bytes;
+          kept = true;
+        } catch (...) {  // freed instead
         }
-      } catch (...) {  // freed instead
-      }
-      g_blocks.erase(it);
+      if (!kept) g_blocks.erase(it);
     }
   }
-  (void)hipFree(p);
+  if (!kept)
+    (void)hipFree(p);
+  else
+    trim_device(device, kKeep);
+}
+
+bool memory_hold(int device) {
+  if (device < 0 || device >= kDevices) return false;
+  std::lock_guard<std::mutex> lock(g_mu);
+  try {
+    ++g_pools[device].models;
+  } catch (...) {
+    return false;
+  }
+  return true;
+}
+
+void memory_release(int device) {
+  {
+    std::lock_guard<std::mutex> lock(g_mu);
+    const auto pool = g_pools.find(device);
+    if (pool == g_pools.end() || --pool->second.models > 0) return;
+  }
+  trim_device(device, 0);
 }
 
 // ------------------------------------------------------------------ copies to host arrays
@@ -221,10 +268,7 @@ hipError_t copy_to_host(void* dst, const void* src, size_t bytes, hipStream_t s)
 }
 
 void memory_trim() {
-  {
-    std::lock_guard<std::mutex> lock(g_mu);
-    trim_locked(-1);
-  }
+  for (int device = 0; device < kDevices; ++device) trim_device(device, 0);
   std::lock_guard<std::mutex> lock(g_staging_mu);
   release_staging();
 }
