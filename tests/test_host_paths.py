@@ -47,7 +47,7 @@ def test_every_call_failing(fake_hip, entry):
     child(fake_hip, entry)
 
 
-@pytest.mark.parametrize("what", ["oldest_leave_first", "given_back_with_the_last_model", "allocations_unlocked"])
+@pytest.mark.parametrize("what", ["oldest_leave_first", "given_back_with_the_last_model", "allocations_unlocked", "staging_per_device"])
 def test_blocks(fake_hip, what):
     child(fake_hip, what)
 
@@ -257,6 +257,23 @@ def allocations_unlocked(fake, lib, L):
     fake.fake_delay_malloc(0)
     lib.ytm_destroy(m)
     assert took < 0.4, took
+
+
+def staging_per_device(fake, lib, L):
+    """Large copies from two devices in turn make each device's pinned buffers once."""
+    models = []
+    for d in (0, 1):
+        assert fake.hipSetDevice(d) == 0
+        models.append(small_model(lib, L))
+    for _ in range(3):
+        for d in (0, 1):
+            assert fake.hipSetDevice(d) == 0
+            binarize(lib, 3 * MB)
+    assert fake.fake_calls(HOST_MALLOC) == 2, fake.fake_calls(HOST_MALLOC)
+    lib.ytm_destroy(models[0])
+    assert fake.fake_calls(HOST_FREE) == 1 and fake.fake_live(0) == 0 and fake.fake_live(1) > 0
+    lib.ytm_destroy(models[1])
+    assert fake.fake_live(-1) == 0 and fake.fake_live(1) == 0
 
 
 def every_call_failing(name, fake, lib, L):

@@ -149,15 +149,6 @@ bool memory_hold(int device) {
   return true;
 }
 
-void memory_release(int device) {
-  {
-    std::lock_guard<std::mutex> lock(g_mu);
-    const auto pool = g_pools.find(device);
-    if (pool == g_pools.end() || --pool->second.models > 0) return;
-  }
-  trim_device(device, 0);
-}
-
 // ------------------------------------------------------------------ copies to host arrays
 // A copy of many megabytes into a numpy array that was just allocated runs at 10 GB/s through
 // the runtime (its single staging thread also takes the array's page faults); the link
@@ -172,51 +163,55 @@ constexpr size_t kPiece = (size_t)1 << 20;
 constexpr size_t kStaged = (size_t)4 << 20;  // from here on (below, starting the threads costs as much as it saves)
 constexpr int kThreads = 8;
 
+// A device's buffers and streams (a program that copies from several devices in turn keeps each
+// one's: making them takes milliseconds), until its last model or memory_trim.
 struct Staging {
-  int device = -1;
+  std::mutex mu;  // held for a whole copy
   unsigned char* pinned = nullptr;  // [kThreads][2][kPiece]
   hipStream_t stream[kThreads] = {};
 };
-std::mutex g_staging_mu;  // held for a whole copy
-Staging g_staging;
+Staging g_staging[kDevices];
 
-void release_staging() {
-  Staging& s = g_staging;
-  if (s.device < 0) return;
-  int prev = 0;
-  (void)hipGetDevice(&prev);
-  (void)hipSetDevice(s.device);
-  for (hipStream_t& st : s.stream) {
+// Both with g.mu held; ready_staging with the device current.
+void release_staging(Staging& g) {
+  for (hipStream_t& st : g.stream) {
     if (st) (void)hipStreamDestroy(st);
     st = nullptr;
   }
-  if (s.pinned) (void)hipHostFree(s.pinned);
-  (void)hipSetDevice(prev);
-  s = Staging{};
+  if (g.pinned) (void)hipHostFree(g.pinned);
+  g.pinned = nullptr;
 }
 
-hipError_t ready_staging(int device) {
-  if (g_staging.device == device) return hipSuccess;
-  release_staging();
-  g_staging.device = device;
-  hipError_t e = hipHostMalloc((void**)&g_staging.pinned, kThreads * 2 * kPiece, hipHostMallocDefault);
-  for (hipStream_t& st : g_staging.stream)
+hipError_t ready_staging(Staging& g) {
+  if (g.pinned) return hipSuccess;
+  hipError_t e = hipHostMalloc((void**)&g.pinned, kThreads * 2 * kPiece, hipHostMallocDefault);
+  if (e != hipSuccess) g.pinned = nullptr;
+  for (hipStream_t& st : g.stream)
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&st, hipStreamNonBlocking);
-  if (e != hipSuccess) release_staging();
+  if (e != hipSuccess) release_staging(g);
   return e;
+}
+
+void trim_staging(int device) {
+  std::lock_guard<std::mutex> lock(g_staging[device].mu);
+  release_staging(g_staging[device]);
 }
 
 }  // namespace
 
 hipError_t copy_to_host(void* dst, const void* src, size_t bytes, hipStream_t s) {
-  std::unique_lock<std::mutex> lock(g_staging_mu, std::defer_lock);
+  std::unique_lock<std::mutex> lock;
   int device = 0;
   static const int threads =  // asked once: the answer takes longer than a small copy
       (int)std::min<unsigned>(kThreads, std::max(1u, std::thread::hardware_concurrency() / 2));
   // another thread's copy has the buffers, there are few CPUs, or they cannot be had: the
   // runtime's own copy
-  if (bytes < kStaged || threads < 2 || hipGetDevice(&device) != hipSuccess || !lock.try_lock() ||
-      ready_staging(device) != hipSuccess) {
+  auto staged = [&] {
+    if (bytes < kStaged || threads < 2 || hipGetDevice(&device) != hipSuccess || device >= kDevices) return false;
+    lock = std::unique_lock<std::mutex>(g_staging[device].mu, std::try_to_lock);
+    return lock.owns_lock() && ready_staging(g_staging[device]) == hipSuccess;
+  };
+  if (!staged()) {
     (void)hipGetLastError();
     const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s);
     return e != hipSuccess ? e : hipStreamSynchronize(s);
@@ -231,8 +226,8 @@ hipError_t copy_to_host(void* dst, const void* src, size_t bytes, hipStream_t s)
       failed = (int)hipErrorInvalidDevice;
       return;
     }
-    unsigned char* buf = g_staging.pinned + (size_t)t * 2 * kPiece;
-    const hipStream_t st = g_staging.stream[t];
+    unsigned char* buf = g_staging[device].pinned + (size_t)t * 2 * kPiece;
+    const hipStream_t st = g_staging[device].stream[t];
     size_t before = pieces;  // the piece that lies in the other buffer
     auto move_on = [&](int b) {
       if (before < pieces)
@@ -267,10 +262,21 @@ hipError_t copy_to_host(void* dst, const void* src, size_t bytes, hipStream_t s)
   return (hipError_t)failed.load();
 }
 
+void memory_release(int device) {
+  {
+    std::lock_guard<std::mutex> lock(g_mu);
+    const auto pool = g_pools.find(device);
+    if (pool == g_pools.end() || --pool->second.models > 0) return;
+  }
+  trim_device(device, 0);
+  trim_staging(device);
+}
+
 void memory_trim() {
-  for (int device = 0; device < kDevices; ++device) trim_device(device, 0);
-  std::lock_guard<std::mutex> lock(g_staging_mu);
-  release_staging();
+  for (int device = 0; device < kDevices; ++device) {
+    trim_device(device, 0);
+    trim_staging(device);
+  }
 }
 
 }  // namespace ytm
