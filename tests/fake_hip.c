@@ -22,7 +22,7 @@ static __thread int device;
 static char fail_name[64];
 static int fail_after = -1, fail_count, fail_seen;
 static __thread hipError_t last_error;
-static long calls_malloc, calls_free, calls_host_malloc, calls_host_free;
+static long calls_malloc, calls_free, calls_host_malloc, calls_host_free, calls_large; /* large: of 1 MiB and more */
 
 void fake_fail(const char *name, int after, int count) { /* calls `after` .. after + count - 1 of `name` fail */
     pthread_mutex_lock(&mu);
@@ -49,7 +49,7 @@ size_t fake_live(int dev) { /* bytes allocated on a device (-1: pinned) */
 static int delay_ms;
 void fake_delay_malloc(int ms) { delay_ms = ms; } /* each hipMalloc takes that long */
 long fake_calls(int which) {
-    const long c[] = {calls_malloc, calls_free, calls_host_malloc, calls_host_free};
+    const long c[] = {calls_malloc, calls_free, calls_host_malloc, calls_host_free, calls_large};
     return c[which];
 }
 
@@ -89,6 +89,7 @@ static hipError_t drop(void *p, int host) {
 hipError_t hipMalloc(void **p, size_t bytes) {
     MAY_FAIL;
     __sync_fetch_and_add(&calls_malloc, 1);
+    if (bytes >= 1 << 20) __sync_fetch_and_add(&calls_large, 1);
     if (delay_ms) usleep(1000 * delay_ms);
     return get(p, bytes, device);
 }

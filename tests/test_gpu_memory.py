@@ -28,6 +28,24 @@ def test_copies_of_every_length(n):
     np.testing.assert_array_equal(got, want)
 
 
+@pytest.mark.parametrize("n", [104857, 104858, 300001])
+def test_class_sums_of_every_length(n):
+    """Class sums below 4 MiB come back through one pinned buffer, from there on in pieces."""
+    tm = MultiClassTM(40, 50, 5.0, (100, 1, 1), 10, seed=3)
+    rng = np.random.default_rng(n)
+    L = tm.number_of_literals
+    ta = np.where(rng.random((40, L)) < 3 / L, 200, 60).astype(np.uint32)
+    w = rng.integers(-50, 51, (40, 10)).astype(np.float32)
+    tm.load_state_dict({"state": {"ta_state": ta, "clause_weights": w, "min_y": None, "max_y": None,
+                                  "patch_weights": np.zeros((40, 1), np.int32)}})
+    bits = rng.integers(0, 2, (n, 100), dtype=np.uint8)
+    lits = np.concatenate([bits, 1 - bits], 1).astype(np.float32)
+    miss = (1 - lits) @ (ta > 128).T.astype(np.float32)
+    fire = (miss == 0) & (ta > 128).any(1)
+    np.testing.assert_array_equal(tm.score(tm.encode(bits.astype(np.uint32)), is_X_encoded=True),
+                                  (fire.astype(np.float64) @ w).astype(np.float32))
+
+
 def test_threads_and_reused_blocks():
     """Calls of several threads at once, each with its own results, over blocks that earlier
     calls of other sizes leave behind."""

@@ -47,7 +47,8 @@ def test_every_call_failing(fake_hip, entry):
     child(fake_hip, entry)
 
 
-@pytest.mark.parametrize("what", ["oldest_leave_first", "given_back_with_the_last_model", "allocations_unlocked", "staging_per_device"])
+@pytest.mark.parametrize("what", ["oldest_leave_first", "given_back_with_the_last_model", "allocations_unlocked", "staging_per_device",
+                                  "new_models_first_score"])
 def test_blocks(fake_hip, what):
     child(fake_hip, what)
 
@@ -211,7 +212,7 @@ def small_model(lib, L):
     return m
 
 
-MALLOC, FREE, HOST_MALLOC, HOST_FREE = range(4)
+MALLOC, FREE, HOST_MALLOC, HOST_FREE, LARGE = range(5)
 MB = 1 << 20
 
 
@@ -276,13 +277,37 @@ def staging_per_device(fake, lib, L):
     assert fake.fake_live(-1) == 0 and fake.fake_live(1) == 0
 
 
+def new_models_first_score(fake, lib, L):
+    """While a model lives, another one's first score finds its pinned and its large buffers there."""
+    def score(m, n, bits):
+        X, out = np.zeros((n, 1, (2 * bits + 31) // 32), np.uint32), np.empty((n, 3), np.float32)
+        before = fake.fake_calls(LARGE) + fake.fake_calls(HOST_MALLOC)
+        assert lib.ytm_score(m, X.ctypes.data, n, out.ctypes.data) == 0
+        return fake.fake_calls(LARGE) + fake.fake_calls(HOST_MALLOC) - before
+
+    def model(bits):
+        p = L.YtmParams(clauses=600, classes=3, dim0=bits, dim1=1, dim2=1, patch_dim0=bits, patch_dim1=1,
+                        number_of_ta_states=256, max_included_literals=2 * bits, append_negated=1, encode_loc=1,
+                        coalesced=1, negative_polarity=1, thresh=10, s_inv=0.2, q_prob=1.0, seed=1)
+        m = ctypes.c_void_p()
+        assert lib.ytm_create(ctypes.byref(p), ctypes.byref(m)) == 0
+        return m
+
+    for bits, n in ((784, 1), (784, 10000), (5000, 3), (40, 2000)):
+        first, second = model(bits), model(bits)
+        score(first, n, bits)
+        assert score(second, n, bits) == 0, (bits, n)
+        lib.ytm_destroy(second)
+        lib.ytm_destroy(first)
+
+
 def every_call_failing(name, fake, lib, L):
     prepare, call, free = entry(name, lib, L)
     wrong = []
     for fn in CALLS:
         for after in range(200):
             h = prepare()
-            fake.fake_fail(fn.encode(), after, 2 if fn == "hipMalloc" else 1)  # hipMalloc is tried again
+            fake.fake_fail(fn.encode(), after, 2 if fn in ("hipMalloc", "hipHostMalloc") else 1)  # tried again
             rc = call(h)
             reached = fake.fake_failed()
             fake.fake_fail(b"", -1, 0)

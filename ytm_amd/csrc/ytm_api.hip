@@ -33,14 +33,11 @@ struct ytm_model {
   int* d_err = nullptr;
   unsigned long long* d_slots = nullptr;
   size_t slots_bytes = 0;
-  // Scoring buffers kept between calls (grow-only): class-sum accumulators, float sums,
-  // literal lists.  Calls are synchronous, so a call never reuses a buffer still in use.
-  void* d_sacc = nullptr;
-  void* d_sout = nullptr;
+  // The scorers' model operands or literal lists, kept between calls (grow-only): first behind
+  // d_planes in its block, then in one of their own (slists_own).
   void* d_slists = nullptr;
-  size_t sacc_bytes = 0, sout_bytes = 0, slists_bytes = 0;
-  void* h_sout = nullptr;  // pinned host staging of the class sums (hipHostMalloc)
-  size_t h_sout_bytes = 0;
+  size_t slists_bytes = 0;
+  bool slists_own = false;
   // The state changes with every fit, ytm_set_ta_state and ytm_set_weights (state_version
   // counts them); d_slists holds the one-patch literal lists or the matrix operands
   // (slists_kind) of version slists_version, so that scoring again an unchanged model does
@@ -176,17 +173,6 @@ int resolve_geometry(const ytm_params& p, Geom* out) {
   return YTM_OK;
 }
 
-// A grow-only device buffer: *p holds at least bytes after a successful call.
-hipError_t ensure_buffer(void** p, size_t* have, size_t bytes) {
-  if (*have >= bytes && *p) return hipSuccess;
-  ytm::pool_free(*p);
-  *p = nullptr;
-  *have = 0;
-  const hipError_t e = ytm::pool_alloc(p, bytes);
-  if (e == hipSuccess) *have = bytes;
-  return e;
-}
-
 int ensure_slots(ytm_model* m, size_t bytes) {
   if (m->slots_bytes >= bytes) return YTM_OK;
   ytm::pool_free(m->d_slots);
@@ -252,6 +238,10 @@ int upload(void** dst, const void* src, size_t bytes, hipStream_t s) {
   *dst = nullptr;
   return fail(YTM_EHIP, std::string("copy to the device failed: ") + hipGetErrorString(e));
 }
+
+// Bytes of the operands or lists that scores of the model will mostly need: of samples with
+// complemented negations, as they are encoded, and weights of two digits.
+size_t operand_room(const Geom& g);
 
 // Picks the persistent grid (one workgroup per CU at most, at least ~12 clauses each, and
 // two workgroups for models of more than one clause) and the class-sum grouping (groups of
@@ -545,7 +535,17 @@ int ytm_create(const ytm_params* params, ytm_model** out) {
   CREATE_TRY(hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking));
   CREATE_TRY(hipEventCreate(&m->ev0));
   CREATE_TRY(hipEventCreate(&m->ev1));
-  CREATE_TRY(ytm::pool_alloc((void**)&m->d_planes, (size_t)(g.C * g.np * g.W) * 4));
+  // One block for the planes and, where it is no larger, the room of the scorers' operands: the
+  // first score of a new model then waits for no hipMalloc (2000 clauses of 784 bits, one sample:
+  // 209 us with buffers and a pinned result of the model's own, 157 from the pool and this).
+  const size_t planes_bytes = ((size_t)(g.C * g.np * g.W) * 4 + 255) & ~(size_t)255;
+  size_t operands = operand_room(g);
+  if (operands > planes_bytes) operands = 0;
+  CREATE_TRY(ytm::pool_alloc((void**)&m->d_planes, planes_bytes + operands));
+  if (operands) {
+    m->d_slists = (unsigned char*)m->d_planes + planes_bytes;
+    m->slists_bytes = operands;
+  }
   CREATE_TRY(ytm::pool_alloc((void**)&m->d_w, (size_t)(g.C * g.K) * 4));
   CREATE_TRY(ytm::pool_alloc((void**)&m->d_pw, (size_t)(g.C * g.P) * 4));
   CREATE_TRY(ytm::pool_alloc((void**)&m->d_bias, (size_t)g.K * 4));
@@ -570,10 +570,9 @@ void ytm_destroy(ytm_model* m) {
   if (!m) return;
   if (m->stream) (void)settle(m->stream);
   void* bufs[] = {m->d_planes, m->d_w,    m->d_pw,   m->d_bias, m->d_ninc,  m->d_inv_rank,
-                  m->d_counters, m->d_err, m->d_slots, m->d_sacc, m->d_sout, m->d_slists};
+                  m->d_counters, m->d_err, m->d_slots, m->slists_own ? m->d_slists : nullptr};
   for (void* b : bufs)
     ytm::pool_free(b);
-  if (m->h_sout) (void)hipHostFree(m->h_sout);
   if (m->ev0) (void)hipEventDestroy(m->ev0);
   if (m->ev1) (void)hipEventDestroy(m->ev1);
   if (m->stream) (void)hipStreamDestroy(m->stream);
@@ -1106,6 +1105,11 @@ ScorePlan list_plan(const Geom& g, bool has_xt) {
   return p;
 }
 
+size_t operand_room(const Geom& g) {
+  const ytm::MatrixPlan mm = ytm::matrix_plan(g, g.P == 1 ? -1 : 1, 32639.0, (int64_t)1 << 31);
+  return mm.steps ? mm.bytes : list_plan(g, ytm::literal_major(g)).lists_bytes;
+}
+
 ScorePlan score_plan(ytm_model* m, const ytm_dataset* ds) {
   ScorePlan p{};
   // One patch: where the product over all literals is long, the samples are looked at first, so
@@ -1139,11 +1143,9 @@ hipError_t score_samples(ytm_model* m, const ScorePlan& plan, const uint32_t* X,
                          long long* acc, void* lists, float* out, bool lists_ready = false) {
   const Geom& g = m->g;
   hipError_t e = hipSuccess;
-  if (plan.mm.steps) {
-    if (!lists_ready) e = ytm::launch_matrix_pack(m->d_planes, m->d_w, g, plan.mm, lists, m->stream);
-    if (e != hipSuccess) return e;
-    return ytm::launch_matrix_score(X, N, g, plan.mm, lists, m->cus, m->d_bias, (uint32_t*)acc, out, m->stream);
-  }
+  if (plan.mm.steps)
+    return ytm::launch_matrix_score(m->d_planes, m->d_w, lists_ready, X, N, g, plan.mm, lists, m->cus, m->d_bias,
+                                    (uint32_t*)acc, out, m->stream);
   if (!plan.chunks) e = ytm::launch_fill_u64((unsigned long long*)acc, N * g.K, m->stream);
   if (e != hipSuccess) return e;
   if (plan.wide)
@@ -1158,6 +1160,8 @@ hipError_t score_samples(ytm_model* m, const ScorePlan& plan, const uint32_t* X,
   return plan.chunks ? ytm::launch_score_parts_finish(acc, plan.chunks, m->d_bias, N, g, out, m->stream)
                      : ytm::launch_score_finish(acc, m->d_bias, N, g, out, m->stream);
 }
+
+constexpr size_t kPinnedSums = (size_t)4 << 20;  // class sums below go through a pinned buffer
 
 // ---- Scratch of the allocation-free scoring entry point: one static device array per GPU
 // (each device that runs it holds its own copy, at its own address, until the process
@@ -1202,46 +1206,55 @@ int ytm_score_dataset(ytm_model* m, const ytm_dataset* ds, float* class_sums) {
   if (N == 0) return YTM_OK;
   const ScorePlan plan = score_plan(m, ds);
   const int64_t per_pass = std::max<int64_t>(score_pass(plan, N, (size_t)256 << 20), std::min<int64_t>(N, 1024));
-  hipError_t e = ensure_buffer(&m->d_sacc, &m->sacc_bytes, pass_bytes(plan, per_pass));
-  if (e == hipSuccess) e = ensure_buffer(&m->d_sout, &m->sout_bytes, (size_t)(N * g.K) * 4);
-  const void* lists_before = m->d_slists;
-  if (e == hipSuccess && plan.lists_bytes) e = ensure_buffer(&m->d_slists, &m->slists_bytes, plan.lists_bytes);
-  if (m->d_slists != lists_before) m->slists_version = ~0ull;
+  // The rows and the sums come from the pool, where a new model finds an earlier one's.
+  void *acc = nullptr, *sums = nullptr, *pinned = nullptr;
+  const size_t out_bytes = (size_t)(N * g.K) * 4;
+  hipError_t e = ytm::pool_alloc(&acc, pass_bytes(plan, per_pass));
+  if (e == hipSuccess) e = ytm::pool_alloc(&sums, out_bytes);
+  if (e == hipSuccess && plan.lists_bytes > m->slists_bytes) {
+    m->slists_version = ~0ull;
+    if (m->slists_own) ytm::pool_free(m->d_slists);
+    m->d_slists = nullptr;
+    m->slists_bytes = 0;
+    m->slists_own = true;
+    e = ytm::pool_alloc(&m->d_slists, plan.lists_bytes);
+    if (e == hipSuccess) m->slists_bytes = plan.lists_bytes;
+  }
   // operands that depend on the model alone are kept from the last call
   bool lists_ready = plan.kept() && m->slists_kind == plan.kept() && m->slists_version == m->state_version;
-  float* dout = (float*)m->d_sout;
+  float* dout = (float*)sums;
   // the include counts, for the scorers that read them (the list-based ones count their lists)
   if (e == hipSuccess && !plan.lists_bytes) e = ytm::launch_ninc(m->d_planes, m->d_ninc, g, m->stream);
   if (e == hipSuccess) e = hipEventRecord(m->ev0, m->stream);
   for (int64_t first = 0; e == hipSuccess && first < N; first += per_pass) {
     // more than one pass only without a literal-major copy (score_pass)
-    e = score_samples(m, plan, ds->d_X + first * g.P * g.W, ds->d_XT, std::min(per_pass, N - first),
-                      (long long*)m->d_sacc, plan.lists_bytes ? m->d_slists : nullptr, dout + first * g.K, lists_ready);
+    e = score_samples(m, plan, ds->d_X + first * g.P * g.W, ds->d_XT, std::min(per_pass, N - first), (long long*)acc,
+                      plan.lists_bytes ? m->d_slists : nullptr, dout + first * g.K, lists_ready);
     lists_ready = plan.kept() != 0;
   }
   m->slists_version = e == hipSuccess && plan.kept() ? m->state_version : ~0ull;
   m->slists_kind = plan.kept();
   if (e == hipSuccess) e = hipEventRecord(m->ev1, m->stream);
-  // the sums come back through a pinned staging buffer of the model (a direct copy into
-  // pageable memory goes through the runtime's own staging, in smaller pieces)
-  const size_t out_bytes = (size_t)(N * g.K) * 4;
-  if (e == hipSuccess && m->h_sout_bytes < out_bytes) {
-    if (m->h_sout) (void)hipHostFree(m->h_sout);
-    m->h_sout = nullptr;
-    m->h_sout_bytes = 0;
-    e = hipHostMalloc(&m->h_sout, out_bytes, hipHostMallocDefault);
-    if (e == hipSuccess) m->h_sout_bytes = out_bytes;
+  // the sums come back through a pinned buffer (a direct copy into pageable memory goes through
+  // the runtime's own staging, in smaller pieces), large ones through copy_to_host's
+  if (e == hipSuccess && out_bytes < kPinnedSums) e = ytm::pinned_alloc(&pinned, out_bytes);
+  if (e == hipSuccess && pinned) {
+    e = hipMemcpyAsync(pinned, sums, out_bytes, hipMemcpyDeviceToHost, m->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(m->stream);
+    if (e == hipSuccess) std::memcpy(class_sums, pinned, out_bytes);
+  } else if (e == hipSuccess) {
+    e = ytm::copy_to_host(class_sums, sums, out_bytes, m->stream);
   }
-  if (e == hipSuccess) e = hipMemcpyAsync(m->h_sout, dout, out_bytes, hipMemcpyDeviceToHost, m->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(m->stream);
-  if (e == hipSuccess) std::memcpy(class_sums, m->h_sout, out_bytes);
   float ms = 0.0f;
   if (e == hipSuccess) e = hipEventElapsedTime(&ms, m->ev0, m->ev1);
   if (e != hipSuccess) {
     m->slists_version = ~0ull;
     (void)settle(m->stream);  // before the samples and the buffers are used again
-    return fail(YTM_EHIP, std::string("score failed: ") + hipGetErrorString(e));
   }
+  ytm::pool_free(acc);
+  ytm::pool_free(sums);
+  ytm::pinned_free(pinned);
+  if (e != hipSuccess) return fail(YTM_EHIP, std::string("score failed: ") + hipGetErrorString(e));
   m->stats.last_score_kernel_ms = ms;
   return YTM_OK;
 }

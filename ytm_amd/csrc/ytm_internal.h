@@ -15,6 +15,9 @@ namespace ytm {
 // whatever they held before; a block is freed once nothing on the GPU uses it any more.
 hipError_t pool_alloc(void** p, size_t bytes);
 void pool_free(void* p);
+// The same for pinned host memory.
+hipError_t pinned_alloc(void** p, size_t bytes);
+void pinned_free(void* p);
 // A model that lives on a device (false: nothing is kept for it) and its end: the device's blocks
 // are kept while one does.
 bool memory_hold(int device);
@@ -80,8 +83,6 @@ struct MatrixPlan {
 // halves: the N samples' negated literals are the complements of the positive ones (1), are not
 // (0), or may be (-1, one patch); w_bound: an upper bound of |weight|.
 MatrixPlan matrix_plan(const Geom& g, int halves, double w_bound, int64_t N);
-hipError_t launch_matrix_pack(const uint32_t* planes, const float* w, const Geom& g, const MatrixPlan& p,
-                              void* scratch, hipStream_t s);
 // One patch: N samples are so few that a block per product tile takes them.
 bool few_rows(const Geom& g, int64_t N);
 // One patch: the product of N samples over all literals takes 70 us or more, twice that over the
@@ -89,8 +90,11 @@ bool few_rows(const Geom& g, int64_t N);
 bool long_rows(const Geom& g, int64_t N);
 size_t matrix_rows_bytes(const MatrixPlan& p, int64_t N);
 // Class sums of N samples (encoded words X) into out (float [N][K]); masks: matrix_rows_bytes.
-hipError_t launch_matrix_score(const uint32_t* X, int64_t N, const Geom& g, const MatrixPlan& p, void* scratch,
-                               int cus, const float* bias, uint32_t* masks, float* out, hipStream_t s);
+// ready: the scratch holds the operands of these planes and weights, which are made first
+// otherwise.
+hipError_t launch_matrix_score(const uint32_t* planes, const float* w, bool ready, const uint32_t* X, int64_t N,
+                               const Geom& g, const MatrixPlan& p, void* scratch, int cus, const float* bias,
+                               uint32_t* masks, float* out, hipStream_t s);
 // Clears *ok unless every negated literal of the N samples' encoded rows is the complement of
 // its positive one (ok set before; models with appended negations).
 hipError_t launch_halves_check(const uint32_t* X, int64_t N, const Geom& g, int* ok, hipStream_t s);

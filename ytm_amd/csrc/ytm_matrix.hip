@@ -42,15 +42,46 @@ __device__ __forceinline__ bool complements(const uint32_t* x, const Geom& g, in
   return (bits_at(x, g.W, 0, g.Lh, j) ^ bits_at(x, g.W, g.Lh, g.Lh, j)) == valid;
 }
 
+// Weight operands wfrag[word of 32 clauses][column group][lane], lane l holding 16 int8 values
+// (clauses 32 word + 16 (l / 32) ...) of column l % 32: digit col % D of class group * (32 / D) +
+// col / D, the weights in signed base-256 digits, least significant first.  By block `first` of
+// `blocks`.
+__device__ __forceinline__ void pack_weights(const float* __restrict__ w, const Geom& g, const MatrixPlan& p, v4i* wfrag,
+                                             int64_t first, int64_t blocks) {
+  const int per = kTile / p.digits;
+  for (int64_t idx = first * (int64_t)blockDim.x + threadIdx.x; idx < p.row_words * p.groups * kWave;
+       idx += blocks * (int64_t)blockDim.x) {
+    const int l = (int)(idx % kWave), grp = (int)(idx / kWave % p.groups);
+    const int64_t c0 = idx / kWave / p.groups * kTile + 16 * (l >> 5);
+    const int col = l & 31, k = grp * per + col / p.digits, digit = col % p.digits;
+    v4i r;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      uint32_t word = 0u;
+#pragma unroll
+      for (int b = 0; b < 4; ++b) {
+        const int64_t c = c0 + 4 * q + b;
+        long long v = c < g.C && col / p.digits < per && k < g.K ? (long long)w[c * g.K + k] : 0;
+        int d = 0;
+        for (int i = 0; i <= digit; ++i) {
+          d = (int)(signed char)(v & 255);
+          v = (v - d) >> 8;
+        }
+        word |= (uint32_t)(d & 255) << (8 * b);
+      }
+      r[q] = (int)word;
+    }
+    wfrag[idx] = r;
+  }
+}
+
 // The model's operands, three independent parts of one launch (after every change of the model
 // and before its first score: 784 bits, 2000 clauses 15.6 us in a launch each, 9.2 us in one):
 //  - clause operands frag[tile of 32 clauses][step][lane], lane l holding 32 values (literals
 //    64 step + 32 (l / 32) ...) of clause 32 tile + l % 32; zero past the last clause or literal;
 //  - thresholds need[32 tiles]: the value a clause's product reaches where it fires, plus the
 //    1 that the products start from; a wave per clause;
-//  - weight operands wfrag[word of 32 clauses][column group][lane], lane l holding 16 int8
-//    values (clauses 32 word + 16 (l / 32) ...) of column l % 32: digit col % D of class
-//    group * (32 / D) + col / D, the weights in signed base-256 digits, least significant first.
+//  - weight operands (pack_weights).
 // With half_steps, operands and thresholds over the positive literals alone come besides.
 __global__ __launch_bounds__(256) void pack_model_kernel(const uint32_t* __restrict__ planes,
                                                          const float* __restrict__ w, Geom g, MatrixPlan p,
@@ -88,31 +119,7 @@ __global__ __launch_bounds__(256) void pack_model_kernel(const uint32_t* __restr
   }
   int64_t first = blockIdx.x - need_blocks;
   if (first < weight_blocks) {
-    const int per = kTile / p.digits;
-    for (int64_t idx = first * (int64_t)blockDim.x + threadIdx.x; idx < p.row_words * p.groups * kWave;
-         idx += weight_blocks * (int64_t)blockDim.x) {
-      const int l = (int)(idx % kWave), grp = (int)(idx / kWave % p.groups);
-      const int64_t c0 = idx / kWave / p.groups * kTile + 16 * (l >> 5);
-      const int col = l & 31, k = grp * per + col / p.digits, digit = col % p.digits;
-      v4i r;
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        uint32_t word = 0u;
-#pragma unroll
-        for (int b = 0; b < 4; ++b) {
-          const int64_t c = c0 + 4 * q + b;
-          long long v = c < g.C && col / p.digits < per && k < g.K ? (long long)w[c * g.K + k] : 0;
-          int d = 0;
-          for (int i = 0; i <= digit; ++i) {
-            d = (int)(signed char)(v & 255);
-            v = (v - d) >> 8;
-          }
-          word |= (uint32_t)(d & 255) << (8 * b);
-        }
-        r[q] = (int)word;
-      }
-      wfrag[idx] = r;
-    }
+    pack_weights(w, g, p, wfrag, first, weight_blocks);
     return;
   }
   first -= weight_blocks;
@@ -449,21 +456,39 @@ __global__ __launch_bounds__(512) void fire_rows_kernel(const v4i* __restrict__ 
 // The same for few samples: a block per product tile, its four waves sharing the steps, the
 // operands read straight from global memory (the samples' from their encoded words) and the
 // partial sums put together in LDS.
+// PACK: the first score of a changed model, up to 32 samples (one tile), over all literals: the
+// operands are made from the include masks here and kept, the weights' by the blocks past the
+// tiles, so that nothing reads them back and there is a launch less (20000 literals, 10000
+// clauses, one sample: 43 us of pack_model_kernel, 27 here and 7 of votes, 68 us with their gaps,
+// against 55 so; 784 bits, 2000 clauses: the call 51 -> 47 us).
+template <bool PACK>
 __global__ __launch_bounds__(256) void fire_few_kernel(const uint32_t* __restrict__ X, int64_t N, Geom g,
-                                                       const v4i* __restrict__ cfrag, const float* __restrict__ need,
-                                                       int steps, int64_t row_words, uint32_t* __restrict__ masks) {
+                                                       const uint32_t* __restrict__ planes,
+                                                       const float* __restrict__ w, unsigned char* __restrict__ base,
+                                                       MatrixPlan p, uint32_t* __restrict__ masks) {
   __shared__ float s_d[3][16][kWave];
+  __shared__ int s_count[4][kWave];
+  const int steps = p.steps;
+  const int64_t row_words = p.row_words;
+  v4i* cfrag = (v4i*)base;
+  float* need = (float*)(base + p.need_at);
   const int lane = lane_id(), wave = threadIdx.x / kWave;
   const int64_t mtiles = (N + kTile - 1) / kTile, ctiles = (g.C + kTile - 1) / kTile;
   const int64_t mt = blockIdx.x % mtiles, ct = blockIdx.x / mtiles;
-  if (ct >= ctiles) return;
+  if (ct >= ctiles) {
+    if (PACK) pack_weights(w, g, p, (v4i*)(base + p.weights_at), blockIdx.x - ctiles, gridDim.x - ctiles);
+    return;
+  }
   const int64_t e = mt * kTile + (lane & 31) < N ? mt * kTile + (lane & 31) : N - 1;
   const uint32_t* x = X + e * g.W;
-  const v4i* cf = cfrag + ct * steps * kWave + lane;
+  v4i* cf = cfrag + ct * steps * kWave + lane;
   v16f d;
 #pragma unroll
   for (int r = 0; r < 16; ++r) d[r] = wave == 0 ? 1.0f : 0.0f;
-  const float want = need[ct * kTile + (lane & 31)];
+  const int64_t c = ct * kTile + (lane & 31);
+  const uint32_t* m = planes + ((c < g.C ? c : g.C - 1) * g.np + g.np - 1) * g.W;
+  int count = 0;  // PACK: the lane's share of its clause's included literals
+  float want = PACK ? 0.0f : need[c];
   constexpr int kAhead = 4;  // operands in flight
   for (int s0 = wave; s0 < steps; s0 += 4 * kAhead) {
     uint32_t xw[kAhead];
@@ -473,13 +498,22 @@ __global__ __launch_bounds__(256) void fire_few_kernel(const uint32_t* __restric
       const int st = s0 + 4 * q < steps ? s0 + 4 * q : steps - 1;  // clamped: every load unconditional
       const int64_t w = 2 * st + (lane >> 5);
       xw[q] = x[w < g.W ? w : g.W - 1];  // past the words the clause operand is 0
-      bv[q] = cf[st * kWave];
+      if (PACK) {
+        const uint32_t on = c < g.C && s0 + 4 * q < steps && w < g.W ? m[w] : 0u;
+        count += __popc(on);
+        bv[q] = fp4_column(on, 0u);
+      } else {
+        bv[q] = cf[st * kWave];
+      }
     }
 #pragma unroll
     for (int q = 0; q < kAhead; ++q)
-      if (s0 + 4 * q < steps)
+      if (s0 + 4 * q < steps) {
         d = fp4_product(fp4_row(xw[q]), bv[q], d);
+        if (PACK) cf[(s0 + 4 * q) * kWave] = bv[q];
+      }
   }
+  if (PACK) s_count[wave][lane] = count;
   if (wave > 0)
 #pragma unroll
     for (int r = 0; r < 16; ++r) s_d[wave - 1][r][lane] = d[r];
@@ -487,6 +521,13 @@ __global__ __launch_bounds__(256) void fire_few_kernel(const uint32_t* __restric
   if (wave > 0) return;
 #pragma unroll
   for (int r = 0; r < 16; ++r) d[r] += s_d[0][r][lane] + s_d[1][r][lane] + s_d[2][r][lane];
+  if (PACK) {  // the threshold as pack_model_kernel makes it
+    int n = 0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) n += s_count[q][lane] + s_count[q][lane ^ 32];
+    want = n ? (float)(n + 1) : kNever;
+    if (lane < kTile) need[c] = want;
+  }
   const uint32_t word = row_words_of(d, want);
   if (lane < kTile && mt * kTile + lane < N) masks[(mt * kTile + lane) * row_words + ct] = word;
 }
@@ -665,19 +706,9 @@ MatrixPlan matrix_plan(const Geom& g, int halves, double w_bound, int64_t N) {
   return p;
 }
 
-hipError_t launch_matrix_pack(const uint32_t* planes, const float* w, const Geom& g, const MatrixPlan& p,
-                              void* scratch, hipStream_t s) {
-  unsigned char* base = (unsigned char*)scratch;
-  const int64_t tiles = clause_tiles(g);
-  const int need_blocks = blocks_for(tiles * kTile * kWave, 256);
-  const int weight_blocks = blocks_for(p.row_words * p.groups * kWave, 256);
-  pack_model_kernel<<<need_blocks + weight_blocks + blocks_for(tiles * (p.steps + p.half_steps) * kWave, 256), 256, 0,
-                      s>>>(planes, w, g, p, base, need_blocks, weight_blocks);
-  return hipGetLastError();
-}
-
-hipError_t launch_matrix_score(const uint32_t* X, int64_t N, const Geom& g, const MatrixPlan& p, void* scratch,
-                               int cus, const float* bias, uint32_t* masks, float* out, hipStream_t s) {
+hipError_t launch_matrix_score(const uint32_t* planes, const float* w, bool ready, const uint32_t* X, int64_t N,
+                               const Geom& g, const MatrixPlan& p, void* scratch, int cus, const float* bias,
+                               uint32_t* masks, float* out, hipStream_t s) {
   if (N == 0) return hipSuccess;
   unsigned char* base = (unsigned char*)scratch;
   int* flag = (int*)(base + p.flag_at);
@@ -685,8 +716,20 @@ hipError_t launch_matrix_score(const uint32_t* X, int64_t N, const Geom& g, cons
   const float* need = (const float*)(base + p.need_at);
   hipError_t e = hipSuccess;
   const int64_t mtiles = (N + kTile - 1) / kTile, ctiles = clause_tiles(g);
-  if (g.P == 1 && few_rows(g, N)) {
-    fire_few_kernel<<<(unsigned)(mtiles * ctiles), 256, 0, s>>>(X, N, g, frag, need, p.steps, p.row_words, masks);
+  const bool few = g.P == 1 && few_rows(g, N), pack_few = few && !ready && mtiles == 1 && !p.half_steps && !p.ternary;
+  const int weight_blocks = blocks_for(p.row_words * p.groups * kWave, 256);
+  if (!ready && !pack_few) {
+    const int need_blocks = blocks_for(ctiles * kTile * kWave, 256);
+    pack_model_kernel<<<need_blocks + weight_blocks + blocks_for(ctiles * (p.steps + p.half_steps) * kWave, 256), 256, 0,
+                        s>>>(planes, w, g, p, base, need_blocks, weight_blocks);
+    e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  if (pack_few) {
+    fire_few_kernel<true><<<(unsigned)ctiles + weight_blocks, 256, 0, s>>>(X, N, g, planes, w, base, p, masks);
+    e = hipGetLastError();
+  } else if (few) {
+    fire_few_kernel<false><<<(unsigned)(mtiles * ctiles), 256, 0, s>>>(X, N, g, planes, w, base, p, masks);
     e = hipGetLastError();
   } else if (g.P == 1) {
     v4i* sfrag = (v4i*)((unsigned char*)masks + rows_room(p, N));

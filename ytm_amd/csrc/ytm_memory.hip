@@ -6,7 +6,9 @@
 // small one that finds the runtime's own chunk of small blocks gone; blocks are therefore kept
 // here when a call is done with them, while a model lives on their device: up to kKeep bytes a
 // device, the longest unused given back first.  All are given back with the device's last
-// model, by memory_trim (ytm_shutdown), and when an allocation fails.
+// model, by memory_trim (ytm_shutdown), and when an allocation fails.  Pinned host blocks (a
+// hipHostMalloc takes 50 to 110 us, as long as scoring one sample) are kept alike, while any
+// model lives.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -28,7 +30,9 @@ namespace {
 constexpr size_t kSmall = (size_t)1 << 20;  // below: powers of two
 constexpr size_t kUnit = (size_t)2 << 20;   // from there on: whole units
 constexpr size_t kKeep = (size_t)1 << 30;   // idle bytes kept per device
+constexpr size_t kKeepPinned = (size_t)64 << 20;
 constexpr int kDevices = 64;                // devices whose blocks are kept
+constexpr int kHost = -1;                   // in a device's place: pinned host memory
 
 struct Block {
   int device;
@@ -41,13 +45,13 @@ struct Idle {
 struct Pool {
   std::multimap<size_t, Idle> idle;  // by size
   size_t idle_bytes = 0;
-  int models = 0;  // living on the device
+  int models = 0;  // living on the device (kHost: on any)
 };
 
 // Held for the books alone: the runtime's own calls, which may take long, are made outside.
 std::mutex g_mu;
 std::unordered_map<void*, Block> g_blocks;  // every block handed out or idle
-std::map<int, Pool> g_pools;                // by device
+std::map<int, Pool> g_pools;                // by device, and kHost
 uint64_t g_given_back = 0;
 
 // Takes the longest idle block of a device out of the books while more than `keep` bytes are
@@ -67,22 +71,23 @@ void* take_oldest(int device, size_t keep) {
   return p;
 }
 
+hipError_t take(int device, void** p, size_t bytes) {
+  return device == kHost ? hipHostMalloc(p, bytes, hipHostMallocDefault) : hipMalloc(p, bytes);
+}
+void give(int device, void* p) { (void)(device == kHost ? hipHostFree(p) : hipFree(p)); }
+
 void trim_device(int device, size_t keep) {
-  while (void* p = take_oldest(device, keep)) (void)hipFree(p);
+  while (void* p = take_oldest(device, keep)) give(device, p);
 }
 
-}  // namespace
-
-hipError_t pool_alloc(void** p, size_t bytes) {
+// A block of at least `bytes`, idle or new.
+hipError_t alloc_block(int device, void** p, size_t bytes) {
   *p = nullptr;
   size_t want = 256;
   if (bytes < kSmall)
     while (want < bytes) want *= 2;
   else
     want = (bytes + kUnit - 1) / kUnit * kUnit;
-  int device = 0;
-  hipError_t e = hipGetDevice(&device);
-  if (e != hipSuccess) return e;
   {
     std::lock_guard<std::mutex> lock(g_mu);
     const auto pool = g_pools.find(device);
@@ -97,11 +102,11 @@ hipError_t pool_alloc(void** p, size_t bytes) {
       }
     }
   }
-  e = hipMalloc(p, want);
+  hipError_t e = take(device, p, want);
   if (e != hipSuccess) {
     (void)hipGetLastError();
     trim_device(device, 0);
-    e = hipMalloc(p, want);
+    e = take(device, p, want);
   }
   if (e != hipSuccess) return e;
   std::lock_guard<std::mutex> lock(g_mu);
@@ -112,9 +117,10 @@ hipError_t pool_alloc(void** p, size_t bytes) {
   return e;
 }
 
-void pool_free(void* p) {
+void free_block(bool pinned, void* p) {
   if (!p) return;
-  int device = -1;
+  int device = kHost;
+  const size_t keep = pinned ? kKeepPinned : kKeep;
   bool kept = false;
   {
     std::lock_guard<std::mutex> lock(g_mu);
@@ -123,7 +129,7 @@ void pool_free(void* p) {
       const Block b = it->second;
       device = b.device;
       const auto pool = g_pools.find(device);
-      if (pool != g_pools.end() && pool->second.models > 0 && b.bytes <= kKeep) try {
+      if (pool != g_pools.end() && pool->second.models > 0 && b.bytes <= keep) try {
           pool->second.idle.emplace(b.bytes, Idle{p, g_given_back++});
           pool->second.idle_bytes += b.bytes;
           kept = true;
@@ -133,16 +139,31 @@ void pool_free(void* p) {
     }
   }
   if (!kept)
-    (void)hipFree(p);
+    give(pinned ? kHost : 0, p);
   else
-    trim_device(device, kKeep);
+    trim_device(device, keep);
 }
+
+}  // namespace
+
+hipError_t pool_alloc(void** p, size_t bytes) {
+  *p = nullptr;
+  int device = 0;
+  const hipError_t e = hipGetDevice(&device);
+  return e == hipSuccess ? alloc_block(device, p, bytes) : e;
+}
+void pool_free(void* p) { free_block(false, p); }
+
+hipError_t pinned_alloc(void** p, size_t bytes) { return alloc_block(kHost, p, bytes); }
+void pinned_free(void* p) { free_block(true, p); }
 
 bool memory_hold(int device) {
   if (device < 0 || device >= kDevices) return false;
   std::lock_guard<std::mutex> lock(g_mu);
   try {
-    ++g_pools[device].models;
+    Pool &own = g_pools[device], &host = g_pools[kHost];  // both, or neither
+    ++own.models;
+    ++host.models;
   } catch (...) {
     return false;
   }
@@ -263,13 +284,18 @@ hipError_t copy_to_host(void* dst, const void* src, size_t bytes, hipStream_t s)
 }
 
 void memory_release(int device) {
+  bool last = false, last_of_all = false;
   {
     std::lock_guard<std::mutex> lock(g_mu);
-    const auto pool = g_pools.find(device);
-    if (pool == g_pools.end() || --pool->second.models > 0) return;
+    const auto own = g_pools.find(device), host = g_pools.find(kHost);
+    last = own != g_pools.end() && --own->second.models == 0;
+    last_of_all = host != g_pools.end() && --host->second.models == 0;
   }
-  trim_device(device, 0);
-  trim_staging(device);
+  if (last) {
+    trim_device(device, 0);
+    trim_staging(device);
+  }
+  if (last_of_all) trim_device(kHost, 0);
 }
 
 void memory_trim() {
@@ -277,6 +303,7 @@ void memory_trim() {
     trim_device(device, 0);
     trim_staging(device);
   }
+  trim_device(kHost, 0);
 }
 
 }  // namespace ytm
