@@ -38,7 +38,7 @@ def child(fake, what):
 
 
 ENTRIES = ["create", "encode", "encode_binarized", "dataset", "dataset_targets", "fit", "fit_inject", "fit_banks",
-           "fit_patches", "score", "score_again", "score_few", "score_patches", "score_lists", "noalloc",
+           "fit_patches", "score", "score_long", "score_again", "score_few", "score_patches", "score_lists", "noalloc",
            "noalloc_patches", "transform", "transform_patches", "get_state", "set_state", "binarize", "collapse"]
 
 
@@ -112,6 +112,7 @@ def entry(name, lib, L):
 
     flat, patches = model(), model(dim=(8, 8, 1), patch=(3, 3))
     wide = model(clauses=400, dim=(800, 1, 1))
+    long = model(clauses=4000, dim=(4000, 1, 1))  # the samples are looked at before their first score
     lists = model(dim=(8, 8, 80), patch=(3, 3))  # more literals than the product takes
 
     def created(h):
@@ -182,6 +183,7 @@ def entry(name, lib, L):
         "fit_banks": lambda: with_model(banks, lambda m: fit(m, banks)),
         "fit_patches": lambda: with_model(patches, lambda m: fit(m, patches)),
         "score": lambda: with_data(wide, 20000, lambda m, d: score(m, d, 20000)),
+        "score_long": lambda: with_data(long, 10000, lambda m, d: score(m, d, 10000)),
         "score_again": lambda: with_data(wide, 3, lambda m, d: score(m, d, 3), first=lambda m, d: score(m, d, 3)),
         "score_few": lambda: with_data(wide, 3, lambda m, d: score(m, d, 3)),
         "score_patches": lambda: with_data(patches, 9, lambda m, d: score(m, d, 9)),

@@ -68,7 +68,7 @@ struct ytm_dataset {
   uint32_t* d_XT;  // [N][L][ceil(P/32)] literal-major copy (several patches, where a kernel reads it), or null
   // every sample's literals Lh..L-1 are the complements of 0..Lh-1 (1), not (0), or not known
   // (-1, one patch until a score asks)
-  int halves;
+  mutable int halves;
   uint32_t* d_order;  // [kOrderBuckets][W] literal order of the training lists (with d_XT), or null
 };
 
@@ -751,15 +751,20 @@ int ytm_encode_binarized(ytm_model* m, const void* X, int x_dtype, int64_t N, co
 namespace {
 // Sets ds->halves.  Encoded samples hold the negations as complements (BaseTM.encode); samples
 // encoded elsewhere may not, so training and scoring rely on it only where this check holds.
-int check_halves(ytm_model* m, ytm_dataset* ds) {
-  ds->halves = 0;
-  if (!m->g.append_negated || ds->N == 0) return YTM_OK;
+int check_halves(ytm_model* m, const ytm_dataset* ds) {
+  if (!m->g.append_negated || ds->N == 0) {
+    ds->halves = 0;
+    return YTM_OK;
+  }
   int ok = 1;
   hipError_t e = hipMemcpyAsync(m->d_err, &ok, sizeof(int), hipMemcpyHostToDevice, m->stream);
   if (e == hipSuccess) e = ytm::launch_halves_check(ds->d_X, ds->N, m->g, m->d_err, m->stream);
   if (e == hipSuccess) e = hipMemcpyAsync(&ok, m->d_err, sizeof(int), hipMemcpyDeviceToHost, m->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(m->stream);
-  if (e != hipSuccess) return fail(YTM_EHIP, std::string("sample check: ") + hipGetErrorString(e));
+  if (e != hipSuccess) {  // still not known
+    (void)settle(m->stream);
+    return fail(YTM_EHIP, std::string("sample check: ") + hipGetErrorString(e));
+  }
   ds->halves = ok == 1;
   return YTM_OK;
 }
@@ -1110,17 +1115,22 @@ size_t operand_room(const Geom& g) {
   return mm.steps ? mm.bytes : list_plan(g, ytm::literal_major(g)).lists_bytes;
 }
 
-ScorePlan score_plan(ytm_model* m, const ytm_dataset* ds) {
+int score_plan(ytm_model* m, const ytm_dataset* ds, ScorePlan* out) {
   ScorePlan p{};
   // One patch: where the product over all literals is long, the samples are looked at first, so
   // that only the operands of the product that will do are made (20000 literals, 10000 clauses
   // and samples: 250 us less product, against 30 us for the round trip).
-  if (ds->halves < 0 && ytm::long_rows(m->g, ds->N)) (void)check_halves(m, const_cast<ytm_dataset*>(ds));
+  if (ds->halves < 0 && ytm::long_rows(m->g, ds->N))
+    if (int rc = check_halves(m, ds)) return rc;
   p.mm = ytm::matrix_plan(m->g, ds->halves, m->w_bound, ds->N);
-  if (!p.mm.steps) return list_plan(m->g, ds->d_XT != nullptr);
-  p.lists_bytes = p.mm.bytes;
-  p.acc_per_sample = (size_t)p.mm.row_words * 4 + p.mm.sample_bytes;
-  return p;
+  if (p.mm.steps) {
+    p.lists_bytes = p.mm.bytes;
+    p.acc_per_sample = (size_t)p.mm.row_words * 4 + p.mm.sample_bytes;
+  } else {
+    p = list_plan(m->g, ds->d_XT != nullptr);
+  }
+  *out = p;
+  return YTM_OK;
 }
 
 // Samples per pass that keep a pass's buffer within `room` bytes (0: not one), all of them
@@ -1204,7 +1214,8 @@ int ytm_score_dataset(ytm_model* m, const ytm_dataset* ds, float* class_sums) {
   const Geom& g = m->g;
   const int64_t N = ds->N;
   if (N == 0) return YTM_OK;
-  const ScorePlan plan = score_plan(m, ds);
+  ScorePlan plan{};
+  if (int rc = score_plan(m, ds, &plan)) return rc;
   const int64_t per_pass = std::max<int64_t>(score_pass(plan, N, (size_t)256 << 20), std::min<int64_t>(N, 1024));
   // The rows and the sums come from the pool, where a new model finds an earlier one's.
   void *acc = nullptr, *sums = nullptr, *pinned = nullptr;
@@ -1272,7 +1283,8 @@ int ytm_score_dataset_noalloc(ytm_model* m, const ytm_dataset* ds, float* d_clas
     return fail(YTM_EINVAL, "model too large for the allocation-free scorer: it needs " +
                                 std::to_string(room(listed) + listed.acc_per_sample) + " bytes of scratch for one sample, " +
                                 "the scratch holds " + std::to_string(kNoAllocScratchBytes));
-  ScorePlan plan = score_plan(m, ds);
+  ScorePlan plan{};
+  if (int rc = score_plan(m, ds, &plan)) return rc;
   if (plan.mm.steps && (room(plan) >= kNoAllocScratchBytes || !score_pass(plan, N, kNoAllocScratchBytes - room(plan))))
     plan = list_plan(g, ds->d_XT != nullptr);
   const size_t lists_room = room(plan);
