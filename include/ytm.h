@@ -108,7 +108,11 @@ typedef struct ytm_stats {
                                     stops (streaming kernel); the sample count for the others */
     int32_t last_fit_stream;     /* 1 when the last fit ran the streaming kernel (train_kind
                                     is then 3) */
-    int32_t reserved;
+    int16_t train_product;       /* 1 when the last fit evaluated its clauses on the matrix cores
+                                    (train_kind 2) */
+    int16_t score_path;          /* scorer of the last score: 0 none yet, 1 a class sum per sample and
+                                    clause, 2 register tiles (one patch), 3 literal lists (one
+                                    patch), 4 literal lists (several patches), 5 matrix cores */
     uint64_t last_fit_draws[3];  /* with YTM_TRAIN_PROFILE=4: counter-stream words computed
                                     by the last fit's training kernel, one per lane and draw
                                     site (a Philox4x32-10 call): reservoir draws, Q-skip /

@@ -184,6 +184,7 @@ def test_training_on_several_patches(monkeypatch, dim, clauses, wgs, opts, env):
     dropped clauses, and samples whose negated literals are not complements (the list walks),
     against the oracle, bit for bit."""
     monkeypatch.setenv("YTM_TRAIN_GLOBAL", "1")
+    monkeypatch.setenv("YTM_TRAIN_MMA", "1")
     monkeypatch.setenv("YTM_TRAIN_WGS", wgs)
     for k, v in env.items():
         monkeypatch.setenv(k, v)
@@ -210,9 +211,28 @@ def test_training_on_several_patches(monkeypatch, dim, clauses, wgs, opts, env):
         upd = ref.fit_encoded(data, encY, **kr)
         st = tm.stats()
         assert st["train_kind"] == 2 and st["last_fit_updates"] == upd
+        assert st["train_product"] == (data is enc or not tm.append_negated)
         np.testing.assert_array_equal(tm.get_ta_state().reshape(ref.ta.shape), ref.ta)
         np.testing.assert_array_equal(tm.get_weights().reshape(ref.w.shape), ref.w)
         np.testing.assert_array_equal(tm.get_patch_weights().reshape(ref.pw.shape), ref.pw)
+
+
+@pytest.mark.parametrize("clauses,wgs,jit,product", [(21, "1", "1", 0), (22, "1", "1", 1), (43, "2", "1", 1), (42, "2", "1", 0),
+                                                     (99, "1", "0", 0), (100, "1", "0", 1)])
+def test_training_product_from_enough_clauses(monkeypatch, clauses, wgs, jit, product):
+    """Fewer than 22 clauses a workgroup (100 with the built-in kernel) train on literal lists."""
+    monkeypatch.setenv("YTM_TRAIN_GLOBAL", "1")
+    monkeypatch.setenv("YTM_TRAIN_WGS", wgs)
+    monkeypatch.setenv("YTM_JIT", jit)
+    rng = np.random.default_rng(2)
+    tm, ref = pair(clauses, (9, 8, 2), 3, rng, patch_dim=(3, 3))
+    y = rng.integers(0, 3, 8)
+    enc = tm.encode(image(rng, 8, (9, 8, 2)))
+    tm.fit(enc, y, is_X_encoded=True)
+    ref.fit_encoded(enc, ref.encode_y_multiclass(y))
+    assert tm.stats()["train_kind"] == 2 and tm.stats()["train_product"] == product
+    np.testing.assert_array_equal(tm.get_ta_state().reshape(ref.ta.shape), ref.ta)
+    np.testing.assert_array_equal(tm.get_weights().reshape(ref.w.shape), ref.w)
 
 
 @pytest.mark.parametrize("clauses,wgs", [(130, "1"), (160, "2")])
@@ -236,7 +256,7 @@ def test_first_sample_of_a_launch_counts_includes(monkeypatch, clauses, wgs):
         tm.fit(enc[e:e + 1], y[e:e + 1], is_X_encoded=True, random_stream=draws)
         upd = ref.fit_encoded(enc[e:e + 1], encY[e:e + 1], inject=draws)
         st = tm.stats()
-        assert st["train_kind"] == 2 and st["last_fit_updates"] == upd
+        assert st["train_kind"] == 2 and st["train_product"] == 1 and st["last_fit_updates"] == upd
         np.testing.assert_array_equal(tm.get_ta_state().reshape(ref.ta.shape), ref.ta)
         np.testing.assert_array_equal(tm.get_weights().reshape(ref.w.shape), ref.w)
         np.testing.assert_array_equal(tm.get_patch_weights().reshape(ref.pw.shape), ref.pw)

@@ -58,7 +58,8 @@ class YtmStats(ctypes.Structure):
         ("last_fit_feedback_samples", ctypes.c_uint64),
         ("last_fit_evaluations", ctypes.c_uint64),
         ("last_fit_stream", ctypes.c_int32),
-        ("reserved", ctypes.c_int32),
+        ("train_product", ctypes.c_int16),
+        ("score_path", ctypes.c_int16),
         ("last_fit_draws", ctypes.c_uint64 * 3),
     ]
 

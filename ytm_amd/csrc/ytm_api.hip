@@ -357,14 +357,30 @@ bool stream_geometry(const ytm_model* m, bool inject, bool force_global, int64_t
 
 // The global kernel of a model with several patches evaluates its clauses on the matrix cores
 // where the shape and the samples (`halves`: negated literals are complements, or not appended)
-// allow it; sets g->mma and then g->list_cap and g->threads.  20000 clauses of 552 literals on
-// samples of 900 patches, sixth epoch: 12.7 us per sample with literal lists, 10.3 with the
-// product by 768 threads; by 512, 640, 704 and 1024: 17.0, 10.6, 10.4 and 14.3 (two waves to a
-// SIMD do not hide the tiles' latency, 1024 threads spill).
+// allow it and a workgroup has kMmClauses clauses; sets g->mma and then g->list_cap and
+// g->threads.  20000 clauses of 552 literals on samples of 900 patches, sixth epoch: 12.7 us per
+// sample with literal lists, 10.3 with the product by 768 threads; by 512, 640, 704 and 1024:
+// 17.0, 10.6, 10.4 and 14.3 (two waves to a SIMD do not hide the tiles' latency, 1024 threads
+// spill).
+// The line, us per sample with lists and with the product, first and fifth epoch of 600 samples:
+//   patches  literals  clauses per workgroup
+//                      12                   20                   23                   31
+//      900     548                          17.9 15.2 16.3 14.1  20.2 17.9 16.7 14.3  21.2 17.9 17.5 14.6
+//     1089     520     14.8 12.2 16.1 13.8  15.9 13.0 17.4 14.2  20.1 17.6 17.8 14.3  21.4 18.0 18.5 14.5
+//     1444     580     16.3 14.4 17.9 14.8  17.3 15.2 19.3 15.1  21.1 19.3 19.6 15.3  22.6 19.6 20.6 15.7
+// and with 156 at 25, 36, 100, 324, 900 and 961 patches (452 to 784 literals) 27 to 37 against 18
+// to 21 in the fifth: also where there are fewer patch tiles than waves.
+// The built-in kernel (512 threads, no constants folded) needs more: 31 clauses 46 against 62, 62
+// clauses 60 against 68, 78 clauses 67 and 63 against 71 and 60, 102 clauses 80 and 72 against 75
+// and 66 (900 and 400 patches).
+// YTM_TRAIN_MMA=1 takes the product wherever it fits, =0 never.
 constexpr int kMmThreads = 768;
-void set_mma(Geom* g, ytm::TrainKind kind, int cpw, bool halves) {
+constexpr int kMmClauses = 22, kMmClausesBuiltin = 100;
+void set_mma(Geom* g, ytm::TrainKind kind, int cpw, bool halves, bool specialised) {
   g->mma = 0;
   if (kind != ytm::TrainKind::kGlobalConv || !ytm::mm_fits(*g) || g->threads < 256 || !(halves || !g->append_negated)) return;
+  const char* env = std::getenv("YTM_TRAIN_MMA");
+  if (env ? std::atoi(env) == 0 : (g->C + g->grid - 1) / g->grid < (specialised ? kMmClauses : kMmClausesBuiltin)) return;
   Geom t = *g;
   t.mma = 1;
   if (!train_lds_fits(t, kind, cpw, 0)) return;
@@ -373,7 +389,7 @@ void set_mma(Geom* g, ytm::TrainKind kind, int cpw, bool halves) {
   if (!std::getenv("YTM_TRAIN_THREADS")) g->threads = kMmThreads;
 }
 
-ytm::TrainKind choose_train_kind(Geom* g, int cpw, bool force_global, bool halves) {
+ytm::TrainKind choose_train_kind(Geom* g, int cpw, bool force_global, bool halves, bool specialised) {
   ytm::TrainKind kind = g->P == 1 ? ytm::TrainKind::kGlobalVanilla : ytm::TrainKind::kGlobalConv;
   if (!force_global && (g->P == 1 || ytm::literal_major(*g))) {
     const int cap = train_list_cap(*g, ytm::TrainKind::kResident, cpw);
@@ -381,7 +397,7 @@ ytm::TrainKind choose_train_kind(Geom* g, int cpw, bool force_global, bool halve
   }
   g->list_cap = train_list_cap(*g, kind, cpw);
   set_mask_lds(g, kind, cpw);
-  set_mma(g, kind, cpw, halves);
+  set_mma(g, kind, cpw, halves, specialised);
   return kind;
 }
 
@@ -483,6 +499,7 @@ int fit_steps(ytm_model* m, const ytm_dataset* ds, int64_t first, int64_t count,
   m->stats.last_fit_wait_frac = 0.0;
   m->stats.train_kind = (int32_t)ytm::TrainKind::kSteps;
   m->stats.train_specialised = 0;
+  m->stats.train_product = 0;
   m->stats.train_workgroups = (int32_t)std::min<int64_t>((g.C * 64 + 255) / 256, 65536);  // per launch
   m->stats.step += (uint64_t)count;
   m->stats.last_fit_samples = (uint64_t)count;
@@ -597,7 +614,7 @@ int ytm_load_train_kernels(ytm_model* m, int32_t kinds[4], int32_t* n_kinds) {
     if (int rc = load(gs, ytm::TrainKind::kStream)) return rc;
   int cpw;
   Geom g = train_geometry(m->g, m->cus, &cpw);
-  const ytm::TrainKind kind = choose_train_kind(&g, cpw, global, true);  // as encoded samples are
+  const ytm::TrainKind kind = choose_train_kind(&g, cpw, global, true, true);  // as encoded samples are
   return load(g, kind);
 }
 
@@ -628,7 +645,7 @@ int ytm_compile_train_kernel(const ytm_params* params, int train_kind, int injec
     return fail(YTM_EINVAL, "train_kind 1 is for one patch, 2 for several, 0 for one patch or a literal-major model");
   g.list_cap = train_list_cap(g, (ytm::TrainKind)train_kind, cpw);
   set_mask_lds(&g, (ytm::TrainKind)train_kind, cpw);
-  set_mma(&g, (ytm::TrainKind)train_kind, cpw, true);  // as encoded samples are
+  set_mma(&g, (ytm::TrainKind)train_kind, cpw, true, true);  // as encoded samples are
   std::vector<char> code;
   std::string why;
   if (!ytm::jit_compile(g, (ytm::TrainKind)train_kind, injected != 0, &code, &why))
@@ -894,6 +911,12 @@ int fit_range(ytm_model* m, const ytm_dataset* ds, int64_t first, int64_t count,
   ytm::TrainKind kind;
   int rng_slots = 0;
   size_t lds = 0;
+  auto choose = [&](bool specialised) {
+    g = train_geometry(m->g, m->cus, &cpw);  // the training kernels read both
+    kind = choose_train_kind(&g, cpw, global, ds->halves == 1, specialised);
+    rng_slots = kind == ytm::TrainKind::kResident ? ytm::train_rng_slots(cpw, g) : 0;
+    lds = ytm::train_lds_bytes(kind, cpw, rng_slots, g);
+  };
   // The streaming kernel pays when few samples need feedback: it is taken unless the last
   // fit had feedback at kStreamBelow of its samples or more, or YTM_TRAIN_STREAM forces it
   // (1) or rules it out (0).
@@ -904,12 +927,8 @@ int fit_range(ytm_model* m, const ytm_dataset* ds, int64_t first, int64_t count,
     cpw = ytm::kStreamClauses;
     lds = ytm::stream_lds_bytes(g, g.threads);
   } else {
-    g = train_geometry(m->g, m->cus, &cpw);  // the training kernels read both
-    kind = choose_train_kind(&g, cpw, global, ds->halves == 1);
-    rng_slots = kind == ytm::TrainKind::kResident ? ytm::train_rng_slots(cpw, g) : 0;
-    lds = ytm::train_lds_bytes(kind, cpw, rng_slots, g);
+    choose(ytm::jit_enabled());
   }
-  const int grid = g.grid, D = g.groups;
   // Kernel specialised for this model's geometry (hipRTC), else the built-in one.
   // YTM_JIT=0 selects the built-in kernel; YTM_JIT=2 makes an unavailable compile an error.
   hipFunction_t jit_fn = nullptr;
@@ -920,7 +939,9 @@ int fit_range(ytm_model* m, const ytm_dataset* ds, int64_t first, int64_t count,
     if (!jit_fn && jit_env && std::atoi(jit_env) == 2)
       return fail(YTM_EHIP, "specialised training kernel unavailable: " + why);
   }
+  if (!jit_fn && g.mma) choose(false);  // the built-in kernel may do better without
   if (!jit_fn) g.threads = ytm::kTrainThreads;
+  const int grid = g.grid, D = g.groups;
   int bpc = 0;
   if (jit_fn)
     HIP_TRY(ytm::jit_occupancy(jit_fn, g.threads, lds, &bpc));
@@ -1055,6 +1076,7 @@ int fit_range(ytm_model* m, const ytm_dataset* ds, int64_t first, int64_t count,
   m->stats.last_fit_wait_frac = cnt[2] ? (double)cnt[1] / (double)cnt[2] : 0.0;
   m->stats.train_kind = (int32_t)kind;
   m->stats.train_specialised = jit_fn != nullptr;
+  m->stats.train_product = kind == ytm::TrainKind::kGlobalConv && g.mma;
   m->stats.step += (uint64_t)count;
   m->stats.last_fit_samples = (uint64_t)count;
   m->stats.last_fit_updates = upd;
@@ -1092,6 +1114,7 @@ struct ScorePlan {
   size_t acc_per_sample;
   // what d_slists holds that outlives a call on an unchanged model, 0 for nothing (the lists of
   // several patches are in the order of the batch they score)
+  int16_t path() const { return mm.steps ? 5 : chunks ? 2 : wide ? 3 : lists_bytes ? 4 : 1; }  // ytm_stats
   int kept() const { return mm.steps ? (mm.half_steps ? 4 : 2 + mm.ternary) : wide; }
 };
 
@@ -1267,6 +1290,7 @@ int ytm_score_dataset(ytm_model* m, const ytm_dataset* ds, float* class_sums) {
   ytm::pinned_free(pinned);
   if (e != hipSuccess) return fail(YTM_EHIP, std::string("score failed: ") + hipGetErrorString(e));
   m->stats.last_score_kernel_ms = ms;
+  m->stats.score_path = plan.path();
   return YTM_OK;
 }
 
@@ -1315,6 +1339,7 @@ int ytm_score_dataset_noalloc(ytm_model* m, const ytm_dataset* ds, float* d_clas
     return fail(YTM_EHIP, std::string("score failed: ") + hipGetErrorString(e));
   }
   m->stats.last_score_kernel_ms = ms;
+  m->stats.score_path = plan.path();
   return YTM_OK;
 }
 
