@@ -144,7 +144,7 @@ int ytm_shutdown(void);
  * idle, the longest unused freed first; ytm_destroy of the device's last model frees it all.
  * Another allocator of the process cannot have it before.  Pinned host memory is kept alike, at
  * most 64 MiB, while any model lives.  A model holds the room of its scorers' operands from the
- * start where it is no larger than its TA states. */
+ * start where it is no larger than its TA states and than 256 MiB and memory allows. */
 int ytm_create(const ytm_params *params, ytm_model **out);
 void ytm_destroy(ytm_model *m);
 /* L, W (=number_of_literal_chunks), P (=number_of_patches), number of TA bit-planes. */

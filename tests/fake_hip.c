@@ -48,6 +48,8 @@ size_t fake_live(int dev) { /* bytes allocated on a device (-1: pinned) */
 }
 static int delay_ms;
 void fake_delay_malloc(int ms) { delay_ms = ms; } /* each hipMalloc takes that long */
+static size_t limit;
+void fake_limit(size_t bytes) { limit = bytes; } /* what a device holds at most; 0: anything */
 long fake_calls(int which) {
     const long c[] = {calls_malloc, calls_free, calls_host_malloc, calls_host_free, calls_large};
     return c[which];
@@ -91,6 +93,7 @@ hipError_t hipMalloc(void **p, size_t bytes) {
     __sync_fetch_and_add(&calls_malloc, 1);
     if (bytes >= 1 << 20) __sync_fetch_and_add(&calls_large, 1);
     if (delay_ms) usleep(1000 * delay_ms);
+    if (limit && fake_live(device) + bytes > limit) return last_error = hipErrorOutOfMemory;
     return get(p, bytes, device);
 }
 hipError_t hipFree(void *p) {

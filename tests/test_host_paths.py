@@ -48,7 +48,7 @@ def test_every_call_failing(fake_hip, entry):
 
 
 @pytest.mark.parametrize("what", ["oldest_leave_first", "given_back_with_the_last_model", "allocations_unlocked", "staging_per_device",
-                                  "new_models_first_score"])
+                                  "new_models_first_score", "room_for_operands"])
 def test_blocks(fake_hip, what):
     child(fake_hip, what)
 
@@ -303,6 +303,27 @@ def new_models_first_score(fake, lib, L):
         lib.ytm_destroy(first)
 
 
+def room_for_operands(fake, lib, L):
+    """A model of 180 MB of states: created where little more than these fits, without the room of
+    its scores' operands; and one of 1.1 GB of states holds no such room."""
+    def model(clauses):
+        p = L.YtmParams(clauses=clauses, classes=3, dim0=10000, dim1=1, dim2=1, patch_dim0=10000, patch_dim1=1,
+                        number_of_ta_states=256, max_included_literals=20000, append_negated=1, encode_loc=1,
+                        coalesced=1, negative_polarity=1, thresh=10, s_inv=0.2, q_prob=1.0, seed=1)
+        m = ctypes.c_void_p()
+        return lib.ytm_create(ctypes.byref(p), ctypes.byref(m)), m
+
+    for clauses, most, least in ((8000, 185 * MB, None), (8000, 0, 250 * MB), (50000, 0, None)):
+        planes = clauses * 9 * 625 * 4
+        fake.fake_limit(most)
+        rc, m = model(clauses)
+        fake.fake_limit(0)
+        assert rc == 0, (clauses, most)
+        held = fake.fake_live(0)
+        assert held > least if least else held < planes + 30 * MB, (clauses, most, held)
+        lib.ytm_destroy(m)
+
+
 def every_call_failing(name, fake, lib, L):
     prepare, call, free = entry(name, lib, L)
     wrong = []
@@ -337,6 +358,7 @@ if __name__ == "__main__":
     fake = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
     fake.fake_live.restype = ctypes.c_size_t
     fake.fake_calls.restype = ctypes.c_long
+    fake.fake_limit.argtypes = [ctypes.c_size_t]
     from ytm_amd import _lib
 
     if sys.argv[2] in ENTRIES:

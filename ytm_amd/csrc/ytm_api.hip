@@ -242,6 +242,7 @@ int upload(void** dst, const void* src, size_t bytes, hipStream_t s) {
 // Bytes of the operands or lists that scores of the model will mostly need: of samples with
 // complemented negations, as they are encoded, and weights of two digits.
 size_t operand_room(const Geom& g);
+constexpr size_t kOperandRoom = (size_t)256 << 20;  // allocated with a model at most
 
 // Picks the persistent grid (one workgroup per CU at most, at least ~12 clauses each, and
 // two workgroups for models of more than one clause) and the class-sum grouping (groups of
@@ -552,13 +553,20 @@ int ytm_create(const ytm_params* params, ytm_model** out) {
   CREATE_TRY(hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking));
   CREATE_TRY(hipEventCreate(&m->ev0));
   CREATE_TRY(hipEventCreate(&m->ev1));
-  // One block for the planes and, where it is no larger, the room of the scorers' operands: the
-  // first score of a new model then waits for no hipMalloc (2000 clauses of 784 bits, one sample:
-  // 209 us with buffers and a pinned result of the model's own, 157 from the pool and this).
+  // One block for the planes and, where it is no larger than they and than kOperandRoom, the room
+  // of the scorers' operands: the first score of a new model then waits for no hipMalloc (2000
+  // clauses of 784 bits, one sample: 209 us with buffers and a pinned result of the model's own,
+  // 157 from the pool and this).  A model that is only trained needs none: no more than
+  // kOperandRoom (10000 clauses of 20000 literals: 149 MB), and the planes alone where memory is
+  // short.
   const size_t planes_bytes = ((size_t)(g.C * g.np * g.W) * 4 + 255) & ~(size_t)255;
   size_t operands = operand_room(g);
-  if (operands > planes_bytes) operands = 0;
-  CREATE_TRY(ytm::pool_alloc((void**)&m->d_planes, planes_bytes + operands));
+  if (operands > std::min(planes_bytes, kOperandRoom) ||
+      ytm::pool_alloc((void**)&m->d_planes, planes_bytes + operands) != hipSuccess) {
+    (void)hipGetLastError();
+    operands = 0;
+    CREATE_TRY(ytm::pool_alloc((void**)&m->d_planes, planes_bytes));
+  }
   if (operands) {
     m->d_slists = (unsigned char*)m->d_planes + planes_bytes;
     m->slists_bytes = operands;
