@@ -213,12 +213,13 @@ int ytm_score_dataset(ytm_model *m, const ytm_dataset *ds, float *class_sums);
  * for callers that cannot allocate device memory (code under HIP graph capture, tight
  * serving loops, harnesses that forbid hipMalloc).  d_class_sums is a DEVICE pointer to
  * float (N, classes), written with the same values ytm_score_dataset returns.  The
- * kernels' literal lists and int64 class-sum accumulators live in a static per-GPU scratch
- * array of YTM_NOALLOC_SCRATCH_BYTES (32 MiB; it is part of libytm's code object, so every
+ * model's operands or literal lists and the samples' firing words or int64 class-sum
+ * accumulators live in a static per-GPU scratch array of YTM_NOALLOC_SCRATCH_BYTES (32 MiB; it is part of libytm's code object, so every
  * GPU on which the library's kernels are loaded holds it until the process ends, whether or
- * not this entry point is called there); samples go through in passes that fit it.  YTM_EINVAL when the model's
- * lists plus one sample's accumulators do not fit (e.g. one-patch models of more than
- * about 65000 wide clauses).  Calls on one GPU share the array, so overlapping calls
+ * not this entry point is called there); samples go through in passes that fit it.  Models
+ * whose matrix operands do not fit are scored on literal lists; YTM_EINVAL when these and one
+ * sample's accumulators do not fit either (e.g. one-patch models of more than about 65000 wide
+ * clauses).  Calls on one GPU share the array, so overlapping calls
  * would race: the library serialises them per GPU with a lock.  Synchronous on return. */
 #define YTM_NOALLOC_SCRATCH_BYTES (32u << 20)
 int ytm_score_dataset_noalloc(ytm_model *m, const ytm_dataset *ds, float *d_class_sums);

@@ -30,11 +30,12 @@ def pair(clauses, dim, classes, rng, weight=50, **kw):
     return tm, ref
 
 
-def check(tm, ref, enc):
+def check(tm, ref, enc, path=5):
     data = tm._device_data(enc)
     want = ref.score(enc)
     np.testing.assert_array_equal(tm.score_device(data), want)
     np.testing.assert_array_equal(tm.score_device(data), want)  # the kept operands
+    assert tm.stats()["score_path"] == path
     return want
 
 
@@ -80,7 +81,7 @@ def test_all_literals(dim, patch, negated):
     odd = enc & rng.integers(0, 2**32, enc.shape, dtype=np.uint32) | enc & rng.integers(0, 2**32, enc.shape,
                                                                                        dtype=np.uint32)
     check(tm, ref, enc)
-    check(tm, ref, odd)
+    check(tm, ref, odd, path=5 if tm.number_of_literals <= 9 * 64 else 4)
     check(tm, ref, enc)
 
 
@@ -142,6 +143,26 @@ def test_one_patch(bits, clauses, n):
     check(tm, ref, enc)
 
 
+@pytest.mark.parametrize("dim,patch,clauses,n,room,odd", [
+    ((784, 1, 1), None, 2000, 2500, 1056 * 1088 + 256, 0),     # 1056 rows a pass, the last of 388 by single tiles
+    ((784, 1, 1), None, 2000, 2500, 1056 * 1088 + 256, 1500),  # one sample of the second pass without complements
+    ((784, 1, 1), None, 2000, 2500, 1056 * 1088 + 256, 2400),  # one of the last
+    ((784, 1, 1), None, 60, 70, 0, 0),                         # 32 a pass: the first makes the operands
+    ((9, 8, 2), (3, 3), 60, 100, 32 * 16 + 256, 0),            # several patches, a last pass of 4
+])
+def test_several_passes(monkeypatch, dim, patch, clauses, n, room, odd):
+    """Rows of more samples than a pass has room for."""
+    monkeypatch.setenv("YTM_SCORE_PASS", str(room))
+    rng = np.random.default_rng(10)
+    tm, ref = pair(clauses, dim, 5, rng, **({"patch_dim": patch} if patch else {}))
+    enc = tm.encode(image(rng, n, dim))
+    if odd:
+        enc = enc.copy()
+        enc[odd] &= rng.integers(0, 2**32, enc[odd].shape, dtype=np.uint32)
+    want = check(tm, ref, enc)
+    assert np.unique(want).size > 1
+
+
 @pytest.mark.parametrize("bits,clauses,n,negated", [(90, 64, 300, False), (1000, 33, 70000, False),
                                                     (10000, 40, 7000, True), (10000, 7000, 300, True)])
 def test_one_patch_without_allocation(bits, clauses, n, negated):
@@ -153,6 +174,7 @@ def test_one_patch_without_allocation(bits, clauses, n, negated):
     tm, ref = pair(clauses, (bits, 1, 1), 4, rng, append_negated=negated)
     enc = tm.encode(image(rng, n, (bits, 1, 1)))
     got, noalloc = score_both(tm, tm._device_data(enc), 4)
+    assert tm.stats()["score_path"] == (3 if clauses == 7000 else 5)
     np.testing.assert_array_equal(got, noalloc)
     np.testing.assert_array_equal(got[:200], ref.score(enc[:200]))
 
@@ -166,7 +188,7 @@ def test_literal_lists_of_wide_patches(monkeypatch):
     enc = tm.encode(image(rng, 5, dim))
     for least in ("1", "1000000"):
         monkeypatch.setenv("YTM_SCORE_WHOLE_MIN", least)
-        check(tm, ref, enc)
+        check(tm, ref, enc, path=4)
 
 
 @pytest.mark.parametrize("dim,clauses,wgs,opts", [

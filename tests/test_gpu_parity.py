@@ -443,10 +443,12 @@ def test_many_classes_injected_and_multioutput(case):
     np.testing.assert_array_equal(mo.score(encX, is_X_encoded=True), refo.score(encX))
 
 
-def test_scoring_lists_follow_the_state():
+@pytest.mark.parametrize("matrix,path", [("0", 3), ("1", 5)])
+def test_scoring_lists_follow_the_state(monkeypatch, matrix, path):
     """One-patch scoring keeps its literal lists between calls while the TA states are
     unchanged: scores after a second call, after more training and after ytm_set_ta_state
-    (load_state_dict) all equal the oracle's."""
+    (load_state_dict) all equal the oracle's.  The same for the matrix cores' operands."""
+    monkeypatch.setenv("YTM_SCORE_MATRIX", matrix)
     tm, ref, X, y, Xt, yt = pair(2, 300, 200, clauses=120)
     encX, encXt = tm.encode(X), tm.encode(Xt)
     encY = ref.encode_y_multiclass(y)
@@ -455,6 +457,7 @@ def test_scoring_lists_follow_the_state():
     ref.fit_encoded(encX[:200], encY[:200])
     for where in ("first", "again"):
         np.testing.assert_array_equal(tm.score_device(data), ref.score(encXt), err_msg=where)
+        assert tm.stats()["score_path"] == path
     tm.fit(encX[200:], y[200:], is_X_encoded=True)
     ref.fit_encoded(encX[200:], encY[200:])
     np.testing.assert_array_equal(tm.score_device(data), ref.score(encXt), err_msg="after training")
@@ -467,14 +470,16 @@ def test_scoring_lists_follow_the_state():
     data.release()
 
 
+@pytest.mark.parametrize("matrix,path", [("0", 3), ("1", 5)])
 @pytest.mark.parametrize("wmax", [2048, 2049, 100000])
-def test_wide_scoring_weight_range(wmax):
+def test_wide_scoring_weight_range(monkeypatch, wmax, matrix, path):
     """One-patch wide scoring with 4 or more classes sums the votes of a wave's 64 clauses
     on the matrix cores while every weight of those clauses is at most 2048 in magnitude
     (f16 holds it exactly) and adds them one by one otherwise: random states with weights
     up to +-2048 (both bounds present), one weight of 2049 in the second wave's clauses,
-    and weights up to +-100000, against the oracle."""
-    print(f"[wide weights] wmax {wmax}", flush=True)
+    and weights up to +-100000, against the oracle; and the same on the matrix scorer."""
+    monkeypatch.setenv("YTM_SCORE_MATRIX", matrix)
+    print(f"[wide weights] wmax {wmax} matrix {matrix}", flush=True)
     rng = np.random.default_rng(31)
     kw = dict(number_of_clauses_per_class=300, T=50, s=5.0, dim=(28, 28, 1), n_classes=10)
     tm = MultiClassTM(**kw, seed=7)
@@ -494,6 +499,7 @@ def test_wide_scoring_weight_range(wmax):
     want = oracle.score(encXt)
     assert np.count_nonzero(want) > want.size // 2, "a meaningful comparison needs firing clauses"
     np.testing.assert_array_equal(tm.score(encXt, is_X_encoded=True), want)
+    assert tm.stats()["score_path"] == path
     tm.release()
 
 
@@ -535,6 +541,7 @@ def test_encoded_samples_without_complement_halves(monkeypatch, halves_env):
     not (bits flipped here), the whole copy.  Both against the oracle; YTM_TRAIN_XT_HALVES=0
     stages the whole copy either way."""
     monkeypatch.setenv("YTM_TRAIN_GLOBAL", "1")
+    monkeypatch.setenv("YTM_TRAIN_MMA", "0")  # the product does not read the copy
     monkeypatch.setenv("YTM_TRAIN_XT_HALVES", halves_env)
     tm, ref, X, y, *_ = pair(4, 8, clauses=40)
     encX = tm.encode(X)
@@ -549,7 +556,7 @@ def test_encoded_samples_without_complement_halves(monkeypatch, halves_env):
     for data in (encX, odd):
         tm.fit(data, y, is_X_encoded=True)
         upd = ref.fit_encoded(data, encY)
-        assert tm.stats()["train_kind"] == 2
+        assert tm.stats()["train_kind"] == 2 and tm.stats()["train_product"] == 0
         assert tm.stats()["last_fit_updates"] == upd
         assert_state_equal(tm, ref)
 
@@ -711,17 +718,19 @@ def random_state(tm, ref, rng, include_p):
     ref.w[...] = w.reshape(ref.w.shape)
 
 
-@pytest.mark.parametrize("dim,patch_dim,classes,clauses", [
-    ((100, 1, 1), None, 3, 300),     # one patch, 7 words
-    ((30, 1, 1), None, 20, 200),     # one patch, more classes than the tiled scorer holds
-    ((1500, 1, 1), None, 2, 150),    # one patch, 94 words
-    ((12, 12, 2), (4, 4), 4, 300),   # several patches, literal lists
-    ((16, 16, 16), (3, 3), 3, 120),  # several patches, 340 literals: some clauses beyond the list capacity
-    ((32, 32, 32), (3, 3), 2, 40),   # 696 literals x 29 patch words: list entries are literal indices
+@pytest.mark.parametrize("matrix", ["0", "1"])
+@pytest.mark.parametrize("dim,patch_dim,classes,clauses,path", [
+    ((100, 1, 1), None, 3, 300, 2),     # one patch, 7 words
+    ((30, 1, 1), None, 20, 200, 1),     # one patch, more classes than the tiled scorer holds
+    ((1500, 1, 1), None, 2, 150, 3),    # one patch, 94 words
+    ((12, 12, 2), (4, 4), 4, 300, 4),   # several patches, literal lists
+    ((16, 16, 16), (3, 3), 3, 120, 4),  # several patches, 340 literals: some clauses beyond the list capacity
+    ((32, 32, 32), (3, 3), 2, 40, 4),   # 696 literals x 29 patch words: list entries are literal indices
 ])
-def test_inference_random_state(dim, patch_dim, classes, clauses):
+def test_inference_random_state(monkeypatch, dim, patch_dim, classes, clauses, path, matrix):
     """Class sums and clause outputs on random states: every inference kernel variant
-    (tiles, lists, the include-mask fallback) against the oracle."""
+    (tiles, lists, the include-mask fallback; the matrix cores) against the oracle."""
+    monkeypatch.setenv("YTM_SCORE_MATRIX", matrix)
     kw = dict(number_of_clauses_per_class=clauses, T=50, s=5.0, dim=dim, n_classes=classes, seed=7)
     if patch_dim is not None:
         kw["patch_dim"] = patch_dim
@@ -737,6 +746,7 @@ def test_inference_random_state(dim, patch_dim, classes, clauses):
     encX = tm.encode(X)
     np.testing.assert_array_equal(encX, ref.encode(X))
     np.testing.assert_array_equal(tm.score(encX, is_X_encoded=True), ref.score(encX))
+    assert tm.stats()["score_path"] == (5 if matrix == "1" else path)
     np.testing.assert_array_equal(tm.transform(encX, is_X_encoded=True), ref.transform(encX))
     ref_pw = ref.transform(encX[:9], patchwise=True)
     np.testing.assert_array_equal(tm.transform_patchwise(encX[:9], is_X_encoded=True), ref_pw)
@@ -759,10 +769,12 @@ def test_score_whole_sample_blocks(monkeypatch):
     random_state(tm, ref, rng, include_p)
     X = (rng.random((20,) + dim) < 0.5).astype(np.uint32).reshape(20, -1)
     encX = tm.encode(X)
+    monkeypatch.setenv("YTM_SCORE_MATRIX", "0")
     monkeypatch.setenv("YTM_SCORE_WHOLE_MIN", "1")
     whole = tm.score(encX, is_X_encoded=True)
     monkeypatch.setenv("YTM_SCORE_WHOLE_MIN", "1000000")
     chunked = tm.score(encX, is_X_encoded=True)
+    assert tm.stats()["score_path"] == 4
     np.testing.assert_array_equal(whole, chunked)
     np.testing.assert_array_equal(whole[:3], ref.score(encX[:3]))
 

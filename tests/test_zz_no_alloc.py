@@ -5,9 +5,10 @@ Both are called through the C-ABI on the same model and device-resident dataset;
 allocation-free one writes into a caller-owned device buffer, and the oracle, loaded with
 the GPU model's state, scores the same samples.  Two calls in a row, the
 second on fewer samples, so a stale scratch array from the first call would show.  Every
-scoring kernel path is covered: wide one-patch clauses (literal lists), several patches
-(literal-major samples), narrow one-patch clauses (per-chunk sums, several passes over the
-scratch), and the plain scorer (more classes than the tiled scorers hold).
+scoring kernel path is covered: the matrix cores, and without them wide one-patch clauses
+(literal lists), several patches (literal-major samples), narrow one-patch clauses (per-chunk
+sums, several passes over the scratch), and the plain scorer (more classes than the tiled
+scorers hold).
 """
 import ctypes
 
@@ -57,9 +58,11 @@ def random_state(tm, rng, include_p):
                                   "min_y": None, "max_y": None}})
 
 
-@pytest.mark.parametrize("case", ["wide_one_patch", "several_patches", "narrow_one_patch_passes", "plain"])
-def test_noalloc_matches_score_dataset(case):
-    print(f"[noalloc] case {case}", flush=True)
+@pytest.mark.parametrize("matrix", ["0", "1"])
+@pytest.mark.parametrize("case,path", [("wide_one_patch", 3), ("several_patches", 4), ("narrow_one_patch_passes", 2), ("plain", 1)])
+def test_noalloc_matches_score_dataset(monkeypatch, case, path, matrix):
+    monkeypatch.setenv("YTM_SCORE_MATRIX", matrix)
+    print(f"[noalloc] case {case} matrix {matrix}", flush=True)
     rng = np.random.default_rng(23)
     if case == "wide_one_patch":  # config 2: 49-word clauses
         X, y, Xt, _, kw = workloads.make(2, 300, 3000)
@@ -93,6 +96,7 @@ def test_noalloc_matches_score_dataset(case):
     for n in sizes:
         data = tm.device_data(encXt[:n], is_X_encoded=True)
         ref, got = score_both(tm, data, tm.number_of_outputs)
+        assert tm.stats()["score_path"] == (5 if matrix == "1" else path)
         data.release()
         np.testing.assert_array_equal(got, ref, err_msg=f"{case} n={n}")
         assert np.any(ref != 0), "a meaningful comparison needs non-zero class sums"

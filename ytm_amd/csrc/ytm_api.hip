@@ -65,7 +65,9 @@ struct ytm_dataset {
   uint32_t* d_X;   // [N][P][W]
   int32_t* d_Y;    // [N][K]
   int64_t N;
-  uint32_t* d_XT;  // [N][L][ceil(P/32)] literal-major copy (several patches, where a kernel reads it), or null
+  // [N][L][ceil(P/32)] literal-major copy (several patches, samples to train on or that the matrix
+  // cores do not score), or null.  Training that evaluates clauses as a product does not read it.
+  uint32_t* d_XT;
   // every sample's literals Lh..L-1 are the complements of 0..Lh-1 (1), not (0), or not known
   // (-1, one patch until a score asks)
   mutable int halves;
@@ -793,6 +795,12 @@ int check_halves(ytm_model* m, const ytm_dataset* ds) {
   ds->halves = ok == 1;
   return YTM_OK;
 }
+
+// The model's scoring on the matrix cores.  YTM_SCORE_MATRIX=0 (a test hook) rules it out.
+ytm::MatrixPlan score_matrix(const ytm_model* m, int halves, int64_t N) {
+  const char* env = std::getenv("YTM_SCORE_MATRIX");
+  return env && std::atoi(env) == 0 ? ytm::MatrixPlan{} : ytm::matrix_plan(m->g, halves, m->w_bound, N);
+}
 }  // namespace
 
 extern "C" {
@@ -806,9 +814,9 @@ int ytm_dataset_create(ytm_model* m, const uint32_t* encX, const int32_t* encY, 
   if (!rc && encY) rc = upload((void**)&ds->d_Y, encY, (size_t)(N * g.K) * 4, m->stream);
   if (!rc && g.P > 1) rc = check_halves(m, ds);
   if (!rc && ytm::literal_major(g) && N > 0 &&
-      (encY || ytm::matrix_plan(g, ds->halves, m->w_bound, N).steps == 0)) {
-    // Several patches: the training kernel evaluates clauses on a literal-major copy, and so
-    // do the scorers of models that the matrix cores do not take.
+      (encY || score_matrix(m, ds->halves, N).steps == 0)) {
+    // Several patches: the training kernels' literal lists are walked on a literal-major copy, and
+    // so are those of the scorers of models that the matrix cores do not take.
     const size_t bytes = (size_t)(N * g.L * ((g.P + 31) / 32)) * 4;
     hipError_t e = ytm::pool_alloc((void**)&ds->d_XT, bytes);
     if (e == hipSuccess) e = ytm::launch_transpose(ds->d_X, N, ds->d_XT, g, m->stream);
@@ -1120,9 +1128,9 @@ struct ScorePlan {
   bool wide;
   int64_t chunks;
   size_t acc_per_sample;
+  int16_t path() const { return mm.steps ? 5 : chunks ? 2 : wide ? 3 : lists_bytes ? 4 : 1; }  // ytm_stats
   // what d_slists holds that outlives a call on an unchanged model, 0 for nothing (the lists of
   // several patches are in the order of the batch they score)
-  int16_t path() const { return mm.steps ? 5 : chunks ? 2 : wide ? 3 : lists_bytes ? 4 : 1; }  // ytm_stats
   int kept() const { return mm.steps ? (mm.half_steps ? 4 : 2 + mm.ternary) : wide; }
 };
 
@@ -1153,7 +1161,7 @@ int score_plan(ytm_model* m, const ytm_dataset* ds, ScorePlan* out) {
   // and samples: 250 us less product, against 30 us for the round trip).
   if (ds->halves < 0 && ytm::long_rows(m->g, ds->N))
     if (int rc = check_halves(m, ds)) return rc;
-  p.mm = ytm::matrix_plan(m->g, ds->halves, m->w_bound, ds->N);
+  p.mm = score_matrix(m, ds->halves, ds->N);
   if (p.mm.steps) {
     p.lists_bytes = p.mm.bytes;
     p.acc_per_sample = (size_t)p.mm.row_words * 4 + p.mm.sample_bytes;
@@ -1247,7 +1255,10 @@ int ytm_score_dataset(ytm_model* m, const ytm_dataset* ds, float* class_sums) {
   if (N == 0) return YTM_OK;
   ScorePlan plan{};
   if (int rc = score_plan(m, ds, &plan)) return rc;
-  const int64_t per_pass = std::max<int64_t>(score_pass(plan, N, (size_t)256 << 20), std::min<int64_t>(N, 1024));
+  // YTM_SCORE_PASS (a test hook): the bytes of a pass's rows
+  const char* room_env = std::getenv("YTM_SCORE_PASS");
+  const size_t pass_room = room_env ? (size_t)std::max(0ll, std::atoll(room_env)) : (size_t)256 << 20;
+  const int64_t per_pass = std::max<int64_t>(score_pass(plan, N, pass_room), std::min<int64_t>(N, room_env ? 32 : 1024));
   // The rows and the sums come from the pool, where a new model finds an earlier one's.
   void *acc = nullptr, *sums = nullptr, *pinned = nullptr;
   const size_t out_bytes = (size_t)(N * g.K) * 4;

@@ -1566,32 +1566,29 @@ __device__ __forceinline__ int mm_select(const TrainArgs& a, const Geom& g, cons
   return row_max(pos + 1) - 1;
 }
 
-// The votes of the clauses of mm_select (c and its weights of each row) to the partial sums.
-__device__ __forceinline__ void mm_vote(const Geom& g, long long* s_part, bool fires, int64_t c, const float* wrow) {
+// The votes of the clauses of mm_select (the weights of each row's) to the partial sums.
+__device__ __forceinline__ void mm_vote(const Geom& g, long long* s_part, bool fires, const float* wrow) {
   const int q = lane_id() & 15;
   if (!fires) return;
-  if (g.coalesced) {
-    for (int k = q; k < g.K; k += 16) atomicAdd((unsigned long long*)&s_part[k], (unsigned long long)(long long)wrow[k]);
-  } else if (q == 0) {
-    const int64_t k = c / g.per_bank;
-    atomicAdd((unsigned long long*)&s_part[k], (unsigned long long)(long long)wrow[k]);
-  }
+  for (int k = q; k < g.K; k += 16) atomicAdd((unsigned long long*)&s_part[k], (unsigned long long)(long long)wrow[k]);
 }
 
 // Clause state in global memory (L2/MALL resident across samples); any P.  A software
 // pipeline over samples, like the resident kernel's; per sample i:
-//   1. wave 0 adds the patch weights of sample i's selections (select_active,
-//      kernel.cu:305) and publishes its partial class sums; then every wave stages sample
-//      i+1 (its literal-major copy; with mask_lds its words) into LDS.
-//   2. wave 0 waits for sample i's totals and derives the targets (phases B/C); the other
-//      waves evaluate sample i+1 with the current state (phase A, speculative).
+//   1. every wave stages sample i+1 into LDS (its literal-major copy; with mask_lds its words;
+//      with mma its rows, copied while sample i-1 was evaluated).
+//   2. wave 0 publishes sample i's partial class sums, waits for the totals and derives the
+//      targets (phases B/C); the last wave adds the patch weights of sample i's selections
+//      (select_active, kernel.cu:305); the waves, wave 0 once it has the totals, evaluate
+//      sample i+1 with the current state (phase A, speculative).
 //   3. D: the feedback decisions of sample i (clause_update, kernel.cu:531-613) take
 //      (clause, class) pairs, 64 / K clauses per claim (decide_pair), or a wave per clause
 //      when K is above 32 (decide); a clause that changes takes back its speculative votes
 //      for sample i+1 and is queued.  Then its literal updates: narrow clauses (W <= 32)
 //      several to a wave, wide ones a 64-word chunk per wave.
 //   4. the updated clauses rebuild their literal lists and are evaluated again for sample
-//      i+1, so the result is exactly the sequential one.
+//      i+1, so the result is exactly the sequential one; with mma those whose include mask
+//      changed (their operands are made again), and the others vote with their new weights.
 // Phase A of sample i and its re-evaluations are over before sample i+1 is staged, so one
 // literal-major buffer serves; the words of samples i and i+1 (mask_lds) take two.
 template <bool VANILLA, bool INJECT>
@@ -1788,7 +1785,7 @@ __device__ __forceinline__ void train_global_body(const TrainArgs& a, const Geom
                                         row < have && s_drop[ix] == 0 ? s_bm + ix * mm_pw : nullptr, s_invr,
                                         use_rb ? s_rb[(j & 1) * cpw + ix] : -1);
       if (sel >= 0 && (lane & 15) == 0) sel_n[ix] = sel;
-      mm_vote(g, part, sel >= 0, c_begin + ix, s_wg + (int64_t)ix * g.K);
+      mm_vote(g, part, sel >= 0, s_wg + (int64_t)ix * g.K);
       have = 0;
     }
   };
@@ -2013,7 +2010,7 @@ __device__ __forceinline__ void train_global_body(const TrainArgs& a, const Geom
             sel_n[idx] = sel;
             ninc_n[idx] = s_nlit[idx];
           }
-          mm_vote(g, s_part[bn], sel >= 0, c_begin + idx, s_wg + (int64_t)idx * g.K);
+          mm_vote(g, s_part[bn], sel >= 0, s_wg + (int64_t)idx * g.K);
         }
       }
     } else {
