@@ -140,10 +140,10 @@ int ytm_shutdown(void);
  * 32-bit literal-draw site index of the counter stream).  YTM_EINVAL otherwise.
  *
  * Device memory that a call is done with (buffers of its host arrays, a destroyed data set's or
- * model's) is kept for later calls while a model lives on that device, at most 1 GiB of it
- * idle, the longest unused freed first; ytm_destroy of the device's last model frees it all.
- * Another allocator of the process cannot have it before.  Pinned host memory is kept alike, at
- * most 64 MiB, while any model lives.  A model holds the room of its scorers' operands from the
+ * model's) is kept for later calls, the longest unused freed first: at most 1 GiB of it idle
+ * while a model lives on that device, and 256 MiB once ytm_destroy ended the last one, until
+ * ytm_shutdown.  Another allocator of the process cannot have it before.  Pinned host memory is
+ * kept alike, at most 64 and 16 MiB, and 16 MiB a device for large copies.  A model holds the room of its scorers' operands from the
  * start where it is no larger than its TA states and than 256 MiB and memory allows. */
 int ytm_create(const ytm_params *params, ytm_model **out);
 void ytm_destroy(ytm_model *m);

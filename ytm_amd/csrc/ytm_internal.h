@@ -18,8 +18,8 @@ void pool_free(void* p);
 // The same for pinned host memory.
 hipError_t pinned_alloc(void** p, size_t bytes);
 void pinned_free(void* p);
-// A model that lives on a device (false: nothing is kept for it) and its end: the device's blocks
-// are kept while one does.
+// A model that lives on a device (false: not counted) and its end: more of the device's blocks are
+// kept while one does.
 bool memory_hold(int device);
 void memory_release(int device);
 // Copies device memory to a host array after the work of stream s; done on return.
