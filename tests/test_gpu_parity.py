@@ -757,6 +757,7 @@ def test_score_whole_sample_blocks(monkeypatch):
     """A literal-major copy above 32 KB (1024-thread scoring blocks) and more than 4096
     clauses: blocks over every clause of a sample (taken from YTM_SCORE_WHOLE_MIN samples
     on) give the class sums of blocks over chunks of 4096 clauses, and the oracle's."""
+    monkeypatch.setenv("YTM_SCORE_MATRIX", "0")
     dim, patch_dim, classes, clauses = (32, 32, 10), (3, 3), 3, 4300
     kw = dict(number_of_clauses_per_class=clauses, T=50, s=5.0, dim=dim, n_classes=classes, seed=7,
               patch_dim=patch_dim)
@@ -769,7 +770,6 @@ def test_score_whole_sample_blocks(monkeypatch):
     random_state(tm, ref, rng, include_p)
     X = (rng.random((20,) + dim) < 0.5).astype(np.uint32).reshape(20, -1)
     encX = tm.encode(X)
-    monkeypatch.setenv("YTM_SCORE_MATRIX", "0")
     monkeypatch.setenv("YTM_SCORE_WHOLE_MIN", "1")
     whole = tm.score(encX, is_X_encoded=True)
     monkeypatch.setenv("YTM_SCORE_WHOLE_MIN", "1000000")

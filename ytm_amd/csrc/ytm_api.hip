@@ -38,6 +38,11 @@ struct ytm_model {
   void* d_slists = nullptr;
   size_t slists_bytes = 0;
   bool slists_own = false;
+  // Test hooks, read once (a look at the environment is 0.1 us): YTM_SCORE_MATRIX=0 rules out
+  // scores on the matrix cores, YTM_SCORE_PASS gives the bytes of a pass's rows.
+  bool score_lists = false;
+  size_t score_room = (size_t)256 << 20;
+  int64_t score_least = 1024;  // samples of a pass
   // The state changes with every fit, ytm_set_ta_state and ytm_set_weights (state_version
   // counts them); d_slists holds the one-patch literal lists or the matrix operands
   // (slists_kind) of version slists_version, so that scoring again an unchanged model does
@@ -542,6 +547,11 @@ int ytm_create(const ytm_params* params, ytm_model** out) {
   };
   if (hipGetDevice(&m->device) != hipSuccess) return cleanup(fail(YTM_EHIP, "no HIP device"));
   m->held = ytm::memory_hold(m->device);
+  if (const char* env = std::getenv("YTM_SCORE_MATRIX")) m->score_lists = std::atoi(env) == 0;
+  if (const char* env = std::getenv("YTM_SCORE_PASS")) {
+    m->score_room = (size_t)std::max(0ll, std::atoll(env));
+    m->score_least = 32;
+  }
   hipDeviceProp_t prop;
   if (hipGetDeviceProperties(&prop, m->device) != hipSuccess) return cleanup(fail(YTM_EHIP, "device query failed"));
   m->cus = prop.multiProcessorCount;
@@ -796,10 +806,8 @@ int check_halves(ytm_model* m, const ytm_dataset* ds) {
   return YTM_OK;
 }
 
-// The model's scoring on the matrix cores.  YTM_SCORE_MATRIX=0 (a test hook) rules it out.
 ytm::MatrixPlan score_matrix(const ytm_model* m, int halves, int64_t N) {
-  const char* env = std::getenv("YTM_SCORE_MATRIX");
-  return env && std::atoi(env) == 0 ? ytm::MatrixPlan{} : ytm::matrix_plan(m->g, halves, m->w_bound, N);
+  return m->score_lists ? ytm::MatrixPlan{} : ytm::matrix_plan(m->g, halves, m->w_bound, N);
 }
 }  // namespace
 
@@ -1255,15 +1263,13 @@ int ytm_score_dataset(ytm_model* m, const ytm_dataset* ds, float* class_sums) {
   if (N == 0) return YTM_OK;
   ScorePlan plan{};
   if (int rc = score_plan(m, ds, &plan)) return rc;
-  // YTM_SCORE_PASS (a test hook): the bytes of a pass's rows
-  const char* room_env = std::getenv("YTM_SCORE_PASS");
-  const size_t pass_room = room_env ? (size_t)std::max(0ll, std::atoll(room_env)) : (size_t)256 << 20;
-  const int64_t per_pass = std::max<int64_t>(score_pass(plan, N, pass_room), std::min<int64_t>(N, room_env ? 32 : 1024));
-  // The rows and the sums come from the pool, where a new model finds an earlier one's.
-  void *acc = nullptr, *sums = nullptr, *pinned = nullptr;
-  const size_t out_bytes = (size_t)(N * g.K) * 4;
-  hipError_t e = ytm::pool_alloc(&acc, pass_bytes(plan, per_pass));
-  if (e == hipSuccess) e = ytm::pool_alloc(&sums, out_bytes);
+  const int64_t per_pass = std::max<int64_t>(score_pass(plan, N, m->score_room), std::min<int64_t>(N, m->score_least));
+  // The sums and the rows come from the pool, where a new model finds an earlier one's; in one
+  // block, since a block taken and given back is 0.1 us of a call of 28.
+  void *sums = nullptr, *pinned = nullptr;
+  const size_t out_bytes = (size_t)(N * g.K) * 4, out_room = (out_bytes + 255) & ~(size_t)255;
+  hipError_t e = ytm::pool_alloc(&sums, out_room + pass_bytes(plan, per_pass));
+  void* acc = e == hipSuccess ? (unsigned char*)sums + out_room : nullptr;
   if (e == hipSuccess && plan.lists_bytes > m->slists_bytes) {
     m->slists_version = ~0ull;
     if (m->slists_own) ytm::pool_free(m->d_slists);
@@ -1304,7 +1310,6 @@ int ytm_score_dataset(ytm_model* m, const ytm_dataset* ds, float* class_sums) {
     m->slists_version = ~0ull;
     (void)settle(m->stream);  // before the samples and the buffers are used again
   }
-  ytm::pool_free(acc);
   ytm::pool_free(sums);
   ytm::pinned_free(pinned);
   if (e != hipSuccess) return fail(YTM_EHIP, std::string("score failed: ") + hipGetErrorString(e));
