@@ -28,6 +28,8 @@ sys.path.insert(0, str(ROOT))
 HBM_PEAK_GBS = 8000.0
 # VALU 32-bit lane-ops per second: 256 CUs x 4 SIMDs x 16 lanes x 2.4 GHz (MI355X).
 VALU_PEAK_T = 256 * 4 * 16 * 2.4e9 / 1e12
+# Literal tests per second of the FP4 matrix instruction (32 x 32 x 64 in 32 cycles per SIMD).
+FP4_PEAK_T = 256 * 4 * 65536 / 32 * 2.4e9 / 1e12
 # Epochs of the configurations run after the headline one: (untimed, timed).
 EXTRA_EPOCHS = {1: (1, 10), 2: (1, 3), 3: (1, 2), 4: (1, 2), 5: (1, 2)}
 KIND_NAMES = {0: "resident", 1: "global one-patch", 2: "global several-patch", 3: "streaming"}
@@ -63,6 +65,26 @@ def train_bytes(tm, samples: int, updates: int) -> float:
 def infer_word_ands(tm, samples: int) -> float:
     """Inference VALU work: every clause tested on every patch, C*P*W word-ANDs per sample."""
     return float(samples) * tm.number_of_clauses * tm.number_of_patches * tm.number_of_literal_chunks
+
+
+def literal_tests(tm, samples: int) -> float:
+    """Work of the clause evaluation as a product: every clause's test of every patch is a sum
+    over its positive literals (all of them without appended negations)."""
+    lits = tm.number_of_literals // (2 if tm.append_negated else 1)
+    return float(samples) * tm.number_of_clauses * tm.number_of_patches * lits
+
+
+def infer_roofline(tm, samples: int, kern_s: float) -> dict:
+    """What the scorer that ran does per second against the peak of its unit."""
+    if tm.stats()["score_path"] == 5:
+        work, peak = literal_tests(tm, samples), FP4_PEAK_T
+        what = {"bound": "mfma", "unit": "T literal tests/s (FP4 products, C*P*(positive literals) per sample)"}
+    else:
+        work, peak = infer_word_ands(tm, samples), VALU_PEAK_T
+        what = {"bound": "valu", "unit": "T word-ANDs/s (C*P*W 32-bit lane-ops per sample, no early exit)"}
+    rate = work / kern_s / 1e12
+    return {"bound": what["bound"], "achieved": round(rate, 3), "peak": round(peak, 2), "unit": what["unit"],
+            "frac": round(rate / peak, 4), "hbm_gbs": round(infer_bytes(tm, samples) / kern_s / 1e9, 2)}
 
 
 def infer_bytes(tm, samples: int) -> float:
@@ -302,7 +324,7 @@ def run_config(cfg: int, warmup: int, steps: int, cpu: bool, n_train=None, n_tes
         st = tm.stats()
         ep = dict(wall_s=wall, kernel_ms=st["last_fit_kernel_ms"], launches=st["last_fit_launches"],
                   updates=st["last_fit_updates"], feedback=st["last_fit_feedback_samples"],
-                  evals=st["last_fit_evaluations"], wait=st["last_fit_wait_frac"], kind=st["train_kind"],
+                  evals=st["last_fit_evaluations"], wait=st["last_fit_wait_frac"], kind=st["train_kind"], product=st["train_product"],
                   wgs=st["train_workgroups"], phase=st["last_fit_phase_us"])
         epochs.append(ep)
         log(f"[bench] config {cfg} epoch {e + 1}{' (timed)' if e >= warmup else ''}: wall {wall:.3f}s "
@@ -383,14 +405,7 @@ def run_config(cfg: int, warmup: int, steps: int, cpu: bool, n_train=None, n_tes
             "feedback_sample_fraction": round(sum(e["feedback"] for e in timed) / (N * steps), 4),
             "evaluations_per_sample": round(sum(e["evals"] for e in timed) / (N * steps), 3),
         },
-        "infer_roofline": {
-            "bound": "valu",
-            "achieved": round(infer_word_ands(tm, Nt) / (inf_kern / 1e3) / 1e12, 3),
-            "peak": round(VALU_PEAK_T, 2),
-            "unit": "T word-ANDs/s (C*P*W 32-bit lane-ops per sample, no early exit)",
-            "frac": round(infer_word_ands(tm, Nt) / (inf_kern / 1e3) / 1e12 / VALU_PEAK_T, 4),
-            "hbm_gbs": round(infer_bytes(tm, Nt) / (inf_kern / 1e3) / 1e9, 2),
-        },
+        "infer_roofline": infer_roofline(tm, Nt, inf_kern / 1e3),
         "_ms_per_step": 1e3 * wall_s / steps,
     }
     traffic = load_traffic(cfg)
@@ -403,18 +418,20 @@ def run_config(cfg: int, warmup: int, steps: int, cpu: bool, n_train=None, n_tes
             res["roofline"]["traffic_gbs"] = traffic["hbm_gbs"]
             res["roofline"]["traffic_frac"] = round(traffic["hbm_gbs"] / HBM_PEAK_GBS, 4)
     counters = load_counters(cfg)
+    ands = None
     if counters:
         # measured instruction mix of the same kernel (timed epochs): how busy its execution units are
         res["binding"]["counters"] = counters
-    if cfg in (4,):
+    if cfg == 4 and last["product"]:
+        res["_literal_tests"] = literal_tests(tm, 1)
+    elif cfg == 4:
         # work model of the list walks from the trained state: each clause ANDs the PW-word
         # bitsets of its included literals (no early exit), per sample
         n_inc = tm.get_literals().reshape(tm.number_of_clauses, -1).sum(axis=1, dtype=np.int64)
         pw_words = (tm.number_of_patches + 31) // 32
         ands = float(n_inc.sum()) * pw_words
     tm.release()
-    res["binding"]["bound"] = bound_of(cfg, kw, res, timed, N, kern_s, traffic, ands if cfg in (4,) else None,
-                                       floors)
+    res["binding"]["bound"] = bound_of(cfg, kw, res, timed, N, kern_s, traffic, ands, floors)
     if cpu:
         res["cpu_baseline"] = cpu_baseline(cfg, kw, encX, y, encXt,
                                            cpu_samples if cpu_samples is not None else CPU_PREFIX[cfg])
@@ -431,8 +448,10 @@ def bound_of(cfg: int, kw: dict, res: dict, timed: list, N: int, kern_s: float, 
       config 2 (streaming kernel): the class-sum rows; peak = the samples/s of the timed
         epochs' mix of stops and streamed samples at the kernel's floors (floor_us "stop"
         for each stop, "stream" for every other sample);
-      config 4: VALU, the list walks' word-ANDs of the trained state (sum of include counts
-        times ceil(P/32) per sample) against 256 CUs x 64 lanes x 2.4 GHz;
+      config 4: the matrix cores, one clause evaluation per sample as an FP4 product (C*P*(positive
+        literals) tests) against their peak; trained on literal lists: VALU, the lists' word-ANDs
+        of the trained state (sum of include counts times ceil(P/32) per sample) against 256 CUs x
+        64 lanes x 2.4 GHz;
       config 5: HBM, the measured traffic of a timed-epoch launch (rocprofv3 FETCH_SIZE +
         WRITE_SIZE, calibrated) against 8 TB/s."""
     steps = len(timed)
@@ -453,6 +472,11 @@ def bound_of(cfg: int, kw: dict, res: dict, timed: list, N: int, kern_s: float, 
         return {"resource": "class-sum rows (streaming kernel): streamed samples and stops", "unit": "samples/s",
                 "achieved": round(rate, 1), "peak": round(N * steps / t_min, 1), "frac": round(t_min / kern_s, 4),
                 "stream_floor_us_per_sample": round(fs, 4), "stop_floor_us": round(fp, 4), "stops": stops}
+    if cfg == 4 and res.get("_literal_tests"):
+        ach = res["_literal_tests"] * rate / 1e12
+        return {"resource": "matrix cores: clause evaluation as an FP4 product, once per sample",
+                "unit": "T literal tests/s", "achieved": round(ach, 3), "peak": round(FP4_PEAK_T, 2),
+                "frac": round(ach / FP4_PEAK_T, 4), "literal_tests_per_sample": res["_literal_tests"]}
     if cfg == 4 and list_ands is not None:
         ach = list_ands * rate / 1e12
         return {"resource": "VALU: list-walk word-ANDs of the trained state (include counts x ceil(P/32))",
